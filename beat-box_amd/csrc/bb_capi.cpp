@@ -112,14 +112,13 @@ bb_status pull_state(bb_batch* b) {
   return BB_OK;
 }
 
-// Rows per world whose velocities the PGS sweeps keep in LDS: the tuning
+// Rows per world whose body state the PGS sweeps keep in LDS: the tuning
 // value, or the largest world when that is smaller.
 uint32_t pgs_lds_rows(const bb_batch* b) {
   uint32_t mx = 0;
   for (auto& hw : b->worlds) mx = std::max(mx, (uint32_t)hw.bodies.size());
   return std::min(mx, b->pgs_lds);
 }
-
 bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_t NA, uint32_t NP) {
   Dev& d = b->base;
   d = Dev{};
@@ -193,10 +192,10 @@ bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_
   d.pgs_lcap = 0;  // set after the layout (pgs_lds_rows)
   d.sv_hdr = A.alloc<int4>(NP);
   d.sv_n = A.alloc<float4>(NP);
-  d.sv_r1 = A.alloc<float4>((size_t)NP * 8);
-  d.sv_r2 = A.alloc<float4>((size_t)NP * 8);
-  d.sv_l = A.alloc<float4>((size_t)NP * 8);
-  d.sv_tm1 = A.alloc<float>((size_t)NP * 8);
+  d.sv_cp = A.alloc<float4>((size_t)NP * 8);
+  d.sv_m = A.alloc<float>((size_t)NP * 32);
+  d.sv_l = A.alloc<float>((size_t)NP * 32);
+  d.sv_t0z = A.alloc<float>((size_t)NP * 8);
   d.s_pos0 = A.alloc<float4>(NB);
   d.s_rot0 = A.alloc<float4>(NB);
   d.s_post = A.alloc<float4>(NB);
@@ -214,7 +213,8 @@ bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_
   d.team_spin = b->team_spin;
   d.sort_blocks = b->sort_blocks;
   d.avbd_lanes = b->avbd_lanes;
-  d.pgs_prefetch = b->pgs_prefetch;
+  d.pgs_quads = b->pgs_prefetch;
+  d.pgs_quad_rows = 0;  // set per launch
   d.walk_budget = b->walk_budget;
   d.teams = A.alloc<TeamTable>(1);
   d.team_ctl = A.alloc<TeamCtl>(kMaxTeams);
@@ -1398,7 +1398,7 @@ bb_status set_param(bb_batch* b, bb_param p, uint32_t value) {
     b->avbd_lanes = b->base.avbd_lanes = value;
   } else if (p == BB_PARAM_PGS_PREFETCH) {
     if (value > 1) return BB_ERR_INVALID;
-    b->pgs_prefetch = b->base.pgs_prefetch = value;
+    b->pgs_prefetch = b->base.pgs_quads = value;
   } else if (p == BB_PARAM_FUSED) {
     if (value > 1) return BB_ERR_INVALID;
     b->fused = value;
@@ -1573,7 +1573,7 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
   bool any_pgs = false;
   for (const WorldInfo& wi : b->infos)
     if (wi.solver != BB_SOLVER_AVBD && wi.n) any_pgs = true;
-  if (any_pgs) tune(b->pgs_prefetch, &b->base.pgs_prefetch, {0u, 1u});
+  if (any_pgs) tune(b->pgs_prefetch, &b->base.pgs_quads, {0u, 1u});
   if (any_avbd) {
     if (b->avbd_lanes == 0) b->avbd_lanes = b->base.avbd_lanes = 4;
     tune(b->avbd_lanes, &b->base.avbd_lanes, {1u, 2u, 4u, 8u});
@@ -1604,7 +1604,7 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
     b->fused = saved_fused;
     b->sort_blocks = b->base.sort_blocks = saved_sort;
     b->avbd_lanes = b->base.avbd_lanes = saved_lanes;
-    b->pgs_prefetch = b->base.pgs_prefetch = saved_prefetch;
+    b->pgs_prefetch = b->base.pgs_quads = saved_prefetch;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

@@ -199,11 +199,11 @@ struct Dev {
   uint32_t np;        // pair slots in the batch
   uint32_t pgs_lcap;  // rows per world whose body state k_pgs keeps in LDS (80 B each)
   int4* sv_hdr;       // a, b, count | 256 a dynamic | 512 b dynamic | 1024 one immovable, friction bits
-  float4* sv_n;       // normal
-  float4* sv_r1;      // [8*np] arm a, penetration
-  float4* sv_r2;      // [8*np] arm b, normal mass
-  float4* sv_l;       // [8*np] normal/tangent impulses, tangent mass 0
-  float* sv_tm1;      // [8*np] tangent mass 1
+  float4* sv_n;       // normal, w: the first tangent's x or y
+  float4* sv_cp;      // [8*np] contact point, penetration
+  float* sv_m;        // [8*np*3] normal mass, tangent masses 0 and 1 (the arrays
+  float* sv_l;        // [8*np*3] normal/tangent impulses        hold 8*np float4)
+  float* sv_t0z;      // [np] first tangent's z (sized like the contact arrays)
   // AVBD
   float4* s_pos0;     // [body] pos_start, w = support depth bits
   float4* s_rot0;
@@ -229,7 +229,8 @@ struct Dev {
   uint32_t team_spin;     // spins before a team barrier wait gives up (0: default)
   uint32_t sort_blocks;   // workgroups of a team that sort (0: kTeamSortBlocks)
   uint32_t avbd_lanes;    // lanes per body in the per-world AVBD primal sweeps (1, 2, 4, 8; 0: 4)
-  uint32_t pgs_prefetch;  // 1: the colour sweeps fetch each thread's next-colour row early
+  uint32_t pgs_quads;     // 1: sweep by quads of lanes whenever the workgroup has enough
+  uint32_t pgs_quad_rows; // ranges of at most this many rows are swept by quads of lanes, longer ones by lanes
   uint32_t walk_budget;   // nodes a broad-phase thread walks before its workgroup takes the row
                           // (0: kWalkBudgetDefault)
   // set (bit 0) by any world whose step flags an overflow; the host reads

@@ -3004,14 +3004,6 @@ BB_DI float plain_bias(float pen, float inv_dt) {
   return -0.2f * inv_dt * fmn(pen + 0.01f, 0.0f);
 }
 
-// Manifold::compute_basis (src/shaders/extensions.slang:262-272)
-BB_DI void contact_basis(v3 n, v3& t0, v3& t1) {
-  if (fab(n.x) > fab(n.y)) t0 = V(n.z, 0.0f, -n.x);
-  else t0 = V(0.0f, -n.z, n.y);
-  t0 = vnorm(t0);
-  t1 = cross(t0, n);
-}
-
 BB_DI mat3 iw_load(const Dev& d, uint32_t g) {
   return mrows(ld3(d.iw[g * 3 + 0]), ld3(d.iw[g * 3 + 1]), ld3(d.iw[g * 3 + 2]));
 }
@@ -3074,223 +3066,481 @@ BB_DI void pgs_compact(const Dev& d, const WorldInfo& W, uint32_t k, uint32_t sl
       kt += dot(rt2, mulmv(Ib, rt2));
       tm[j] = kt == 0.0f ? 0.0f : 1.0f / kt;
     }
-    d.sv_r1[i * NP + k] = st3(r1, cp.w);
-    d.sv_r2[i * NP + k] = st3(r2, nm);
-    d.sv_l[i * NP + k] = make_float4(lam.x, lam.y, lam.z, tm[0]);
-    d.sv_tm1[i * NP + k] = tm[1];
+    d.sv_cp[i * NP + k] = cp;
+    reinterpret_cast<v3*>(d.sv_m)[i * NP + k] = V(nm, tm[0], tm[1]);
+    reinterpret_cast<v3*>(d.sv_l)[i * NP + k] = ld3(lam);
   }
   d.sv_hdr[k] = make_int4(h.x, h.y, h.w | (da ? 256 : 0) | (db ? 512 : 0) | (soft_static ? 1024 : 0),
                           __float_as_int(__builtin_sqrtf(fa * fb)));
-  d.sv_n[k] = st3(n, 0.0f);
+  // one component of the first tangent is zero (compute_basis); the sweeps
+  // take the others from here
+  d.sv_n[k] = st3(n, fab(n.x) > fab(n.y) ? t0.x : t0.y);
+  d.sv_t0z[k] = t0.z;
 }
 
-// Body state during the PGS sweeps: rows below `lcap` keep velocity, angular
-// velocity and the three cached world inverse-inertia rows (inv_mass in
-// row0.w) in LDS, kBodyLds float4 per row; the rest stay in HBM.
-static constexpr uint32_t kBodyLds = 5;
-struct VelCache {
-  float4* lds;
-  uint32_t off, lcap;
-  BB_DI void load(const Dev& d, uint32_t i, v3& v, v3& w) const {
-    if (i < lcap) {
-      v = ld3(lds[kBodyLds * i]);
-      w = ld3(lds[kBodyLds * i + 1]);
+// ---- the sweeps.  A colour phase of a world is one row's chain of
+// operations, contact after contact.  A wave issues one vector operation
+// about every 8 cycles (10-12 with DPP or 64-bit encodings) however few of
+// its lanes are on and whether or not the operations depend on each other;
+// four waves per SIMD issue side by side at that rate.  So a phase takes the
+// instructions of a row, and the lanes are free until a CU has 16 busy waves.
+// Rows are therefore solved in two forms, chosen per range of rows:
+//  - by quads of lanes (QuadRow): lane i < 3 holds component i of every
+//    vector of the row and row i of its matrices; lane 3 computes along and
+//    is never read (it carries the w component of what was loaded).  Scalars
+//    are computed by all four lanes alike.  A contact takes about 165
+//    instructions instead of 350, and dot and matrix-vector products take
+//    their operands from the neighbours through DPP quad permutations;
+//  - by single lanes (LaneRow): half the instructions per row in total, for
+//    ranges with more rows than the workgroup has quads and for launches
+//    whose worlds fill every CU, which are bound by the chip's issue rate.
+// Each component is the same expression of the same operands in both, so the
+// results are the same bits.  Measured before (one lane per row, 311 spilled
+// registers and both row forms' code in one loop) and after: a fresh 49-body
+// world's sweeps 753 -> about 480 us a step, 513 worlds on the per-island
+// path 17.3 -> 13.0 ms, 4,096 batched worlds 6.6 -> 6.0 ms.
+template <int CTRL>
+BB_DI float quad_perm(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+// the quad's lane k in every lane
+BB_DI float qc0(float x) { return quad_perm<0x00>(x); }
+BB_DI float qc1(float x) { return quad_perm<0x55>(x); }
+BB_DI float qc2(float x) { return quad_perm<0xAA>(x); }
+BB_DI float qc3(float x) { return quad_perm<0xFF>(x); }
+// component i+1 and i+2 (mod 3) in lane i
+BB_DI float qr1(float x) { return quad_perm<0xC9>(x); }
+BB_DI float qr2(float x) { return quad_perm<0xD2>(x); }
+BB_DI float qdot(float a, float b) {
+  const float p = a * b;
+  return (qc0(p) + qc1(p)) + qc2(p);
+}
+// A vector with its rotations: cross(a, b) = a1*b2 - a2*b1 per component.
+struct QV {
+  float c, r1, r2;
+};
+BB_DI QV qv(float x) { return QV{x, qr1(x), qr2(x)}; }
+BB_DI QV operator*(QV a, float s) { return QV{a.c * s, a.r1 * s, a.r2 * s}; }
+BB_DI float qcross(QV a, QV b) { return a.r1 * b.r2 - a.r2 * b.r1; }
+// row i (m) of a matrix times the vector x
+BB_DI float qmulmv(v3 m, float x) { return (m.x * qc0(x) + m.y * qc1(x)) + m.z * qc2(x); }
+
+// What the PGS sweeps of a world keep in LDS, in floats: for its first `rows`
+// body rows velocity, inverse mass, angular velocity, position at detection
+// and world inverse inertia (19 of kBodyLds floats each; the rest stay in
+// HBM).  kMem: every body row in LDS, none, or by row.
+static constexpr uint32_t kBodyLds = 20;
+static constexpr int kPgsPre = 4;
+enum : int { kMemLds = 0, kMemHbm = 1, kMemBoth = 2 };
+template <int kMem>
+struct PgsLds {
+  float* lds;
+  uint32_t off, rows;
+  BB_DI bool in_lds(uint32_t i) const { return kMem == kMemLds || (kMem == kMemBoth && i < rows); }
+  BB_DI float4* body(uint32_t i) const { return reinterpret_cast<float4*>(lds) + 5u * i; }
+  BB_DI void fill(const Dev& d, uint32_t i, float4 p) const {
+    const uint32_t g = off + i;
+    const float4 v = d.cur.vel[g], o = d.cur.omg[g];
+    float4* b = body(i);
+    b[0] = make_float4(v.x, v.y, v.z, d.iw[g * 3].w);
+    b[1] = make_float4(o.x, o.y, o.z, p.x);
+    b[2].x = p.y;
+    b[2].y = p.z;
+    fill_iw(d, i);
+  }
+  BB_DI void fill_iw(const Dev& d, uint32_t i) const {
+    const uint32_t g = off + i;
+    const float4 m0 = d.iw[g * 3], m1 = d.iw[g * 3 + 1], m2 = d.iw[g * 3 + 2];
+    float4* b = body(i);
+    b[2].z = m0.x;
+    b[2].w = m0.y;
+    b[3] = make_float4(m0.z, m1.x, m1.y, m1.z);
+    b[4] = make_float4(m2.x, m2.y, m2.z, 0.0f);
+  }
+  // this lane's component of the velocities and position and row of the
+  // inverse inertia, and (all lanes) the inverse mass of row i
+  BB_DI void load(const Dev& d, uint32_t i, uint32_t ln, float& v, float& w, float& p, v3& m, float& im) const {
+    const uint32_t lr = ln < 3u ? ln : 2u;
+    if (in_lds(i)) {
+      const float* b = lds + kBodyLds * i;
+      v = b[ln];
+      im = b[3];
+      w = b[4 + ln];
+      p = b[7 + lr];
+      const float* r = b + 10u + 3u * lr;
+      m = V(r[0], r[1], r[2]);
     } else {
-      v = ld3(d.cur.vel[off + i]);
-      w = ld3(d.cur.omg[off + i]);
+      const uint32_t g = off + i;
+      v = reinterpret_cast<const float*>(d.cur.vel + g)[ln];
+      w = reinterpret_cast<const float*>(d.cur.omg + g)[ln];
+      p = reinterpret_cast<const float*>(d.s_pos0 + g)[ln];
+      m = ld3(d.iw[g * 3 + lr]);
+      im = d.iw[g * 3].w;
     }
   }
-  BB_DI void store(const Dev& d, uint32_t i, v3 v, v3 w) const {
-    if (i < lcap) {
-      lds[kBodyLds * i] = st3(v, 0.0f);
-      lds[kBodyLds * i + 1] = st3(w, 0.0f);
+  BB_DI void store(const Dev& d, uint32_t i, uint32_t ln, float v, float w) const {
+    if (in_lds(i)) {
+      if (ln < 3u) {
+        float* b = lds + kBodyLds * i;
+        b[ln] = v;
+        b[4 + ln] = w;
+      }
+    } else {
+      reinterpret_cast<float*>(d.cur.vel + off + i)[ln] = ln < 3u ? v : 0.0f;
+      reinterpret_cast<float*>(d.cur.omg + off + i)[ln] = ln < 3u ? w : 0.0f;
+    }
+  }
+  // the same with one lane per row
+  BB_DI void load_lane(const Dev& d, uint32_t i, v3& v, v3& w, v3& p, mat3& m, float& im) const {
+    if (in_lds(i)) {
+      const float4* b = body(i);
+      const float4 a0 = b[0], a1 = b[1], a2 = b[2], a3 = b[3], a4 = b[4];
+      v = ld3(a0);
+      im = a0.w;
+      w = ld3(a1);
+      p = V(a1.w, a2.x, a2.y);
+      m = mrows(V(a2.z, a2.w, a3.x), V(a3.y, a3.z, a3.w), ld3(a4));
+    } else {
+      const uint32_t g = off + i;
+      const float4 m0 = d.iw[g * 3], m1 = d.iw[g * 3 + 1], m2 = d.iw[g * 3 + 2];
+      m = mrows(ld3(m0), ld3(m1), ld3(m2));
+      v = ld3(d.cur.vel[g]);
+      w = ld3(d.cur.omg[g]);
+      p = ld3(d.s_pos0[g]);
+      im = m0.w;
+    }
+  }
+  BB_DI void store_lane(const Dev& d, uint32_t i, v3 v, v3 w) const {
+    if (in_lds(i)) {
+      float* b = lds + kBodyLds * i;
+      b[0] = v.x; b[1] = v.y; b[2] = v.z;
+      b[4] = w.x; b[5] = w.y; b[6] = w.z;
     } else {
       d.cur.vel[off + i] = st3(v, 0.0f);
       d.cur.omg[off + i] = st3(w, 0.0f);
     }
   }
-  BB_DI void load_iw(const Dev& d, uint32_t i, float4& r0, float4& r1, float4& r2) const {
-    if (i < lcap) {
-      r0 = lds[kBodyLds * i + 2];
-      r1 = lds[kBodyLds * i + 3];
-      r2 = lds[kBodyLds * i + 4];
-    } else {
-      const uint32_t g = off + i;
-      r0 = d.iw[g * 3];
-      r1 = d.iw[g * 3 + 1];
-      r2 = d.iw[g * 3 + 2];
-    }
-  }
 };
 
-// Contacts per row whose solver data pgs_row loads up front.
-static constexpr int kPgsPre = 4;
-// A row's solver data that pgs_row loads before it touches the body state:
-// the header, the normal and the first kPgsPre contacts.  None of it is
-// written by any other row, so it can be loaded early: the colour sweeps
-// fetch a thread's row of the next colour while it solves this colour's.
+// The solver rows of one world: the arrays' first entries of it (contact c of
+// row k lies np entries times c behind them), indexed by 32-bit offsets.
+struct PgsRows {
+  const int4* hdr;
+  const float* n;
+  const float* t0z;
+  const float *cp, *m;
+  float* l;
+  uint32_t np;
+  BB_DI PgsRows(const Dev& d, uint32_t base)
+      : hdr(d.sv_hdr + base), n(reinterpret_cast<const float*>(d.sv_n + base)), t0z(d.sv_t0z + base),
+        cp(reinterpret_cast<const float*>(d.sv_cp + base)), m(d.sv_m + (size_t)base * 3u), l(d.sv_l + (size_t)base * 3u),
+        np(d.np) {}
+  // contact c's entries: float4 (cp), three floats (m, l)
+  BB_DI const float* cp_at(int c) const { return cp + (size_t)c * np * 4u; }
+  BB_DI const float* m_at(int c) const { return m + (size_t)c * np * 3u; }
+  BB_DI float* l_at(int c) const { return l + (size_t)c * np * 3u; }
+};
+// A row's solver data in a quad: the header, the normal, the first tangent's
+// last component and the first kPgsPre contacts (kPgsPre float4 pairs are
+// loaded whatever the row's count: the contact arrays hold 8 entries per row
+// slot, so the loads stay in bounds, and entries past the count are never
+// used), one dword per lane and float4.  No row's sweep writes any of it, so
+// a quad fetches its next row (of this colour or the next one, across the
+// barrier) before it solves this one and the loads are in flight meanwhile.
 struct PgsRow {
   int4 h;
-  float4 n;
-  float4 r1[kPgsPre], r2[kPgsPre], l[kPgsPre];
-  float tm[kPgsPre];
+  float n, t0z;
+  float cp[kPgsPre], m[kPgsPre], l[kPgsPre];
 };
-// The first kPgsPre contacts' data are loaded whatever the row's contact
-// count: the contact arrays hold 8 entries per row slot, so the loads stay in
-// bounds, and issuing them with the header instead of after it (the count is
-// in the header) saves a dependent round trip per colour phase.  Entries past
-// the count are never used.
-BB_DI void pgs_fetch(const Dev& d, uint32_t k, int kind, PgsRow& R) {
-  const uint32_t NP = d.np;
-  R.h = d.sv_hdr[k];
-  R.n = d.sv_n[k];
+BB_DI void pgs_fetch(const PgsRows& S, uint32_t k, uint32_t ln, PgsRow& R) {
+  const uint32_t q = k * 4u + ln;
+  R.h = S.hdr[k];
+  R.n = S.n[q];
+  R.t0z = S.t0z[k];
 #pragma unroll
   for (int c = 0; c < kPgsPre; ++c) {
-    R.r1[c] = d.sv_r1[c * NP + k];
-    R.r2[c] = d.sv_r2[c * NP + k];
-    R.l[c] = d.sv_l[c * NP + k];
-    R.tm[c] = kind != 0 ? d.sv_tm1[c * NP + k] : 0.0f;
+    R.cp[c] = S.cp_at(c)[q];
+    R.m[c] = S.m_at(c)[k * 3u + ln];
+    R.l[c] = S.l_at(c)[k * 3u + ln];
   }
 }
-// kind 0: warm-start impulses of pre_step; 1: solve with bias; 2: relax.
-// kPlain: PGS (the per-island path) instead of PGS_SOFT.  R: the row's
-// fetched data (pgs_fetch).
-template <bool kPlain>
-BB_DI void pgs_solve(const Dev& d, const VelCache& vc, uint32_t off, uint32_t k, const Pgs& s, int kind,
-                     const PgsRow& R) {
-  const uint32_t NP = d.np;
+// Row k of the world's rows, fetched into R.  kWarm: the warm-start impulses
+// of pre_step; otherwise one solve (with bias, or a relaxation).  kPlain: PGS
+// (the per-island path) instead of PGS_SOFT.  kUsual: impulses accumulate
+// and there is friction (the default flags), so neither is tested per
+// contact.  ln: this lane's place in its quad.
+template <bool kPlain, bool kWarm, bool kUsual, int kMem>
+BB_DI void pgs_solve(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc, uint32_t k, uint32_t ln, const Pgs& s,
+                     bool use_bias, const PgsRow& R) {
+  const bool accum = kUsual || s.accum, friction = kUsual || s.friction;
+  const uint32_t q = k * 4u + ln;
   const int4 h = R.h;
   const int count = h.z & 255;
-  if (kind == 0 && !s.accum) return;
   const bool da = (h.z & 256) != 0, db = (h.z & 512) != 0;
-  float4 pr1[kPgsPre], pr2[kPgsPre], pl[kPgsPre];
-  float ptm[kPgsPre];
-#pragma unroll
-  for (int c = 0; c < kPgsPre; ++c) {
-    pr1[c] = R.r1[c];
-    pr2[c] = R.r2[c];
-    pl[c] = R.l[c];
-    ptm[c] = R.tm[c];
-  }
-  const v3 n = ld3(R.n);
-  float4 ia0, ia1, ia2, ib0, ib1, ib2;
-  vc.load_iw(d, (uint32_t)h.x, ia0, ia1, ia2);
-  vc.load_iw(d, (uint32_t)h.y, ib0, ib1, ib2);
-  const float ima = ia0.w, imb = ib0.w;
-  const mat3 Ia = mrows(ld3(ia0), ld3(ia1), ld3(ia2));
-  const mat3 Ib = mrows(ld3(ib0), ld3(ib1), ld3(ib2));
-  v3 va, wa, vb, wb;
-  vc.load(d, (uint32_t)h.x, va, wa);
-  vc.load(d, (uint32_t)h.y, vb, wb);
-  v3 t0, t1;
-  contact_basis(n, t0, t1);
-  if (kind == 0) {
-    auto warm = [&](float4 l, float4 c1, float4 c2) {
-      const v3 r1 = ld3(c1), r2 = ld3(c2);
-      v3 P = n * l.x;
-      if (s.friction) {
-        P = P + t0 * l.y;
-        P = P + t1 * l.z;
+  float va, wa, vb, wb, pa, pb, ima, imb;
+  v3 Ia, Ib;
+  vc.load(d, (uint32_t)h.x, ln, va, wa, pa, Ia, ima);
+  vc.load(d, (uint32_t)h.y, ln, vb, wb, pb, Ib, imb);
+  // Manifold::compute_basis: one component of the first tangent is zero,
+  // which one follows from the normal; the other two come with the row
+  const QV n = qv(R.n);
+  const float nx = qc0(R.n), ny = qc1(R.n), t0a = qc3(R.n);
+  const uint32_t la = fab(nx) > fab(ny) ? 0u : 1u;
+  const QV t0 = qv(ln == 2u ? R.t0z : (ln == la ? t0a : 0.0f));
+  const QV t1 = qv(qcross(t0, n));
+  // impulse P on the bodies at arms r1, r2
+  auto apply = [&](QV P, QV r1, QV r2) __attribute__((always_inline)) {
+    const float va2 = va - P.c * ima, wa2 = wa - qmulmv(Ia, qcross(r1, P));
+    const float vb2 = vb + P.c * imb, wb2 = wb + qmulmv(Ib, qcross(r2, P));
+    va = da ? va2 : va;
+    wa = da ? wa2 : wa;
+    vb = db ? vb2 : vb;
+    wb = db ? wb2 : wb;
+  };
+  if constexpr (kWarm) {
+    auto warm = [&](float l4, float cp) __attribute__((always_inline)) {
+      float P = n.c * qc0(l4);
+      if (friction) {
+        P = P + t0.c * qc1(l4);
+        P = P + t1.c * qc2(l4);
       }
-      if (da) {
-        va = va - P * ima;
-        wa = wa - mulmv(Ia, cross(r1, P));
-      }
-      if (db) {
-        vb = vb + P * imb;
-        wb = wb + mulmv(Ib, cross(r2, P));
-      }
+      apply(qv(P), qv(cp - pa), qv(cp - pb));
     };
 #pragma unroll
     for (int c = 0; c < kPgsPre; ++c)
-      if (c < count) warm(pl[c], pr1[c], pr2[c]);
-    for (int c = kPgsPre; c < count; ++c) warm(d.sv_l[c * NP + k], d.sv_r1[c * NP + k], d.sv_r2[c * NP + k]);
+      if (c < count) warm(R.l[c], R.cp[c]);
+    for (int c = kPgsPre; c < count; ++c) warm(S.l_at(c)[k * 3u + ln], S.cp_at(c)[q]);
   } else {
-    const bool use_bias = kind == 1;
     const float fr = __int_as_float(h.w);
-    const Soft sc = (h.z & 1024) ? s.soft[1] : s.soft[0];
-    const float bias_factor = sc.bias_factor, impulse_coef = sc.impulse_coef, mass_coef = sc.mass_coef;
-    auto solve = [&](int c, float4 c1, float4 c2, float4 l, float tm1) {
-      const v3 r1 = ld3(c1), r2 = ld3(c2);
-      const float pen = c1.w, nm = c2.w;
-      v3 rv = ((vb + cross(wb, r2)) - va) - cross(wa, r1);
-      if (s.friction) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const v3 tj = j == 0 ? t0 : t1;
-          const float tmass = j == 0 ? l.w : tm1;
-          const float tv = dot(rv, tj);
-          float ti = tmass * -tv;
-          const float maxf = fr * l.x;
-          if (s.accum) {
-            const float old = j == 0 ? l.y : l.z;
-            const float nw = fcl(old + ti, -maxf, maxf);
-            if (j == 0) l.y = nw; else l.z = nw;
-            ti = nw - old;
+    const bool immovable = (h.z & 1024) != 0;
+    const float bias_factor = immovable ? s.soft[1].bias_factor : s.soft[0].bias_factor;
+    const float impulse_coef = immovable ? s.soft[1].impulse_coef : s.soft[0].impulse_coef;
+    const float mass_coef = immovable ? s.soft[1].mass_coef : s.soft[0].mass_coef;
+    auto rel_vel = [&](QV r1, QV r2) {
+      return ((vb + qcross(qv(wb), r2)) - va) - qcross(qv(wa), r1);
+    };
+    auto solve = [&](int c, float cp, float m, float l4) __attribute__((always_inline)) {
+      const QV r1 = qv(cp - pa), r2 = qv(cp - pb);
+      const float pen = qc3(cp), nm = qc0(m), tm0 = qc1(m), tm1 = qc2(m);
+      float lx = qc0(l4), ly = qc1(l4), lz = qc2(l4);
+      if (friction) {
+        const float rv = rel_vel(r1, r2);
+        const float maxf = fr * lx;
+        auto tangent = [&](const QV& t, float tmass, float& lt, float v) {
+          float ti = tmass * -qdot(v, t.c);
+          if (accum) {
+            const float nw = fcl(lt + ti, -maxf, maxf);
+            ti = nw - lt;
+            lt = nw;
           } else {
             ti = fcl(ti, -maxf, maxf);
           }
-          const v3 tiv = tj * ti;
-          if (da) {
-            va = va - tiv * ima;
-            wa = wa - mulmv(Ia, cross(r1, tiv));
-          }
-          if (db) {
-            vb = vb + tiv * imb;
-            wb = wb + mulmv(Ib, cross(r2, tiv));
-          }
-        }
+          apply(t * ti, r1, r2);
+        };
+        tangent(t0, tm0, ly, rv);
+        tangent(t1, tm1, lz, rv);
       }
-      rv = ((vb + cross(wb, r2)) - va) - cross(wa, r1);
-      const float nv = dot(rv, n);
+      const float nv = qdot(rel_vel(r1, r2), n.c);
       float imp;
       if (kPlain) {
         // PGS::solve (solvers.slang:106-117)
         imp = nm * (-nv + plain_bias(pen, s.inv_dt));
       } else {
-        float bias = 0.0f, mass_scale = 1.0f, impulse_scale = 0.0f;
-        if (pen > 0.0f) {
-          bias = pen * s.inv_dt;
-        } else if (use_bias) {
-          bias = fmx(bias_factor * pen, -4.0f);
-          mass_scale = mass_coef;
-          impulse_scale = impulse_coef;
-        }
-        imp = -nm * mass_scale * (nv + bias) - impulse_scale * l.x;
+        const bool sep = pen > 0.0f, soft = !sep && use_bias;
+        const float bias = sep ? pen * s.inv_dt : (soft ? fmx(bias_factor * pen, -4.0f) : 0.0f);
+        const float mass_scale = soft ? mass_coef : 1.0f;
+        const float impulse_scale = soft ? impulse_coef : 0.0f;
+        imp = -nm * mass_scale * (nv + bias) - impulse_scale * lx;
       }
-      if (s.accum) {
-        const float old = l.x;
-        l.x = fmx(old + imp, 0.0f);
-        imp = l.x - old;
+      if (accum) {
+        const float old = lx;
+        lx = fmx(old + imp, 0.0f);
+        imp = lx - old;
       } else {
         imp = fmx(imp, 0.0f);
       }
-      const v3 niv = n * imp;
-      if (da) {
-        va = va - niv * ima;
-        wa = wa - mulmv(Ia, cross(r1, niv));
-      }
-      if (db) {
-        vb = vb + niv * imb;
-        wb = wb + mulmv(Ib, cross(r2, niv));
-      }
-      d.sv_l[c * NP + k] = l;
+      apply(n * imp, r1, r2);
+      float out = 0.0f;
+      out = ln == 0u ? lx : out;
+      out = ln == 1u ? ly : out;
+      out = ln == 2u ? lz : out;
+      if (ln < 3u) S.l_at(c)[k * 3u + ln] = out;
     };
 #pragma unroll
     for (int c = 0; c < kPgsPre; ++c)
-      if (c < count) solve(c, pr1[c], pr2[c], pl[c], ptm[c]);
-    for (int c = kPgsPre; c < count; ++c)
-      solve(c, d.sv_r1[c * NP + k], d.sv_r2[c * NP + k], d.sv_l[c * NP + k], d.sv_tm1[c * NP + k]);
+      if (c < count) solve(c, R.cp[c], R.m[c], R.l[c]);
+    for (int c = kPgsPre; c < count; ++c) solve(c, S.cp_at(c)[q], S.m_at(c)[k * 3u + ln], S.l_at(c)[k * 3u + ln]);
   }
-  if (da) vc.store(d, (uint32_t)h.x, va, wa);
-  if (db) vc.store(d, (uint32_t)h.y, vb, wb);
+  if (da) vc.store(d, (uint32_t)h.x, ln, va, wa);
+  if (db) vc.store(d, (uint32_t)h.y, ln, vb, wb);
 }
-// One row, fetched and solved in turn.
-template <bool kPlain>
-BB_DI void pgs_row(const Dev& d, const VelCache& vc, uint32_t off, uint32_t k, const Pgs& s, int kind) {
+
+// A row's solver data in one lane: header, normal, first tangent, and the
+// contact at hand; the next contact is loaded while this one is solved.
+struct PgsContact {
+  float4 cp;
+  v3 m, l;
+};
+BB_DI PgsContact pgs_contact(const PgsRows& S, uint32_t k, int c) {
+  return PgsContact{reinterpret_cast<const float4*>(S.cp_at(c))[k], reinterpret_cast<const v3*>(S.m_at(c))[k],
+                    reinterpret_cast<const v3*>(S.l_at(c))[k]};
+}
+struct PgsLaneRow {
+  int4 h;
+  float4 n;
+  float t0z;
+  PgsContact c0;
+};
+BB_DI void pgs_fetch_lane(const PgsRows& S, uint32_t k, PgsLaneRow& R) {
+  R.h = S.hdr[k];
+  R.n = reinterpret_cast<const float4*>(S.n)[k];
+  R.t0z = S.t0z[k];
+  R.c0 = pgs_contact(S, k, 0);
+}
+// Row k by one lane, with the default flags (impulses accumulate, friction).
+template <bool kPlain, bool kWarm, int kMem>
+BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc, uint32_t k, const Pgs& s,
+                          bool use_bias, const PgsLaneRow& R) {
+  const int4 h = R.h;
+  const int count = h.z & 255;
+  const bool da = (h.z & 256) != 0, db = (h.z & 512) != 0;
+  v3 va, wa, pa, vb, wb, pb;
+  mat3 Ia, Ib;
+  float ima, imb;
+  vc.load_lane(d, (uint32_t)h.x, va, wa, pa, Ia, ima);
+  vc.load_lane(d, (uint32_t)h.y, vb, wb, pb, Ib, imb);
+  const v3 n = ld3(R.n);
+  const bool xz = fab(n.x) > fab(n.y);
+  const v3 t0 = V(xz ? R.n.w : 0.0f, xz ? 0.0f : R.n.w, R.t0z);
+  const v3 t1 = cross(t0, n);
+  const float fr = __int_as_float(h.w);
+  const bool immovable = (h.z & 1024) != 0;
+  const float bias_factor = immovable ? s.soft[1].bias_factor : s.soft[0].bias_factor;
+  const float impulse_coef = immovable ? s.soft[1].impulse_coef : s.soft[0].impulse_coef;
+  const float mass_coef = immovable ? s.soft[1].mass_coef : s.soft[0].mass_coef;
+  auto apply = [&](v3 P, v3 r1, v3 r2) __attribute__((always_inline)) {
+    if (da) {
+      va = va - P * ima;
+      wa = wa - mulmv(Ia, cross(r1, P));
+    }
+    if (db) {
+      vb = vb + P * imb;
+      wb = wb + mulmv(Ib, cross(r2, P));
+    }
+  };
+  PgsContact x = R.c0;
+  for (int c = 0; c < count; ++c) {
+    // (the last contact fetches itself again)
+    const PgsContact next = pgs_contact(S, k, c + 1 < count ? c + 1 : c);
+    const v3 r1 = ld3(x.cp) - pa, r2 = ld3(x.cp) - pb;
+    v3 l = x.l;
+    if constexpr (kWarm) {
+      v3 P = n * l.x;
+      P = P + t0 * l.y;
+      P = P + t1 * l.z;
+      apply(P, r1, r2);
+    } else {
+      const float pen = x.cp.w, nm = x.m.x;
+      auto rel_vel = [&]() __attribute__((always_inline)) {
+        return ((vb + cross(wb, r2)) - va) - cross(wa, r1);
+      };
+      const v3 rv = rel_vel();
+      const float maxf = fr * l.x;
+      auto tangent = [&](v3 t, float tmass, float& lt) __attribute__((always_inline)) {
+        const float ti = tmass * -dot(rv, t);
+        const float nw = fcl(lt + ti, -maxf, maxf);
+        const float di = nw - lt;
+        lt = nw;
+        apply(t * di, r1, r2);
+      };
+      tangent(t0, x.m.y, l.y);
+      tangent(t1, x.m.z, l.z);
+      const float nv = dot(rel_vel(), n);
+      float imp;
+      if (kPlain) {
+        imp = nm * (-nv + plain_bias(pen, s.inv_dt));
+      } else {
+        const bool sep = pen > 0.0f, soft = !sep && use_bias;
+        const float bias = sep ? pen * s.inv_dt : (soft ? fmx(bias_factor * pen, -4.0f) : 0.0f);
+        const float mass_scale = soft ? mass_coef : 1.0f;
+        const float impulse_scale = soft ? impulse_coef : 0.0f;
+        imp = -nm * mass_scale * (nv + bias) - impulse_scale * l.x;
+      }
+      const float old = l.x;
+      l.x = fmx(old + imp, 0.0f);
+      apply(n * (l.x - old), r1, r2);
+      reinterpret_cast<v3*>(S.l_at(c))[k] = l;
+    }
+    x = next;
+  }
+  if (da) vc.store_lane(d, (uint32_t)h.x, va, wa);
+  if (db) vc.store_lane(d, (uint32_t)h.y, vb, wb);
+}
+
+// One sweep over the ranges [ro[c], ro[c+1]) of a world's rows (colours, or
+// dependency levels), c < nr, a barrier after each non-empty one, then the
+// rows [ovf_lo, ovf_hi) one after another by the first quad.  Row k is always
+// solved by the same lanes.  Ranges of at most quad_rows rows go to quads,
+// longer ones to single lanes (kUsual; otherwise all go to quads).
+template <bool kPlain, bool kWarm, bool kUsual, int kMem, class T>
+BB_DI void pgs_sweep(const Dev& d, const T& t, const PgsLds<kMem>& vc, const Pgs& s, const PgsRows& S,
+                     const uint32_t* ro, uint32_t nr, uint32_t ovf_lo, uint32_t ovf_hi, bool use_bias,
+                     uint32_t quad_rows) {
+  const uint32_t tid = t.rank(), NT = t.size();
+  const uint32_t ln = tid & 3u, q = tid >> 2, NQ = NT >> 2;
+  const uint32_t wl = tid & (WAVE - 1);
+  if (kWarm && !s.accum) return;
+  // offsets of up to WAVE - 1 ranges, one per lane
+  uint32_t chunk = 0, offs = wl <= nr ? ro[wl] : 0u;
+  auto bound = [&](uint32_t c) __attribute__((always_inline)) {  // ro[c], c uniform and ascending
+    if (c - chunk >= (uint32_t)WAVE) {
+      chunk = c;
+      offs = c + wl <= nr ? ro[c + wl] : 0u;
+    }
+    return (uint32_t)__builtin_amdgcn_readlane((int)offs, (int)(c - chunk));
+  };
+  uint32_t lo = bound(0), hi = nr ? bound(1) : lo;
+  const uint32_t end = nr ? ro[nr] : lo;
+  // Every quad (lane) fetches a row every round, the last one when it has
+  // none of its own: a load under a condition would make the compiler wait
+  // for all loads at once.
+  auto in = [&](uint32_t k) __attribute__((always_inline)) { return k < end ? k : end - 1u; };
   PgsRow R;
-  pgs_fetch(d, k, kind, R);
-  pgs_solve<kPlain>(d, vc, off, k, s, kind, R);
+  bool have = false;  // R holds this quad's first row of the range
+  for (uint32_t c = 0; c < nr && lo < end; ++c) {
+    const uint32_t hi2 = c + 2 <= nr ? bound(c + 2) : hi;
+    if (!kUsual || hi - lo <= quad_rows) {
+      if (!have) pgs_fetch(S, in(lo + q), ln, R);
+      for (uint32_t k0 = lo; k0 < hi; k0 += NQ) {
+        const uint32_t k = k0 + q;
+        PgsRow X;
+        pgs_fetch(S, in((k0 + NQ < hi ? k0 + NQ : hi) + q), ln, X);
+        if (k < hi) pgs_solve<kPlain, kWarm, kUsual, kMem>(d, S, vc, k, ln, s, use_bias, R);
+        R = X;
+      }
+      have = true;
+    } else {
+      have = false;
+      PgsLaneRow L;
+      pgs_fetch_lane(S, in(lo + tid), L);
+      for (uint32_t k0 = lo; k0 < hi; k0 += NT) {
+        const uint32_t k = k0 + tid;
+        if (k < hi) pgs_solve_lane<kPlain, kWarm, kMem>(d, S, vc, k, s, use_bias, L);
+        if (k0 + NT < hi) pgs_fetch_lane(S, in(k + NT), L);
+      }
+    }
+    if (hi > lo) t.sync();
+    lo = hi;
+    hi = hi2;
+  }
+  if (ovf_hi > ovf_lo) {
+    if (q == 0)
+      for (uint32_t r = ovf_lo; r < ovf_hi; ++r) {
+        pgs_fetch(S, r, ln, R);
+        pgs_solve<kPlain, kWarm, kUsual, kMem>(d, S, vc, r, ln, s, use_bias, R);
+      }
+    t.sync();
+  }
 }
 
 // RigidBody::apply_angular_velocity (src/shaders/extensions.slang:148-166)
@@ -3311,7 +3561,7 @@ BB_DI qt apply_angular_velocity(qt q, v3 om, float dt) {
 // sweep dependency levels; kPlain: PGS (per-island path only) rather than
 // PGS_SOFT.  k_pgs, the colour sweeps, carries neither.
 template <bool kIsland, bool kPlain, class T>
-BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float4* pgs_lds, uint32_t lcap) {
+BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t lcap) {
   const uint32_t tid = t.rank(), NT = t.size();
   const WorldInfo W = d.worlds[w];
   if (W.solver == BB_SOLVER_AVBD || W.n == 0) return;
@@ -3334,104 +3584,74 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float4* pgs_lds, uint32_t
   const uint32_t used = kIsland ? kColors : d.stats[w * ST_COUNT + ST_GC_COUNT];
   const uint32_t base = W.pair_off;
   const uint32_t ovf_lo = bo[kColors], ovf_hi = bo[kBuckets];
-  const VelCache vc{pgs_lds, off, N < lcap ? N : lcap};
-  for (uint32_t i = tid; i < vc.lcap; i += NT) {
-    const uint32_t g = off + i;
-    pgs_lds[kBodyLds * i] = d.cur.vel[g];
-    pgs_lds[kBodyLds * i + 1] = d.cur.omg[g];
-    pgs_lds[kBodyLds * i + 2] = d.iw[g * 3];
-    pgs_lds[kBodyLds * i + 3] = d.iw[g * 3 + 1];
-    pgs_lds[kBodyLds * i + 4] = d.iw[g * 3 + 2];
+  const uint32_t ncache = N < lcap ? N : lcap;
+  const PgsLds<kMemBoth> cache{pgs_lds, off, ncache};
+  for (uint32_t i = tid; i < N; i += NT) {
+    const float4 p = d.cur.pos[off + i];
+    if (i < ncache) cache.fill(d, i, p);
+    else d.s_pos0[off + i] = p;
   }
   t.sync();
-  auto row = [&](uint32_t k, int kind) { pgs_row<kPlain>(d, vc, off, base + k, s, kind); };
-  // exact dependency levels of the per-island path (0: buckets)
+  // the sweeps' ranges: exact dependency levels of the per-island path, its
+  // capped level buckets, or colours
   const uint32_t nlev = kIsland ? d.nlev[w] : 0u;
-  const uint32_t* lvoff = d.adj + 2 * W.pair_off;
-  auto sweep = [&](int kind) {
-    if (nlev) {
-      for (uint32_t lv = 0; lv < nlev; ++lv) {
-        for (uint32_t k = lvoff[lv] + tid; k < lvoff[lv + 1]; k += NT) row(k, kind);
-        t.sync();
-      }
-      return;
-    }
-    if (d.pgs_prefetch) {
-      // each thread fetches its first row of the next colour as soon as it
-      // is done with this colour, before the barrier, so the loads are in
-      // flight while the slower threads finish (rows beyond the first, when a
-      // colour has more rows than threads, are fetched where they are solved)
-      uint32_t c = 0;
-      while (c < used && bo[c] == bo[c + 1]) ++c;
-      PgsRow R;
-      bool have = c < used && bo[c] + tid < bo[c + 1];
-      if (have) pgs_fetch(d, base + bo[c] + tid, kind, R);
-      while (c < used) {
-        if (have) pgs_solve<kPlain>(d, vc, off, base + bo[c] + tid, s, kind, R);
-        for (uint32_t k = bo[c] + tid + NT; k < bo[c + 1]; k += NT) row(k, kind);
-        uint32_t cn = c + 1;
-        while (cn < used && bo[cn] == bo[cn + 1]) ++cn;
-        have = cn < used && bo[cn] + tid < bo[cn + 1];
-        if (have) pgs_fetch(d, base + bo[cn] + tid, kind, R);
-        t.sync();
-        c = cn;
-      }
+  const uint32_t* ro = nlev ? d.adj + 2 * W.pair_off : bo;
+  const uint32_t nr = nlev ? nlev : used;
+  const uint32_t olo = nlev ? 0u : ovf_lo, ohi = nlev ? 0u : ovf_hi;
+  const PgsRows S(d, base);
+  const bool usual = s.accum && s.friction;
+  const uint32_t quad_rows = T::kGlobalScalars ? NT / 4u : d.pgs_quad_rows;
+  auto sweep_in = [&](auto warm, auto vc, bool use_bias) __attribute__((always_inline)) {
+    constexpr bool kWarm = decltype(warm)::value;
+    if (usual) pgs_sweep<kPlain, kWarm, true>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
+    else pgs_sweep<kPlain, kWarm, false>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
+  };
+  auto sweep = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
+    if constexpr (T::kGlobalScalars) {  // teams keep no rows in LDS
+      sweep_in(warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
+    } else if (ncache == N) {
+      sweep_in(warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
     } else {
-      // the next colour's end offset is loaded while this colour's rows are
-      // solved, so no phase starts with a dependent load of its range
-      uint32_t b0 = bo[0], b1 = used > 0 ? bo[1] : 0u;
-      for (uint32_t c = 0; c < used; ++c) {
-        const uint32_t b2 = c + 1 < used ? bo[c + 2] : 0u;
-        if (b0 != b1) {
-          for (uint32_t k = b0 + tid; k < b1; k += NT) row(k, kind);
-          t.sync();
-        }
-        b0 = b1;
-        b1 = b2;
-      }
-    }
-    if (ovf_hi > ovf_lo) {
-      if (tid == 0)
-        for (uint32_t k = ovf_lo; k < ovf_hi; ++k) row(k, kind);
-      t.sync();
+      sweep_in(warm, cache, use_bias);
     }
   };
-  sweep(0);
-  for (uint32_t it = 0; it < W.iterations; ++it) sweep(1);
-  // integrate positions (RB_sim.slang:1287-1326), same row quirk as advect
-  if (W.flags & BB_SIM_ADVECTION) {
-    uint32_t lim = N;
-    if (W.quirks & BB_QUIRK_ACTIVE_DISPATCH_ROWS) {
-      uint32_t r = ((A + 31u) / 32u) * 32u;
-      lim = r < N ? r : N;
+  sweep(std::true_type{}, false);
+  // I solves with bias, the position integration, then I relaxations
+  // (PGS_SOFT only, RB_sim.slang:1398-1402)
+  const uint32_t I = W.iterations, total = kPlain ? I : 2u * I;
+  for (uint32_t it = 0; it <= total; ++it) {
+    if (it == I) {
+      // integrate positions (RB_sim.slang:1287-1326), same row quirk as advect
+      if (W.flags & BB_SIM_ADVECTION) {
+        uint32_t lim = N;
+        if (W.quirks & BB_QUIRK_ACTIVE_DISPATCH_ROWS) {
+          uint32_t r = ((A + 31u) / 32u) * 32u;
+          lim = r < N ? r : N;
+        }
+        for (uint32_t i = tid; i < lim; i += NT) {
+          const uint32_t g = off + i;
+          uint32_t fl = d.cur.flags[g];
+          if (!((fl & BB_BODY_DYNAMIC) && !(fl & BB_BODY_SLEEPING))) continue;
+          const float* b = pgs_lds + kBodyLds * i;
+          const v3 v = i < ncache ? V(b[0], b[1], b[2]) : ld3(d.cur.vel[g]);
+          const v3 om = i < ncache ? V(b[4], b[5], b[6]) : ld3(d.cur.omg[g]);
+          const v3 p = ld3(d.cur.pos[g]);
+          d.cur.pos[g] = st3(p + v * W.dt, 0.0f);
+          d.cur.rot[g] = stq(apply_angular_velocity(ldq(d.cur.rot[g]), om, W.dt));
+        }
+      }
+      t.sync();
+      iw_refresh(d, W, t);
+      t.sync();
+      for (uint32_t i = tid; i < ncache; i += NT) cache.fill_iw(d, i);
+      t.sync();
     }
-    for (uint32_t i = tid; i < lim; i += NT) {
-      const uint32_t g = off + i;
-      uint32_t fl = d.cur.flags[g];
-      if (!((fl & BB_BODY_DYNAMIC) && !(fl & BB_BODY_SLEEPING))) continue;
-      v3 v, om;
-      vc.load(d, i, v, om);
-      const v3 p = ld3(d.cur.pos[g]);
-      d.cur.pos[g] = st3(p + v * W.dt, 0.0f);
-      d.cur.rot[g] = stq(apply_angular_velocity(ldq(d.cur.rot[g]), om, W.dt));
-    }
+    if (it < total) sweep(std::false_type{}, it < I);
   }
-  t.sync();
-  iw_refresh(d, W, t);
-  t.sync();
-  for (uint32_t i = tid; i < vc.lcap; i += NT) {
-    const uint32_t g = off + i;
-    pgs_lds[kBodyLds * i + 2] = d.iw[g * 3];
-    pgs_lds[kBodyLds * i + 3] = d.iw[g * 3 + 1];
-    pgs_lds[kBodyLds * i + 4] = d.iw[g * 3 + 2];
-  }
-  t.sync();
-  // relaxation sweeps: PGS_SOFT only (RB_sim.slang:1398-1402)
-  if (!s.plain)
-    for (uint32_t it = 0; it < W.iterations; ++it) sweep(2);
-  for (uint32_t i = tid; i < vc.lcap; i += NT) {
-    d.cur.vel[off + i] = pgs_lds[kBodyLds * i];
-    d.cur.omg[off + i] = pgs_lds[kBodyLds * i + 1];
+  for (uint32_t i = tid; i < ncache; i += NT) {
+    const float* b = pgs_lds + kBodyLds * i;
+    d.cur.vel[off + i] = make_float4(b[0], b[1], b[2], 0.0f);
+    d.cur.omg[off + i] = make_float4(b[4], b[5], b[6], 0.0f);
   }
   // impulses and pre-step quantities back into the manifold slots (warm start
   // of the next step, taps)
@@ -3442,18 +3662,18 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float4* pgs_lds, uint32_t
     const Soft sc = (h.z & 1024) ? s.soft[1] : s.soft[0];
     const float mass_coef = sc.mass_coef, bias_factor = sc.bias_factor, impulse_coef = sc.impulse_coef;
     for (int c = 0; c < (h.z & 255); ++c) {
-      const float4 l = d.sv_l[c * NP + row];
-      const float nm = d.sv_r2[c * NP + row].w, tm1 = d.sv_tm1[c * NP + row];
+      const v3 l = reinterpret_cast<const v3*>(d.sv_l)[c * NP + row];
+      const v3 m = reinterpret_cast<const v3*>(d.sv_m)[c * NP + row];  // normal mass, tangent masses
       if (s.plain) {
         // PGS::pre_step leaves the soft coefficients as the narrow phase set
         // them
         const float mc = d.man_cur.clam[slot * 8 + c].w;
-        d.man_cur.clam[slot * 8 + c] = make_float4(l.x, l.y, l.z, mc);
-        d.man_cur.cmas[slot * 8 + c] = make_float4(nm, l.w, tm1, plain_bias(d.sv_r1[c * NP + row].w, s.inv_dt));
+        d.man_cur.clam[slot * 8 + c] = st3(l, mc);
+        d.man_cur.cmas[slot * 8 + c] = st3(m, plain_bias(d.sv_cp[c * NP + row].w, s.inv_dt));
         continue;
       }
-      d.man_cur.clam[slot * 8 + c] = make_float4(l.x, l.y, l.z, mass_coef);
-      d.man_cur.cmas[slot * 8 + c] = make_float4(nm, l.w, tm1, bias_factor);
+      d.man_cur.clam[slot * 8 + c] = st3(l, mass_coef);
+      d.man_cur.cmas[slot * 8 + c] = st3(m, bias_factor);
       float4 a = d.man_cur.cana[slot * 8 + c];
       a.w = impulse_coef;
       d.man_cur.cana[slot * 8 + c] = a;
@@ -3463,7 +3683,7 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float4* pgs_lds, uint32_t
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_pgs(Dev d) {
-  HIP_DYNAMIC_SHARED(float4, pgs_lds)
+  HIP_DYNAMIC_SHARED(float, pgs_lds)
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{nullptr, nullptr};
@@ -3472,7 +3692,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_pgs(Dev d) {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_pgs_island(Dev d) {
-  HIP_DYNAMIC_SHARED(float4, pgs_lds)
+  HIP_DYNAMIC_SHARED(float, pgs_lds)
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{nullptr, nullptr};
@@ -4275,7 +4495,7 @@ struct FusedShared {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
-  HIP_DYNAMIC_SHARED(float4, pgs_lds)
+  HIP_DYNAMIC_SHARED(float, pgs_lds)
   __shared__ FusedShared<BLOCK> G;
   __shared__ ScanLds<BLOCK> S;
   const uint32_t w = d.order[blockIdx.x];
@@ -4489,6 +4709,16 @@ template <int B>
 void launch_fused_b(const Lane& l, hipStream_t st);
 
 #ifdef BB_BLOCK_TU
+// Which ranges of the colour sweeps go to quads of lanes (see pgs_solve): with
+// a CU for every workgroup, or when asked for, every range that the workgroup
+// has quads for; otherwise only ranges that fill no more than one wave of
+// quads, since a crowded CU is bound by the instructions of all its waves.
+template <int B>
+Dev sweep_form(const Dev& d, uint32_t grid) {
+  Dev r = d;
+  r.pgs_quad_rows = d.pgs_quads || grid <= 256u ? (uint32_t)B / 4u : 16u;
+  return r;
+}
 // Stages of the per-world path, in launch order (k_team, when there is one,
 // goes before the first).  Stage k of the timed launch is bracketed by events
 // ev[k] and ev[k + 1]; the narrow phase's two kernels share stage 2; the
@@ -4508,7 +4738,8 @@ void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid) {
     case 3: hipLaunchKernelGGL(k_post<B>, g, b, 0, st, d); break;
     case 4:
       if (d.any_island) hipLaunchKernelGGL(k_levels<B>, g, b, 0, st, d);
-      if (d.any_island) hipLaunchKernelGGL(k_pgs_island<B>, g, b, (size_t)d.pgs_lcap * 16 * kBodyLds, st, d);
+      if (d.any_island)
+        hipLaunchKernelGGL(k_pgs_island<B>, g, b, (size_t)d.pgs_lcap * kBodyLds * 4, st, sweep_form<B>(d, grid));
       break;
     case 5: hipLaunchKernelGGL(k_avbd<B>, g, b, 0, st, d); break;
     default: hipLaunchKernelGGL(k_finish<B>, g, b, 0, st, d); break;
@@ -4516,11 +4747,12 @@ void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid) {
 }
 template <int B>
 void launch_pgs_b(const Dev& d, hipStream_t st, uint32_t grid) {
-  hipLaunchKernelGGL(k_pgs<B>, dim3(grid), dim3(B), (size_t)d.pgs_lcap * 16 * kBodyLds, st, d);
+  hipLaunchKernelGGL(k_pgs<B>, dim3(grid), dim3(B), (size_t)d.pgs_lcap * kBodyLds * 4, st, sweep_form<B>(d, grid));
 }
 template <int B>
 void launch_fused_b(const Lane& l, hipStream_t st) {
-  hipLaunchKernelGGL(k_fused<B>, dim3(l.grid), dim3(B), (size_t)l.d.pgs_lcap * 16 * kBodyLds, st, l.d);
+  hipLaunchKernelGGL(k_fused<B>, dim3(l.grid), dim3(B), (size_t)l.d.pgs_lcap * kBodyLds * 4, st,
+                     sweep_form<B>(l.d, l.grid));
 }
 template void launch_stage_b<BB_BLOCK>(int, const Dev&, hipStream_t, uint32_t);
 template void launch_pgs_b<BB_BLOCK>(const Dev&, hipStream_t, uint32_t);

@@ -581,11 +581,12 @@ typedef enum bb_param {
                                 4 or 8; 0 = the default 4).  The partial
                                 sums are added in manifold order whatever
                                 the value, so results do not change        */
-  BB_PARAM_PGS_PREFETCH = 11, /* the PGS colour-sweep tile: 1 = each thread
-                                fetches its row of the next colour while it
-                                solves this colour's row (the next colour's
-                                rows are written by nobody else meanwhile);
-                                0 (default) = fetch where solved            */
+  BB_PARAM_PGS_PREFETCH = 11, /* the PGS colour-sweep tile: 1 = a row is
+                                solved by four lanes whenever the workgroup
+                                has enough of them; 0 (default) = that form
+                                while the launch has a CU for every world,
+                                one lane per row otherwise.  The next row is
+                                fetched while one is solved either way      */
   BB_PARAM_WALK_BUDGET = 12, /* broad phase: tree nodes one thread walks for
                                 its body before the body is handed to its
                                 whole workgroup (up to 64 bodies per world;

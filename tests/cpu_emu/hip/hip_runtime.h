@@ -104,6 +104,16 @@ static inline T __shfl_down(T v, unsigned d, int width = 64) {
 }
 static inline uint64_t __ballot(int p) { return emu::wave_op(EMU_BALLOT, p ? 1 : 0, 0, 64); }
 
+// DPP moves with all rows and banks enabled: quad permutations (control below
+// 256), and shifts left within rows of 16 (0x100 + n)
+static inline int emu_mov_dpp(int v, int ctrl) {
+  const int lane = (int)(threadIdx.x & 63u);
+  if (ctrl < 256) return __shfl(v, (ctrl >> (2 * (lane & 3))) & 3, 4);
+  return __shfl_down(v, (unsigned)(ctrl & 15), 16);
+}
+#define __builtin_amdgcn_mov_dpp(v, ctrl, row_mask, bank_mask, bound) emu_mov_dpp((v), (ctrl))
+#define __builtin_amdgcn_readlane(v, l) __shfl((v), (l), 64)
+
 static inline int __popc(uint32_t x) { return __builtin_popcount(x); }
 static inline int __popcll(uint64_t x) { return __builtin_popcountll(x); }
 static inline int __ffs(uint32_t x) { return __builtin_ffs((int)x); }

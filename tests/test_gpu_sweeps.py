@@ -1,0 +1,60 @@
+"""The PGS sweeps' two forms (a row per quad of lanes, a row per lane) and the
+places their body rows can lie (all in LDS, some, none) give the oracle's
+bits: sizes around a wave of quads, a workgroup of quads and a second round,
+the flags that change the contact's arithmetic, manifolds of more than four
+contacts and the serial bucket's rows included."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import beatbox
+import scenes
+from oracle_bind import OracleWorld
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("position", "rotation", "velocity", "omega", "flags")
+ACCUM, FRICTION = 1, 2
+
+
+def _flags():
+    f = scenes.SIM_DEFAULT_FLAGS
+    return (f, f & ~ACCUM, f & ~FRICTION, f & ~(ACCUM | FRICTION))
+
+
+@pytest.mark.parametrize("pgs_block,lds,quads", [(64, 0, 0), (64, 16, 1), (128, 512, 0), (256, 40, 1), (512, 512, 1),
+                                                 (1024, 64, 0)])
+def test_sweep_forms_equal_oracle(pgs_block, lds, quads):
+    sizes = (1, 9, 17, 40, 70, 150, 260)
+    b = beatbox.Batch()
+    b.set_param(beatbox.PARAM_BLOCK, 256)
+    b.set_param(beatbox.PARAM_PGS_BLOCK, pgs_block)
+    b.set_param(beatbox.PARAM_PGS_LDS_ROWS, lds)
+    b.set_param(beatbox.PARAM_PGS_PREFETCH, quads)
+    oracles = []
+    for k, n in enumerate(sizes):
+        for m, flags in enumerate(_flags()):
+            solver = scenes.SOLVER_PGS if (k + m) % 3 == 0 else scenes.SOLVER_PGS_SOFT
+            if solver == scenes.SOLVER_PGS:  # plain PGS: the per-island path
+                flags &= ~scenes.SIM_USE_GRAPH_COLORING
+            d = beatbox.WorldDesc.make(**scenes.world_desc(solver=solver, iterations=3 + m, flags=flags,
+                                                           morton_bits=63, quirks=0))
+            bodies = scenes.random_boxes(100 + 10 * k + m, n, extent=max(1.0, 0.5 * n ** 0.5), y0=0.55, y1=2.5)
+            b.add_world(d, bodies)
+            o = OracleWorld(d)
+            o.add_bodies(bodies)
+            oracles.append((o, len(bodies)))
+    # 300 more worlds make the launch a crowded one: ranges over a wave of
+    # quads go to single lanes
+    tiny = beatbox.WorldDesc.make(**scenes.world_desc(iterations=2, morton_bits=63, quirks=0))
+    for k in range(300):
+        b.add_world(tiny, scenes.random_boxes(5000 + k, 2, extent=0.6, y0=0.55, y1=1.5))
+    for steps in (1, 4):
+        b.step(steps)
+        b.sync(allow_overflow=True)
+        for w, (o, n) in enumerate(oracles):
+            o.step(steps)
+            g, r = b.read_world(w, n), o.read_bodies()
+            for f in FIELDS:
+                assert np.array_equal(g[f], r[f]), (w, n, f)
