@@ -195,7 +195,7 @@ bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_
   d.sv_cp = A.alloc<float4>((size_t)NP * 8);
   d.sv_m = A.alloc<float>((size_t)NP * 32);
   d.sv_l = A.alloc<float>((size_t)NP * 32);
-  d.sv_t0z = A.alloc<float>((size_t)NP * 8);
+  d.sv_list = A.alloc<uint32_t>((size_t)NP * 8);
   d.s_pos0 = A.alloc<float4>(NB);
   d.s_rot0 = A.alloc<float4>(NB);
   d.s_post = A.alloc<float4>(NB);
@@ -212,7 +212,6 @@ bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_
   d.ovf_any = A.alloc<uint32_t>(1);
   d.team_spin = b->team_spin;
   d.sort_blocks = b->sort_blocks;
-  d.avbd_lanes = b->avbd_lanes;
   d.pgs_quads = b->pgs_prefetch;
   d.pgs_quad_rows = 0;  // set per launch
   d.walk_budget = b->walk_budget;
@@ -1395,7 +1394,7 @@ bb_status set_param(bb_batch* b, bb_param p, uint32_t value) {
     b->base.team_spin = value;
   } else if (p == BB_PARAM_AVBD_LANES) {
     if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8) return BB_ERR_INVALID;
-    b->avbd_lanes = b->base.avbd_lanes = value;
+    b->avbd_lanes = value;
   } else if (p == BB_PARAM_PGS_PREFETCH) {
     if (value > 1) return BB_ERR_INVALID;
     b->pgs_prefetch = b->base.pgs_quads = value;
@@ -1489,7 +1488,7 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
   };
   float best = 3.4e38f;
   uint32_t best_block = saved_block, best_lds = saved_lds;
-  const uint32_t saved_fused = b->fused, saved_sort = b->sort_blocks, saved_lanes = b->avbd_lanes,
+  const uint32_t saved_fused = b->fused, saved_sort = b->sort_blocks,
                  saved_prefetch = b->pgs_prefetch,
                  saved_team_blocks = b->team_blocks, saved_pgs_block = b->pgs_block;
   bb_status rc = BB_OK;
@@ -1513,12 +1512,8 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
     if (rc != BB_OK) break;
   }
   // then, one at a time from the best so far: one launch per step or per
-  // stage; the solver tile of the per-world AVBD sweeps (lanes per body)
-  // when a world runs AVBD in them; the sort's sub-team when a world runs
-  // as a workgroup team
-  bool any_avbd = false;
-  for (const WorldInfo& wi : b->infos)
-    if (wi.solver == BB_SOLVER_AVBD && !(wi.mode & kModeTeam) && wi.n) any_avbd = true;
+  // stage; the form of the colour sweeps; the sort's sub-team and the launch
+  // size when a world runs as a workgroup team
   if (rc == BB_OK) {
     b->block = best_block;
     b->pgs_lds = best_lds;
@@ -1574,10 +1569,6 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
   for (const WorldInfo& wi : b->infos)
     if (wi.solver != BB_SOLVER_AVBD && wi.n) any_pgs = true;
   if (any_pgs) tune(b->pgs_prefetch, &b->base.pgs_quads, {0u, 1u});
-  if (any_avbd) {
-    if (b->avbd_lanes == 0) b->avbd_lanes = b->base.avbd_lanes = 4;
-    tune(b->avbd_lanes, &b->base.avbd_lanes, {1u, 2u, 4u, 8u});
-  }
   if (b->base.team_grid) {
     if (b->sort_blocks == 0) b->sort_blocks = b->base.sort_blocks = kTeamSortBlocks;
     tune(b->sort_blocks, &b->base.sort_blocks, {8u, 16u, 32u, 64u, 128u});
@@ -1603,7 +1594,6 @@ bb_status autotune_batch(bb_batch* b, uint32_t reps, float* best_ms) {
     b->team_blocks = saved_team_blocks;
     b->fused = saved_fused;
     b->sort_blocks = b->base.sort_blocks = saved_sort;
-    b->avbd_lanes = b->base.avbd_lanes = saved_lanes;
     b->pgs_prefetch = b->base.pgs_quads = saved_prefetch;
   }
   (void)hipEventDestroy(e0);

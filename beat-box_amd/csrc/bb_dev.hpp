@@ -203,7 +203,7 @@ struct Dev {
   float4* sv_cp;      // [8*np] contact point, penetration
   float* sv_m;        // [8*np*3] normal mass, tangent masses 0 and 1 (the arrays
   float* sv_l;        // [8*np*3] normal/tangent impulses        hold 8*np float4)
-  float* sv_t0z;      // [np] first tangent's z (sized like the contact arrays)
+  uint32_t* sv_list;  // [8*np] AVBD: the world's contacts, slot * 8 + contact
   // AVBD
   float4* s_pos0;     // [body] pos_start, w = support depth bits
   float4* s_rot0;
@@ -228,7 +228,6 @@ struct Dev {
   uint32_t team_vox;      // a team world holds voxel bodies (the k_team instance with their narrow phase)
   uint32_t team_spin;     // spins before a team barrier wait gives up (0: default)
   uint32_t sort_blocks;   // workgroups of a team that sort (0: kTeamSortBlocks)
-  uint32_t avbd_lanes;    // lanes per body in the per-world AVBD primal sweeps (1, 2, 4, 8; 0: 4)
   uint32_t pgs_quads;     // 1: sweep by quads of lanes whenever the workgroup has enough
   uint32_t pgs_quad_rows; // ranges of at most this many rows are swept by quads of lanes, longer ones by lanes
   uint32_t walk_budget;   // nodes a broad-phase thread walks before its workgroup takes the row

@@ -159,7 +159,7 @@ struct bb_batch {
   uint32_t pair_scale = 1;   // BB_PARAM_PAIR_SCALE: pair slots per world, times the default
   uint32_t fused = 0;        // BB_PARAM_FUSED: each lane's step as one k_fused launch
   uint32_t sort_blocks = 0;  // BB_PARAM_SORT_BLOCKS (0: kTeamSortBlocks)
-  uint32_t avbd_lanes = 0;   // BB_PARAM_AVBD_LANES (0: 4)
+  uint32_t avbd_lanes = 0;   // BB_PARAM_AVBD_LANES (0: 4), kept for the caller
   uint32_t pgs_prefetch = 0; // BB_PARAM_PGS_PREFETCH
   uint32_t walk_budget = 0;  // BB_PARAM_WALK_BUDGET (0: kWalkBudgetDefault)
   uint32_t team_blocks = 0;  // BB_PARAM_TEAM_BLOCKS (0: half the resident workgroups)

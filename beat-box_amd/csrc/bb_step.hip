@@ -26,9 +26,6 @@
 namespace bb {
 
 #define WAVE 64
-// Lanes per body in the AVBD primal sweeps of the per-world kernels (the
-// default of BB_PARAM_AVBD_LANES) and of workgroup teams.
-static constexpr uint32_t kAvG = 4, kAvGTeam = 8;
 
 // ============================================================ block helpers
 template <int BLOCK>
@@ -264,8 +261,7 @@ template <int BLOCK>
 struct BlockTeam {
   ScanLds<BLOCK>* scan_lds;
   SortLds<BLOCK>* sort_lds;
-  // AVBD primal: kAvG lanes per body; empty cascade buckets skip their barrier
-  static constexpr uint32_t kAvGroup = kAvG;
+  // empty AVBD cascade buckets skip their barrier
   static constexpr bool kSkipEmpty = true;
   static constexpr bool kGlobalScalars = false;  // stage scalars in LDS
   static constexpr int kBlock = BLOCK;
@@ -311,11 +307,8 @@ struct GroupTeam {
   uint32_t spin;   // spins before a wait gives up
   unsigned long long* clk;  // this team's clock marks (profiling launches), or null
   uint32_t sort_blocks;     // the first sort_blocks workgroups run the radix sort
-  // AVBD primal: kAvGTeam lanes per body (a pile's bodies have half a dozen
-  // manifolds, so eight lanes take about one each); empty cascade buckets
-  // skip their barrier (the bucket offsets are team scalars every workgroup
-  // reads after the same barrier, so all of them skip the same buckets)
-  static constexpr uint32_t kAvGroup = kAvGTeam;
+  // empty AVBD cascade buckets skip their barrier (every workgroup reads the
+  // bucket offsets after the same barrier, so all of them skip the same ones)
   static constexpr bool kSkipEmpty = true;
   static constexpr bool kGlobalScalars = true;  // stage scalars in a global slot
   static constexpr int kBlock = BLOCK;
@@ -3073,9 +3066,9 @@ BB_DI void pgs_compact(const Dev& d, const WorldInfo& W, uint32_t k, uint32_t sl
   d.sv_hdr[k] = make_int4(h.x, h.y, h.w | (da ? 256 : 0) | (db ? 512 : 0) | (soft_static ? 1024 : 0),
                           __float_as_int(__builtin_sqrtf(fa * fb)));
   // one component of the first tangent is zero (compute_basis); the sweeps
-  // take the others from here
+  // take the others from n.w and the colouring's scratch word of the slot
   d.sv_n[k] = st3(n, fab(n.x) > fab(n.y) ? t0.x : t0.y);
-  d.sv_t0z[k] = t0.z;
+  d.pick[k] = __float_as_uint(t0.z);
 }
 
 // ---- the sweeps.  A colour phase of a world is one row's chain of
@@ -3232,7 +3225,7 @@ struct PgsRows {
   float* l;
   uint32_t np;
   BB_DI PgsRows(const Dev& d, uint32_t base)
-      : hdr(d.sv_hdr + base), n(reinterpret_cast<const float*>(d.sv_n + base)), t0z(d.sv_t0z + base),
+      : hdr(d.sv_hdr + base), n(reinterpret_cast<const float*>(d.sv_n + base)), t0z(reinterpret_cast<const float*>(d.pick + base)),
         cp(reinterpret_cast<const float*>(d.sv_cp + base)), m(d.sv_m + (size_t)base * 3u), l(d.sv_l + (size_t)base * 3u),
         np(d.np) {}
   // contact c's entries: float4 (cp), three floats (m, l)
@@ -3767,262 +3760,291 @@ BB_DI void avbd_solve6(float H[6][6], float b[6], float x[6]) {
   }
 }
 
-struct AvBody {  // pose and step-start state of one side of a contact
-  bool dyn;
-  v3 pos;
-  qt rot;
-  v3 p0;
-  qt q0;
+// What the sweeps of an AVBD world read, prepared once per step (nothing of
+// it changes between the sweeps):
+//  - per body row: step-start pose (s_pos0, s_rot0; immovable and sleeping
+//    rows hold their pose), mass and body inverse inertia in row order (iw0,
+//    iw1, iw2);
+//  - per manifold: rows, contact count and who moves, friction (hdr);
+//  - per contact: the anchors turned by the step-start rotations (ar1, ar2)
+//    and their step-start offsets along the tangents (c0t);
+//  - per body its contacts in ascending (manifold, contact) order (item), and
+//    all contacts of the world (all): slot of the world * 8 + contact.
+// The pose's change since the step start (dp, dth) is kept per row beside
+// pos and rot, with whether the row moves in dp.w: a neighbour reads two
+// vectors instead of two poses, and computes nothing with them.
+// The arrays are those of the PGS rows and of the cached inertia, which an
+// AVBD world has no use for: a world's part of each is the same for both.
+struct AvData {
+  float4 *dp, *dth;         // [row * 3]
+  float4 *iw0, *iw1, *iw2;  // [row]
+  int4* hdr;                // [slot]
+  v3 *ar1, *ar2;            // [contact * np + slot]
+  float2* c0t;              // [2 * (contact * np + slot)]
+  uint32_t *list0, *list1;  // first 8 * cap and the remaining list entries
+  uint32_t* all;
+  uint32_t np, cap8;
+  BB_DI AvData(const Dev& d, const WorldInfo& W) {
+    dp = d.iw + 3u * (size_t)W.body_off;
+    dth = dp + 1;
+    iw0 = d.sv_n + W.pair_off;  // 3 n <= pair_cap
+    iw1 = iw0 + W.n;
+    iw2 = iw1 + W.n;
+    hdr = d.sv_hdr + W.pair_off;
+    np = d.np;
+    ar1 = reinterpret_cast<v3*>(d.sv_m) + W.pair_off;
+    ar2 = reinterpret_cast<v3*>(d.sv_l) + W.pair_off;
+    c0t = reinterpret_cast<float2*>(d.sv_cp + W.pair_off);
+    // the arrays hold 8 * np float4; contacts take 8 * np * 3 floats of them
+    list0 = reinterpret_cast<uint32_t*>(d.sv_m + 24u * (size_t)np + 8u * (size_t)W.pair_off);
+    list1 = reinterpret_cast<uint32_t*>(d.sv_l + 24u * (size_t)np + 8u * (size_t)W.pair_off);
+    all = d.sv_list + 8u * (size_t)W.pair_off;
+    cap8 = 8u * W.pair_cap;
+  }
+  BB_DI size_t at(uint32_t slot, uint32_t j) const { return (size_t)j * np + slot; }
+  BB_DI uint32_t& item(uint32_t x) const { return x < cap8 ? list0[x] : list1[x - cap8]; }
 };
-BB_DI AvBody av_body(const Dev& d, uint32_t g) {
-  AvBody b;
-  uint32_t fl = d.cur.flags[g];
-  b.dyn = (fl & BB_BODY_DYNAMIC) && !(fl & BB_BODY_SLEEPING);
-  b.pos = ld3(d.cur.pos[g]);
-  b.rot = ldq(d.cur.rot[g]);
-  if (b.dyn) {
-    b.p0 = ld3(d.s_pos0[g]);
-    b.q0 = ldq(d.s_rot0[g]);
-  } else {
-    b.p0 = b.pos;
-    b.q0 = b.rot;
-  }
-  return b;
+
+// One contact of a manifold between rows h.x and h.y (rows of the world,
+// slots of the world): what both the primal and the dual update read of it.
+struct AvContact {
+  v3 n, t0, t1;
+  v3 p, ar1, ar2;
+  float pen;
+  float2 c0t;
+  float4 lm, cm;
+};
+BB_DI AvContact av_contact(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t slot, uint32_t j) {
+  const uint32_t g = W.pair_off + slot, cs = g * 8u + j;
+  AvContact c;
+  const float4 cp = d.man_cur.cpos[cs];
+  c.lm = d.man_cur.clam[cs];
+  c.cm = d.man_cur.cmas[cs];
+  c.ar1 = D.ar1[D.at(slot, j)];
+  c.ar2 = D.ar2[D.at(slot, j)];
+  c.c0t = D.c0t[2u * D.at(slot, j)];
+  c.n = ld3(d.man_cur.nrm[g]);
+  c.t0 = ld3(d.man_cur.t0[g]);
+  c.t1 = ld3(d.man_cur.t1[g]);
+  c.p = ld3(cp);
+  c.pen = cp.w;
+  return c;
 }
-// avbd_contact_C (avbd.slang:232-258)
-BB_DI float av_contact_C(v3 n, v3 p, float pen, const AvBody& b1, const AvBody& b2, float alpha, v3& rr1,
-                         v3& rr2) {
-  rr1 = p - b1.p0;
-  rr2 = p - b2.p0;
-  float C0 = pen + AV_MARGIN;
-  float C = C0 * (1.0f - alpha);
-  if (b1.dyn) {
-    v3 dp1 = b1.pos - b1.p0;
-    v3 dth1 = small_angle_delta(b1.rot, b1.q0);
-    C -= dot(n, dp1 + cross(dth1, rr1));
-  }
-  if (b2.dyn) {
-    v3 dp2 = b2.pos - b2.p0;
-    v3 dth2 = small_angle_delta(b2.rot, b2.q0);
-    C += dot(n, dp2 + cross(dth2, rr2));
-  }
+// avbd_contact_C and avbd_dir_C (avbd.slang:232-305) of the contact's three
+// rows; s1, s2 are the rows' values dot(dir, dp + cross(dth, arm)) of the two
+// bodies, taken in when the body moves.
+BB_DI float av_C(float c0, float alpha, bool d1, float s1, bool d2, float s2) {
+  float C = c0 * (1.0f - alpha);
+  C = d1 ? C - s1 : C;
+  C = d2 ? C + s2 : C;
   return C;
 }
-// avbd_dir_C (avbd.slang:274-305)
-BB_DI float av_dir_C(v3 dir, v3 anc_a, v3 anc_b, const AvBody& b1, const AvBody& b2, float alpha, v3& ar1,
-                     v3& ar2, float& C0t) {
-  ar1 = avbd_q_rotate(b1.q0, anc_a);
-  ar2 = avbd_q_rotate(b2.q0, anc_b);
-  C0t = dot(dir, (b2.p0 + ar2) - (b1.p0 + ar1));
-  float c0e = fsign(C0t) * fmx(0.0f, fab(C0t) - AV_STICK_SLOP);
-  float C = c0e * (1.0f - alpha);
-  if (b1.dyn) {
-    v3 dp1 = b1.pos - b1.p0;
-    v3 dth1 = small_angle_delta(b1.rot, b1.q0);
-    C -= dot(dir, dp1 + cross(dth1, ar1));
-  }
-  if (b2.dyn) {
-    v3 dp2 = b2.pos - b2.p0;
-    v3 dth2 = small_angle_delta(b2.rot, b2.q0);
-    C += dot(dir, dp2 + cross(dth2, ar2));
-  }
-  return C;
+BB_DI float av_c0e(float c0t) { return fsign(c0t) * fmx(0.0f, fab(c0t) - AV_STICK_SLOP); }
+
+// Lanes of a wave that share LDS words: every lane's writes before, every
+// lane's reads after.
+BB_DI void group_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// entry_avbd_primal (avbd.slang:475-658) for row i, by a group of G lanes
-// (lane = 0..G-1; G = 1, 2, 4 or 8 in the per-world kernels, a launch
-// parameter, and 1 in teams).  The
-// Hessian and gradient are the inertial terms plus one partial sum per
-// incident manifold, added in ascending manifold order (the adjacency
-// order); lane e % G assembles manifold e, so the dependent loads of G
-// manifolds are in flight together.  Only the lower triangle of H is formed:
-// avbd_solve6 reads no other entry.
-static constexpr int kAvH = 21;  // lower-triangle entries of the 6x6 H
-BB_DI void av_manifold_terms(const Dev& d, const WorldInfo& W, uint32_t i, uint32_t slot, float alpha,
-                             float (&He)[kAvH], float (&ge)[6]) {
-  const uint32_t off = W.body_off;
-  const int4 h = d.man_cur.hdr[slot];
-  const uint32_t b1 = (uint32_t)h.x, b2 = (uint32_t)h.y;
-  const bool i1 = b1 == i;
-  const AvBody B1 = av_body(d, off + b1), B2 = av_body(d, off + b2);
-  const float f1 = d.props.mass[off + d.cur.id[off + b1]].z, f2 = d.props.mass[off + d.cur.id[off + b2]].z;
-  const float mu = __builtin_sqrtf(fmx(f1, 0.0f) * fmx(f2, 0.0f));
-  const v3 n = ld3(d.man_cur.nrm[slot]);
-  const v3 tdir[2] = {ld3(d.man_cur.t0[slot]), ld3(d.man_cur.t1[slot])};
-#pragma unroll
-  for (int q = 0; q < kAvH; ++q) He[q] = 0.0f;
-#pragma unroll
-  for (int a = 0; a < 6; ++a) ge[a] = 0.0f;
-  auto add_row = [&](float k, float f, const float (&J)[6]) {
-#pragma unroll
-    for (int a = 0; a < 6; ++a) ge[a] += f * J[a];
-    int q = 0;
-#pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-      for (int b = 0; b <= a; ++b) He[q++] += k * J[a] * J[b];
-  };
-  for (int j = 0; j < h.w; ++j) {
-    const uint32_t cs = slot * 8 + j;
-    const float4 cp = d.man_cur.cpos[cs];
-    const float4 lm = d.man_cur.clam[cs];
-    const float4 cmv = d.man_cur.cmas[cs];
-    const v3 anc_a = ld3(d.man_cur.cana[cs]), anc_b = ld3(d.man_cur.canb[cs]);
-    v3 rr1, rr2;
-    const float C = av_contact_C(n, ld3(cp), cp.w, B1, B2, alpha, rr1, rr2);
-    const float lam = lm.x, kk = lm.w;
-    const float f = fmn(kk * C + lam, 0.0f);
-    const v3 Jl = i1 ? -n : n;
-    const v3 Ja = i1 ? -cross(rr1, n) : cross(rr2, n);
-    const float J[6] = {Jl.x, Jl.y, Jl.z, Ja.x, Ja.y, Ja.z};
-    add_row(kk, f, J);
-    const float bound = mu * fab(lam);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const v3 td = tdir[t];
-      v3 ar1, ar2;
-      float C0t;
-      const float Ct = av_dir_C(td, anc_a, anc_b, B1, B2, alpha, ar1, ar2, C0t);
-      const float lt = t == 0 ? lm.y : lm.z;
-      const float kt = t == 0 ? cmv.y : cmv.z;
-      const float ft = fcl(kt * Ct + lt, -bound, bound);
-      const v3 Jlt = i1 ? -td : td;
-      const v3 Jat = i1 ? -cross(ar1, td) : cross(ar2, td);
-      const float Jt[6] = {Jlt.x, Jlt.y, Jlt.z, Jat.x, Jat.y, Jat.z};
-      add_row(kt, ft, Jt);
-    }
-  }
-}
-
-template <uint32_t G>
-BB_DI void av_primal(const Dev& d, const WorldInfo& W, uint32_t i, float alpha, uint32_t lane) {
+// entry_avbd_primal (avbd.slang:475-658) for row i, by a group of kAvGroup
+// lanes (l: this lane's place).  The Hessian and gradient are the inertial
+// terms plus one partial sum per incident manifold, added in ascending
+// manifold order.  Lane l evaluates the body's contacts l, l + 8, ...: three
+// constraint rows each, left in the group's LDS words (rec) as Jacobian,
+// stiffness and force.  Then lane a < 6 sums row a of H and entry a of the
+// gradient over all rows in order: a wave issues an instruction every 8 or
+// more cycles whatever its lanes do, so a body's time is its instructions,
+// and here eight lanes share both the contacts and the sums (one lane per
+// manifold took four times as many on a manifold of four contacts, and the
+// sums went through 27 cross-lane moves per manifold).  avbd_solve6 reads the
+// lower triangle only.  Measured, per step, against one lane per manifold
+// that read both bodies' poses: 27 tower bodies 571 -> 330 us, a 1,501-body
+// world 4.1 -> 2.6 ms, the 20,000-body pile 8.2 -> 4.6 and the 100,000-body
+// pile 9.7 -> 6.2 ms.
+static constexpr uint32_t kAvGroup = 8;
+static constexpr uint32_t kAvRec = 8;                          // floats of a row's record
+static constexpr uint32_t kAvGroupLds = kAvGroup * 3 * kAvRec;  // LDS floats per group
+BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t i, float alpha, uint32_t l,
+                     float* rec) {
   const uint32_t off = W.body_off, g = off + i;
-  const uint32_t id = d.cur.id[g];
   const bool quirk = (W.quirks & BB_QUIRK_TRANSPOSED_WORLD_INERTIA) != 0;
   const float dt = W.dt;
   const float inv_dt2 = dt > 0.0f ? 1.0f / (dt * dt) : 0.0f;
+  const uint32_t c0 = d.poff[g], cn = d.pcount[g];
   v3 pos = ld3(d.cur.pos[g]);
   qt rot = ldq(d.cur.rot[g]);
-  const float m_lin = d.props.mass[off + id].x * inv_dt2;
-  const mat3 Iw = avbd_inverse3(world_inv_inertia(d, off + id, rot, quirk));
-  // inertial terms (every lane of the group holds all of H and g)
-  float Hi[kAvH], gi[6];
+  const v3 p0 = ld3(d.s_pos0[g]);
+  const qt q0 = ldq(d.s_rot0[g]);
+  const v3 dpo = ld3(D.dp[i * 3u]), dtho = ld3(D.dth[i * 3u]);
+  const float4 m0 = D.iw0[i], m1 = D.iw1[i], m2 = D.iw2[i];
+  // inertial terms: row l of H, entry l of the gradient
+  float H[6], gr;
   {
-    int q = 0;
-#pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-      for (int b = 0; b <= a; ++b) {
-        float v = 0.0f;
-        if (a == b && a < 3) v = m_lin;
-        if (a >= 3 && b >= 3) v = Iw.m[a - 3][b - 3] * inv_dt2;
-        Hi[q++] = v;
-      }
+    const float m_lin = m0.w * inv_dt2;
+    const mat3 I = mrows(ld3(m0), ld3(m1), ld3(m2));
+    const mat3 R = qmat(rot);
+    const mat3 Rt = mT(R);
+    const mat3 Iw = avbd_inverse3(quirk ? mmul(Rt, mmul(I, mT(Rt))) : mmul(R, mmul(I, mT(R))));
     const v3 dpos = pos - ld3(d.s_post[g]);
     const v3 dth = small_angle_delta(rot, ldq(d.s_rott[g]));
     const v3 ga = mulmv(Iw, dth) * inv_dt2;
-    gi[0] = m_lin * dpos.x; gi[1] = m_lin * dpos.y; gi[2] = m_lin * dpos.z;
-    gi[3] = ga.x; gi[4] = ga.y; gi[5] = ga.z;
+    const uint32_t r = l % 3u;  // lanes 0-2: position rows, 3-5: rotation rows
+    const bool ang = l >= 3u;
+    const float ix = r == 0u ? Iw.m[0][0] : (r == 1u ? Iw.m[1][0] : Iw.m[2][0]);
+    const float iy = r == 0u ? Iw.m[0][1] : (r == 1u ? Iw.m[1][1] : Iw.m[2][1]);
+    const float iz = r == 0u ? Iw.m[0][2] : (r == 1u ? Iw.m[1][2] : Iw.m[2][2]);
+    const float dl = r == 0u ? dpos.x : (r == 1u ? dpos.y : dpos.z);
+    const float gl = r == 0u ? ga.x : (r == 1u ? ga.y : ga.z);
+    H[0] = !ang && r == 0u ? m_lin : 0.0f;
+    H[1] = !ang && r == 1u ? m_lin : 0.0f;
+    H[2] = !ang && r == 2u ? m_lin : 0.0f;
+    H[3] = ang ? ix * inv_dt2 : 0.0f;
+    H[4] = ang ? iy * inv_dt2 : 0.0f;
+    H[5] = ang ? iz * inv_dt2 : 0.0f;
+    gr = ang ? gl : m_lin * dl;
   }
-  const uint32_t a0 = 2 * W.pair_off + d.adj_off[g], deg = d.deg[g];
-  for (uint32_t e0 = 0; e0 < deg; e0 += G) {
-    float He[kAvH], ge[6];
-    const uint32_t e = e0 + lane;
-    if (e < deg) av_manifold_terms(d, W, i, d.adj[a0 + e], alpha, He, ge);
-    if constexpr (G == 1) {
+  float he[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, ge = 0.0f;  // the manifold's partial sum
+  for (uint32_t r0 = 0; r0 < cn; r0 += kAvGroup) {
+    if (r0 + l < cn) {
+      const uint32_t w = D.item(c0 + r0 + l), slot = w >> 3, j = w & 7u;
+      const int4 h = D.hdr[slot];
+      const AvContact c = av_contact(d, W, D, slot, j);
+      const bool i1 = (uint32_t)h.x == i;
+      const uint32_t o = i1 ? (uint32_t)h.y : (uint32_t)h.x;
+      const float4 odp = D.dp[o * 3u];
+      const v3 dpx = ld3(odp), dthx = ld3(D.dth[o * 3u]), px = ld3(d.s_pos0[off + o]);
+      const bool omoves = odp.w != 0.0f;
+      const bool d1 = i1 || omoves, d2 = !i1 || omoves;
+      const v3 rro = c.p - p0, rrx = c.p - px;
+      const v3 aro = i1 ? c.ar1 : c.ar2, arx = i1 ? c.ar2 : c.ar1;
+      const v3 vo = dpo + cross(dtho, rro), vx = dpx + cross(dthx, rrx);
+      const v3 uo = dpo + cross(dtho, aro), ux = dpx + cross(dthx, arx);
+      float* out = rec + l * (3u * kAvRec);
+      auto put = [&](uint32_t t, v3 dir, v3 arm, float k, float f) __attribute__((always_inline)) {
+        const v3 cr = cross(arm, dir);
+        const v3 jl = i1 ? -dir : dir, ja = i1 ? -cr : cr;
+        float4* q = reinterpret_cast<float4*>(out + t * kAvRec);
+        q[0] = make_float4(jl.x, jl.y, jl.z, ja.x);
+        q[1] = make_float4(ja.y, ja.z, k, f);
+      };
+      const float lam = c.lm.x, kk = c.lm.w, bound = __int_as_float(h.w) * fab(lam);
+      {
+        const float so = dot(c.n, vo), sx = dot(c.n, vx);
+        const float C = av_C(c.pen + AV_MARGIN, alpha, d1, i1 ? so : sx, d2, i1 ? sx : so);
+        put(0, c.n, rro, kk, fmn(kk * C + lam, 0.0f));
+      }
+      auto tangent = [&](uint32_t t, v3 td, float c0t, float lt, float kt, uint32_t sign)
+                         __attribute__((always_inline)) {
+        const float so = dot(td, uo), sx = dot(td, ux);
+        const float C = av_C(av_c0e(c0t), alpha, d1, i1 ? so : sx, d2, i1 ? sx : so);
+        put(t, td, aro, __uint_as_float(__float_as_uint(kt) | sign), fcl(kt * C + lt, -bound, bound));
+      };
+      tangent(1, c.t0, c.c0t.x, c.lm.y, c.cm.y, 0u);
+      // stiffnesses are positive: the sign bit of the last row's marks the
+      // manifold's last contact
+      tangent(2, c.t1, c.c0t.y, c.lm.z, c.cm.z, j + 1u == ((uint32_t)h.z & 255u) ? 0x80000000u : 0u);
+    }
+    group_sync();
+    const uint32_t m = cn - r0 < kAvGroup ? cn - r0 : kAvGroup;
+    const uint32_t la = l < 6u ? l : 5u;
+    for (uint32_t c = 0; c < m; ++c) {
+      uint32_t kb = 0;
 #pragma unroll
-      for (int q = 0; q < kAvH; ++q) Hi[q] += He[q];
-#pragma unroll
-      for (int a = 0; a < 6; ++a) gi[a] += ge[a];
-    } else {
-      // add the group's partial sums in manifold order
-#pragma unroll
-      for (uint32_t src = 0; src < G; ++src) {
-        const bool has = e0 + src < deg;
-#pragma unroll
-        for (int q = 0; q < kAvH; ++q) {
-          const float v = __shfl(He[q], (int)src, (int)G);
-          if (has) Hi[q] += v;
-        }
+      for (uint32_t t = 0; t < 3; ++t) {
+        const float* q = rec + (c * 3u + t) * kAvRec;
+        const float4 qa = reinterpret_cast<const float4*>(q)[0], qb = reinterpret_cast<const float4*>(q)[1];
+        const float ja = q[la];
+        kb = __float_as_uint(qb.z);
+        const float k = t == 2u ? __uint_as_float(kb & 0x7FFFFFFFu) : qb.z;
+        const float kj = k * ja;
+        ge += qb.w * ja;
+        he[0] += kj * qa.x;
+        he[1] += kj * qa.y;
+        he[2] += kj * qa.z;
+        he[3] += kj * qa.w;
+        he[4] += kj * qb.x;
+        he[5] += kj * qb.y;
+      }
+      if (kb & 0x80000000u) {
 #pragma unroll
         for (int a = 0; a < 6; ++a) {
-          const float v = __shfl(ge[a], (int)src, (int)G);
-          if (has) gi[a] += v;
+          H[a] += he[a];
+          he[a] = 0.0f;
         }
+        gr += ge;
+        ge = 0.0f;
       }
     }
+    group_sync();
   }
-  if (lane != 0) return;
-  float H[6][6], rhs[6], dx[6];
-  {
-    int q = 0;
-#pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-      for (int b = 0; b < 6; ++b) H[a][b] = 0.0f;
-#pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-      for (int b = 0; b <= a; ++b) H[a][b] = Hi[q++];
+  // every lane solves the whole system
+  if (l < 6u) {
+    float4* q = reinterpret_cast<float4*>(rec + l * 8u);
+    q[0] = make_float4(H[0], H[1], H[2], H[3]);
+    q[1] = make_float4(H[4], H[5], gr, 0.0f);
   }
+  group_sync();
+  float A[6][6], rhs[6], dx[6];
 #pragma unroll
-  for (int a = 0; a < 6; ++a) rhs[a] = -gi[a];
-  avbd_solve6(H, rhs, dx);
+  for (int a = 0; a < 6; ++a) {
+    const float4* q = reinterpret_cast<const float4*>(rec + a * 8);
+    const float4 qa = q[0], qb = q[1];
+    A[a][0] = qa.x; A[a][1] = qa.y; A[a][2] = qa.z; A[a][3] = qa.w; A[a][4] = qb.x; A[a][5] = qb.y;
+    rhs[a] = -qb.z;
+  }
+  group_sync();  // the words are free for the group's next body
+  avbd_solve6(A, rhs, dx);
   pos = pos + V(dx[0], dx[1], dx[2]);
-  v3 half = V(dx[3], dx[4], dx[5]) * 0.5f;
+  const v3 half = V(dx[3], dx[4], dx[5]) * 0.5f;
   rot = qnorm(qmul(qt{half, 1.0f}, rot));
-  d.cur.pos[g] = st3(pos, 0.0f);
-  d.cur.rot[g] = stq(rot);
+  if (l == 0u) {
+    d.cur.pos[g] = st3(pos, 0.0f);
+    d.cur.rot[g] = stq(rot);
+    D.dp[i * 3u] = st3(pos - p0, 1.0f);
+    D.dth[i * 3u] = st3(small_angle_delta(rot, q0), 0.0f);
+  }
 }
 
-// entry_avbd_dual (avbd.slang:726-808) for one manifold slot
-BB_DI void av_dual(const Dev& d, const WorldInfo& W, uint32_t slot) {
-  const uint32_t off = W.body_off;
-  const int4 h = d.man_cur.hdr[slot];
-  const AvBody B1 = av_body(d, off + h.x), B2 = av_body(d, off + h.y);
-  if (!B1.dyn && !B2.dyn) return;
-  const float f1 = d.props.mass[off + d.cur.id[off + h.x]].z, f2 = d.props.mass[off + d.cur.id[off + h.y]].z;
-  const float mu = __builtin_sqrtf(fmx(f1, 0.0f) * fmx(f2, 0.0f));
-  const v3 n = ld3(d.man_cur.nrm[slot]);
-  const v3 tdir[2] = {ld3(d.man_cur.t0[slot]), ld3(d.man_cur.t1[slot])};
-  for (int j = 0; j < h.w; ++j) {
-    const uint32_t cs = slot * 8 + j;
-    const float4 cp = d.man_cur.cpos[cs];
-    float4 lm = d.man_cur.clam[cs];
-    float4 cmv = d.man_cur.cmas[cs];
-    float4 cb = d.man_cur.canb[cs];
-    const v3 anc_a = ld3(d.man_cur.cana[cs]), anc_b = ld3(cb);
-    v3 rr1, rr2;
-    float C = av_contact_C(n, ld3(cp), cp.w, B1, B2, 1.0f, rr1, rr2);
-    const float lam = lm.x, kk = lm.w;
-    const float nl = fmn(kk * C + lam, 0.0f);
-    lm.x = nl;
-    if (nl < 0.0f) lm.w = fmn(kk + AV_BETA * fab(C), AV_KMAX);
-    const float bound = mu * fab(lam);
-    bool stick_ok = true;
-    float drift2 = 0.0f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      v3 ar1, ar2;
-      float C0t;
-      float Ct = av_dir_C(tdir[t], anc_a, anc_b, B1, B2, 1.0f, ar1, ar2, C0t);
-      float lt = t == 0 ? lm.y : lm.z;
-      float kt = t == 0 ? cmv.y : cmv.z;
-      float nlt = fcl(kt * Ct + lt, -bound, bound);
-      if (t == 0) lm.y = nlt; else lm.z = nlt;
-      if (nlt > -bound && nlt < bound) {
-        float nk = fmn(kt + AV_BETA * fab(Ct), AV_KMAX);
-        if (t == 0) cmv.y = nk; else cmv.z = nk;
-      } else {
-        stick_ok = false;
-      }
-      drift2 += C0t * C0t;
-    }
-    cb.w = __uint_as_float((stick_ok && drift2 < AV_STICK_THRESH * AV_STICK_THRESH) ? 1u : 0u);
-    d.man_cur.clam[cs] = lm;
-    d.man_cur.cmas[cs] = cmv;
-    d.man_cur.canb[cs] = cb;
-  }
+// entry_avbd_dual (avbd.slang:726-808) for one contact.  The stick flag is
+// read by the next step only, so the last pass writes it (set_stick).
+BB_DI void av_dual(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t slot, uint32_t j, bool set_stick) {
+  const uint32_t off = W.body_off, cs = (W.pair_off + slot) * 8u + j;
+  const int4 h = D.hdr[slot];
+  const AvContact c = av_contact(d, W, D, slot, j);
+  const float4 p1 = D.dp[(uint32_t)h.x * 3u], p2 = D.dp[(uint32_t)h.y * 3u];
+  const v3 th1 = ld3(D.dth[(uint32_t)h.x * 3u]), th2 = ld3(D.dth[(uint32_t)h.y * 3u]);
+  const v3 x1 = ld3(d.s_pos0[off + h.x]), x2 = ld3(d.s_pos0[off + h.y]);
+  const bool d1 = p1.w != 0.0f, d2 = p2.w != 0.0f;
+  if (!d1 && !d2) return;
+  const v3 v1 = ld3(p1) + cross(th1, c.p - x1), v2 = ld3(p2) + cross(th2, c.p - x2);
+  const v3 u1 = ld3(p1) + cross(th1, c.ar1), u2 = ld3(p2) + cross(th2, c.ar2);
+  float4 lm = c.lm, cm = c.cm;
+  const float lam = lm.x, kk = lm.w;
+  const float C = av_C(c.pen + AV_MARGIN, 1.0f, d1, dot(c.n, v1), d2, dot(c.n, v2));
+  const float nl = fmn(kk * C + lam, 0.0f);
+  lm.x = nl;
+  if (nl < 0.0f) lm.w = fmn(kk + AV_BETA * fab(C), AV_KMAX);
+  const float bound = __int_as_float(h.w) * fab(lam);
+  bool stick_ok = true;
+  float drift2 = 0.0f;
+  auto tangent = [&](v3 td, float c0t, float& lt, float& kt) __attribute__((always_inline)) {
+    const float Ct = av_C(av_c0e(c0t), 1.0f, d1, dot(td, u1), d2, dot(td, u2));
+    const float nlt = fcl(kt * Ct + lt, -bound, bound);
+    lt = nlt;
+    if (nlt > -bound && nlt < bound) kt = fmn(kt + AV_BETA * fab(Ct), AV_KMAX);
+    else stick_ok = false;
+    drift2 += c0t * c0t;
+  };
+  tangent(c.t0, c.c0t.x, lm.y, cm.y);
+  tangent(c.t1, c.c0t.y, lm.z, cm.z);
+  d.man_cur.clam[cs] = lm;
+  d.man_cur.cmas[cs] = cm;
+  if (set_stick)
+    d.man_cur.canb[cs].w =
+        __uint_as_float((stick_ok && drift2 < AV_STICK_THRESH * AV_STICK_THRESH) ? 1u : 0u);
 }
 
 struct AvbdShared {
@@ -4033,10 +4055,12 @@ struct AvbdShared {
   uint32_t boff[AV_NB + 1];
 };
 
-template <class T, uint32_t kLanes = T::kAvGroup>
-BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
+// rec: the workgroup's LDS words of the primal groups (kAvGroupLds floats per
+// group).
+template <class T>
+BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* rec) {
   const uint32_t tid = t.rank(), NT = t.size();
-  constexpr uint32_t G = kLanes;  // lanes per body in the primal sweeps
+  constexpr uint32_t G = kAvGroup;  // lanes per body in the primal sweeps
   const WorldInfo W = d.worlds[w];
   if (W.solver != BB_SOLVER_AVBD || W.n == 0) return;
   const uint32_t N = W.n, off = W.body_off, P = d.npairs_cur[w];
@@ -4044,6 +4068,7 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
   // ---- adjacency (CSR, ascending slot per row) for dynamic rows
   build_adj(d, W, P, t, L.carry);
   uint32_t* adj = d.adj + 2 * W.pair_off;
+  const AvData D(d, W);
   for (uint32_t i = tid; i < N; i += NT) d.bcolor[off + i] = kMAX;
   t.sync();
   // ---- Jones-Plassmann body colouring, round-snapshot semantics
@@ -4117,7 +4142,17 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
   for (uint32_t i = tid; i < N; i += NT) {
     const uint32_t g = off + i;
     const uint32_t fl = d.cur.flags[g];
-    if (!(fl & BB_BODY_DYNAMIC) || (fl & BB_BODY_SLEEPING)) continue;
+    if (!(fl & BB_BODY_DYNAMIC) || (fl & BB_BODY_SLEEPING)) {
+      d.s_pos0[g] = d.cur.pos[g];
+      d.s_rot0[g] = d.cur.rot[g];
+      D.dp[i * 3u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      D.dth[i * 3u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      continue;
+    }
+    const uint32_t pid = off + d.cur.id[g];
+    D.iw0[i] = st3(ld3(d.props.ii0[pid]), d.props.mass[pid].x);
+    D.iw1[i] = d.props.ii1[pid];
+    D.iw2[i] = d.props.ii2[pid];
     v3 om = ld3(d.cur.omg[g]);
     float oml = vlen(om);
     if (oml > 50.0f) {
@@ -4137,8 +4172,45 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
       float accel_y = (v.y - pv.y) / dt;
       accel_w = fcl(accel_y * fsign(grav) / fab(grav), 0.0f, 1.0f);
     }
-    d.cur.pos[g] = st3((p + v * dt) + V(0.0f, grav, 0.0f) * (accel_w * dt * dt), 0.0f);
+    const v3 pn = (p + v * dt) + V(0.0f, grav, 0.0f) * (accel_w * dt * dt);
+    d.cur.pos[g] = st3(pn, 0.0f);
     d.cur.rot[g] = stq(qtl);
+    D.dp[i * 3u] = st3(pn - p, 1.0f);
+    D.dth[i * 3u] = st3(small_angle_delta(qtl, q), 0.0f);
+  }
+  // contacts per row, and the lists of contacts (per row in ascending
+  // manifold order, and of the whole world)
+  for (uint32_t i = tid; i < N; i += NT) {
+    const uint32_t g = off + i;
+    uint32_t c = 0;
+    if (d.cur.flags[g] & BB_BODY_DYNAMIC) {
+      const uint32_t* l = adj + d.adj_off[g];
+      for (uint32_t e = 0; e < d.deg[g]; ++e) c += (uint32_t)d.man_cur.hdr[l[e]].w;
+    }
+    d.pcount[g] = c;
+  }
+  t.sync();
+  (void)scan_range(t, N, [&](uint32_t i) { return d.pcount[off + i]; },
+                   [&](uint32_t i, uint32_t ex) { d.poff[off + i] = ex; });
+  const uint32_t contacts = scan_range(
+      t, P,
+      [&](uint32_t p) {
+        const int c = d.man_cur.hdr[W.pair_off + p].w;
+        return c > 0 ? (uint32_t)c : 0u;
+      },
+      [&](uint32_t p, uint32_t ex) {
+        const int c = d.man_cur.hdr[W.pair_off + p].w;
+        for (int j = 0; j < c; ++j) D.all[ex + (uint32_t)j] = p * 8u + (uint32_t)j;
+      });
+  for (uint32_t i = tid; i < N; i += NT) {
+    const uint32_t g = off + i;
+    if (!(d.cur.flags[g] & BB_BODY_DYNAMIC)) continue;
+    const uint32_t* l = adj + d.adj_off[g];
+    uint32_t x = d.poff[g];
+    for (uint32_t e = 0; e < d.deg[g]; ++e) {
+      const uint32_t c = (uint32_t)d.man_cur.hdr[l[e]].w;
+      for (uint32_t j = 0; j < c; ++j) D.item(x++) = (l[e] - W.pair_off) * 8u + j;
+    }
   }
   t.sync();
   t.mark(kMarkAvColour);
@@ -4150,8 +4222,14 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
       const uint32_t slot = W.pair_off + p;
       int4 h = d.man_cur.hdr[slot];
       if (h.w <= 0) continue;
-      const AvBody B1 = av_body(d, off + h.x), B2 = av_body(d, off + h.y);
-      const qt q1c = qconj(B1.q0), q2c = qconj(B2.q0);
+      const uint32_t ga = off + h.x, gb = off + h.y;
+      const v3 x1 = ld3(d.s_pos0[ga]), x2 = ld3(d.s_pos0[gb]);
+      const qt q1 = ldq(d.s_rot0[ga]), q2 = ldq(d.s_rot0[gb]);
+      const qt q1c = qconj(q1), q2c = qconj(q2);
+      const float f1 = d.props.mass[off + d.cur.id[ga]].z, f2 = d.props.mass[off + d.cur.id[gb]].z;
+      const float mu = __builtin_sqrtf(fmx(f1, 0.0f) * fmx(f2, 0.0f));
+      D.hdr[p] = make_int4(h.x, h.y, h.w, __float_as_int(mu));
+      const v3 t0 = ld3(d.man_cur.t0[slot]), t1 = ld3(d.man_cur.t1[slot]);
       for (int j = 0; j < h.w; ++j) {
         const uint32_t cs = slot * 8 + j;
         float4 lm = d.man_cur.clam[cs];
@@ -4175,8 +4253,8 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
         const bool sticking = matched && stick != 0;
         if (!sticking) {
           const v3 pp = ld3(d.man_cur.cpos[cs]);
-          ca = st3(avbd_q_rotate(q1c, pp - B1.p0), ca.w);
-          cb = st3(avbd_q_rotate(q2c, pp - B2.p0), cb.w);
+          ca = st3(avbd_q_rotate(q1c, pp - x1), ca.w);
+          cb = st3(avbd_q_rotate(q2c, pp - x2), cb.w);
         } else {
           ++sticks;
         }
@@ -4185,6 +4263,12 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
         d.man_cur.cmas[cs] = cmv;
         d.man_cur.cana[cs] = ca;
         d.man_cur.canb[cs] = cb;
+        const v3 ar1 = avbd_q_rotate(q1, ld3(ca)), ar2 = avbd_q_rotate(q2, ld3(cb));
+        const v3 gap = (x2 + ar2) - (x1 + ar1);
+        const size_t at = D.at(p, (uint32_t)j);
+        D.ar1[at] = ar1;
+        D.ar2[at] = ar2;
+        D.c0t[2u * at] = make_float2(dot(t0, gap), dot(t1, gap));
       }
     }
     stat_add(d, w, ST_AV_STICK, sticks);
@@ -4272,15 +4356,28 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
   t.sync();
   t.mark(kMarkAvGroup);
   const uint32_t used = L.used;
+  // the buckets' offsets (a team's live in global memory: a copy in the LDS
+  // words that counted them)
+  const uint32_t* boff = L.boff;
+  if constexpr (T::kGlobalScalars) {
+    for (uint32_t k = threadIdx.x; k <= AV_NB; k += blockDim.x) lc[k] = L.boff[k];
+    __syncthreads();
+    boff = lc;
+  }
+  float* const mine = rec + (threadIdx.x / G) * kAvGroupLds;
+  auto primal = [&](uint32_t k0, uint32_t k1, float alpha) __attribute__((always_inline)) {
+    for (uint32_t k = k0 + tid / G; k < k1; k += NT / G) av_primal(d, W, D, bb[k], alpha, tid % G, mine);
+  };
   // ---- main sweeps: 10 x (colours, dual) (rigid_body_manager.cpp:1366-1373)
   for (uint32_t it = 0; it < AV_ITERS; ++it) {
     for (uint32_t c = 0; c < used; ++c) {
-      for (uint32_t k = L.boff[c * kAvbdLayers] + tid / G; k < L.boff[(c + 1) * kAvbdLayers]; k += NT / G)
-        av_primal<G>(d, W, bb[k], 1.0f, tid % G);
+      primal(boff[c * kAvbdLayers], boff[(c + 1) * kAvbdLayers], 1.0f);
       t.sync();
     }
-    for (uint32_t p = tid; p < P; p += NT)
-      if (d.man_cur.hdr[W.pair_off + p].w > 0) av_dual(d, W, W.pair_off + p);
+    for (uint32_t x = tid; x < contacts; x += NT) {
+      const uint32_t q = D.all[x];
+      av_dual(d, W, D, q >> 3, q & 7u, it + 1u == AV_ITERS);
+    }
     t.sync();
   }
   t.mark(kMarkAvSweeps);
@@ -4313,16 +4410,15 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L) {
   // (rigid_body_manager.cpp:1391-1423)
   for (uint32_t layer = 0; layer < kAvbdLayers; ++layer) {
     for (uint32_t c = 0; c < used; ++c) {
-      const uint32_t k0 = L.boff[c * kAvbdLayers + layer], k1 = L.boff[c * kAvbdLayers + layer + 1];
+      const uint32_t k0 = boff[c * kAvbdLayers + layer], k1 = boff[c * kAvbdLayers + layer + 1];
       if (T::kSkipEmpty && k1 == k0) continue;  // an empty bucket needs no barrier
-      for (uint32_t k = k0 + tid / G; k < k1; k += NT / G) av_primal<G>(d, W, bb[k], 0.0f, tid % G);
+      primal(k0, k1, 0.0f);
       t.sync();
     }
   }
   for (uint32_t ps = 1; ps < AV_POST_STAB; ++ps) {
     for (uint32_t c = 0; c < used; ++c) {
-      for (uint32_t k = L.boff[c * kAvbdLayers] + tid / G; k < L.boff[(c + 1) * kAvbdLayers]; k += NT / G)
-        av_primal<G>(d, W, bb[k], 0.0f, tid % G);
+      primal(boff[c * kAvbdLayers], boff[(c + 1) * kAvbdLayers], 0.0f);
       t.sync();
     }
   }
@@ -4332,15 +4428,11 @@ template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_avbd(Dev d) {
   __shared__ AvbdShared L;
   __shared__ ScanLds<BLOCK> S;
+  __shared__ __align__(16) float rec[BLOCK / kAvGroup * kAvGroupLds];
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{&S, nullptr};
-  switch (d.avbd_lanes) {  // the solver tile: lanes per body in the primal sweeps
-    case 1: s_avbd<BlockTeam<BLOCK>, 1>(d, w, t, L); break;
-    case 2: s_avbd<BlockTeam<BLOCK>, 2>(d, w, t, L); break;
-    case 8: s_avbd<BlockTeam<BLOCK>, 8>(d, w, t, L); break;
-    default: s_avbd<BlockTeam<BLOCK>, 4>(d, w, t, L); break;
-  }
+  s_avbd(d, w, t, L, rec);
 }
 
 // ============================================================== k_finish
@@ -4406,6 +4498,10 @@ template <int BLOCK>
 union TeamLds {
   TeamSortLds<BLOCK> sort;
   WalkLds<BLOCK> walk;
+  struct {
+    SortLds<BLOCK> count;  // the bucket counts' staging area
+    __align__(16) float rec[BLOCK / kAvGroup * kAvGroupLds];
+  } avbd;
 };
 
 // kVox: the instance that also runs the voxel narrow phase, launched when a
@@ -4456,7 +4552,7 @@ __global__ __launch_bounds__(BLOCK) void k_team(Dev d) {
   else s_pgs<true, false>(d, w, t, nullptr, 0u);
   t.sync();
   mark(5);
-  s_avbd(d, w, t, G.avbd);
+  s_avbd(d, w, t, G.avbd, Q.avbd.rec);
   t.sync();
   mark(6);
   s_finish(d, w, t);
@@ -4492,6 +4588,13 @@ struct FusedShared {
     AvbdShared avbd;
   };
 };
+// Dynamic LDS of k_fused: the colour sweeps' body rows, then the AVBD groups'
+// words, one after the other in the same bytes.
+template <int BLOCK>
+size_t fused_lds(uint32_t pgs_rows) {
+  const size_t a = (size_t)pgs_rows * kBodyLds * 4, b = (size_t)(BLOCK / kAvGroup) * kAvGroupLds * 4;
+  return a > b ? a : b;
+}
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
@@ -4523,12 +4626,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
     else s_pgs<true, false>(d, w, t, pgs_lds, d.pgs_lcap);
   }
   __syncthreads();
-  switch (d.avbd_lanes) {
-    case 1: s_avbd<BlockTeam<BLOCK>, 1>(d, w, t, G.avbd); break;
-    case 2: s_avbd<BlockTeam<BLOCK>, 2>(d, w, t, G.avbd); break;
-    case 8: s_avbd<BlockTeam<BLOCK>, 8>(d, w, t, G.avbd); break;
-    default: s_avbd<BlockTeam<BLOCK>, 4>(d, w, t, G.avbd); break;
-  }
+  s_avbd(d, w, t, G.avbd, pgs_lds);
   __syncthreads();
   s_finish(d, w, t);
 }
@@ -4751,7 +4849,7 @@ void launch_pgs_b(const Dev& d, hipStream_t st, uint32_t grid) {
 }
 template <int B>
 void launch_fused_b(const Lane& l, hipStream_t st) {
-  hipLaunchKernelGGL(k_fused<B>, dim3(l.grid), dim3(B), (size_t)l.d.pgs_lcap * kBodyLds * 4, st,
+  hipLaunchKernelGGL(k_fused<B>, dim3(l.grid), dim3(B), fused_lds<B>(l.d.pgs_lcap), st,
                      sweep_form<B>(l.d, l.grid));
 }
 template void launch_stage_b<BB_BLOCK>(int, const Dev&, hipStream_t, uint32_t);

@@ -575,12 +575,9 @@ typedef enum bb_param {
                                 waiting for the lane's slowest world); 0
                                 (default): one launch per stage.  Profiling
                                 (bb_batch_profile) always times the stages  */
-  BB_PARAM_AVBD_LANES = 10,  /* the AVBD solver tile of the per-world
-                                kernels: lanes that assemble one body's 6x6
-                                system together in the primal sweeps (1, 2,
-                                4 or 8; 0 = the default 4).  The partial
-                                sums are added in manifold order whatever
-                                the value, so results do not change        */
+  BB_PARAM_AVBD_LANES = 10,  /* accepted (1, 2, 4 or 8; 0 = the default 4)
+                                and returned, without effect: a body of the
+                                AVBD sweeps is solved by eight lanes        */
   BB_PARAM_PGS_PREFETCH = 11, /* the PGS colour-sweep tile: 1 = a row is
                                 solved by four lanes whenever the workgroup
                                 has enough of them; 0 (default) = that form
@@ -616,9 +613,7 @@ bb_status bb_world_set_param(bb_world* w, bb_param p, uint32_t value);
  * each replay restarting from the same state, and keeps the fastest: first
  * the grid of workgroup size x PGS LDS rows, then, one at a time from the
  * best so far, one launch per step or per stage (BB_PARAM_FUSED), the PGS
- * sweep tile (BB_PARAM_PGS_PREFETCH, when a world runs PGS), the AVBD
- * solver tile (BB_PARAM_AVBD_LANES, when a world runs AVBD in the per-world
- * kernels), the radix sort's sub-team (BB_PARAM_SORT_BLOCKS, when a world
+ * sweep tile (BB_PARAM_PGS_PREFETCH, when a world runs PGS), the radix sort's sub-team (BB_PARAM_SORT_BLOCKS, when a world
  * runs as a workgroup team), the colour sweeps' workgroup and LDS rows
  * (BB_PARAM_PGS_BLOCK) and the team launch's size (BB_PARAM_TEAM_BLOCKS:
  * half or all of the resident workgroups).  The broad phase's walk budget

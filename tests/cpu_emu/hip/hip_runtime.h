@@ -113,6 +113,8 @@ static inline int emu_mov_dpp(int v, int ctrl) {
 }
 #define __builtin_amdgcn_mov_dpp(v, ctrl, row_mask, bank_mask, bound) emu_mov_dpp((v), (ctrl))
 #define __builtin_amdgcn_readlane(v, l) __shfl((v), (l), 64)
+// lanes that share LDS words wait for each other in groups of eight
+#define __builtin_amdgcn_wave_barrier() ((void)__shfl(0, 0, 8))
 
 static inline int __popc(uint32_t x) { return __builtin_popcount(x); }
 static inline int __popcll(uint64_t x) { return __builtin_popcountll(x); }

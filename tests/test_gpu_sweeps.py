@@ -58,3 +58,54 @@ def test_sweep_forms_equal_oracle(pgs_block, lds, quads):
             g, r = b.read_world(w, n), o.read_bodies()
             for f in FIELDS:
                 assert np.array_equal(g[f], r[f]), (w, n, f)
+
+
+def _plate(n: int):
+    """A dynamic plate on the ground under n spheres: the plate's contacts
+    take several rounds of its group."""
+    bodies = scenes.random_boxes(1, 1, extent=0.1, y0=0.55, y1=0.56, half=0.5, tilt=False)
+    bodies[1]["minimum"] = (-4.0, -0.25, -4.0)
+    bodies[1]["maximum"] = (4.0, 0.25, 4.0)
+    bodies[1]["position"] = (0.0, 0.249, 0.0)
+    bodies[1]["mass"] = 8.0
+    top = np.zeros(n, scenes.BODY_DESC)
+    k = np.arange(n)
+    top["shape"] = scenes.SHAPE_SPHERE
+    top["flags"] = scenes.BODY_DYNAMIC | scenes.BODY_GRAVITY
+    top["position"] = np.stack([0.5 * (k % 14) - 3.3, 0.69 + 0.0 * k, 0.5 * (k // 14) - 3.3], 1)
+    top["rotation"] = (0.0, 0.0, 0.0, 1.0)
+    top["radius"] = 0.2
+    top["minimum"], top["maximum"] = -0.2, 0.2
+    top["mass"], top["friction"] = 0.1, 0.5
+    return np.concatenate([bodies, top])
+
+
+@pytest.mark.parametrize("block,team,fused", [(128, 0, 0), (256, 0, 1), (512, 0, 0), (1024, 0, 0), (256, 9, 0)])
+def test_avbd_groups_equal_oracle(block, team, fused):
+    """Bodies solved by groups of eight lanes: one contact and several
+    rounds of them per body, sizes around a workgroup's groups, both inertia
+    conventions, every workgroup size and workgroup teams."""
+    b = beatbox.Batch()
+    b.set_param(beatbox.PARAM_BLOCK, block)
+    b.set_param(beatbox.PARAM_TEAM_BODIES, team)
+    b.set_param(beatbox.PARAM_FUSED, fused)
+    b.set_param(beatbox.PARAM_LANE_BODIES, 0)
+    scenes_ = [_plate(1), _plate(9), _plate(170)] + [
+        scenes.random_boxes(200 + n, n, extent=max(1.0, 0.4 * n ** 0.5), y0=0.55, y1=3.0) for n in (8, 33, 129)]
+    oracles = []
+    for k, bodies in enumerate(scenes_):
+        for bits in (30, 63):
+            d = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10, morton_bits=bits,
+                                                           quirks=scenes.QUIRKS_PARITY if bits == 30 else 0))
+            b.add_world(d, bodies)
+            o = OracleWorld(d)
+            o.add_bodies(bodies)
+            oracles.append((o, len(bodies)))
+    for steps in (1, 5):
+        b.step(steps)
+        b.sync(allow_overflow=True)
+        for w, (o, n) in enumerate(oracles):
+            o.step(steps)
+            g, r = b.read_world(w, n), o.read_bodies()
+            for f in FIELDS:
+                assert np.array_equal(g[f], r[f]), (w, n, f)
