@@ -3718,46 +3718,51 @@ BB_DI v3 small_angle_delta(qt now, qt start) {
   return dq.v * (2.0f * sg);
 }
 BB_DI v3 avbd_q_rotate(qt q, v3 u) { return u + cross(q.v, cross(q.v, u) + u * q.w) * 2.0f; }
-BB_DI mat3 avbd_inverse3(const mat3& a) {
-  v3 c0 = mcol(a, 0), c1 = mcol(a, 1), c2 = mcol(a, 2);
-  v3 r0 = cross(c1, c2), r1 = cross(c2, c0), r2 = cross(c0, c1);
-  float det = dot(c0, r0);
-  float inv = fab(det) > 1e-12f ? 1.0f / det : 0.0f;
-  return mrows(r0 * inv, r1 * inv, r2 * inv);
+// Row ROW's lane (0-2 in the first quad, 3-5 in the second) to all eight lanes
+// of its group: a broadcast within the quad, then the other quad's lanes from
+// their mirror images.
+template <int ROW>
+BB_DI float bc8(float x) {
+  constexpr int p = ROW < 3 ? ROW : ROW + 1;
+  const int q = __float_as_int(quad_perm<(p & 3) * 0x55>(x));
+  return __int_as_float(__builtin_amdgcn_update_dpp(q, q, 0x141 /* row_half_mirror */, 0xF, p < 4 ? 0xA : 0x5, false));
 }
-// avbd_solve6 (avbd.slang:324-387): in-place LDL^T, diagonal >= 1e-8
-BB_DI void avbd_solve6(float H[6][6], float b[6], float x[6]) {
-#pragma unroll
-  for (int jj = 0; jj < 6; ++jj) {
-    float dd = H[jj][jj];
-#pragma unroll
-    for (int kk = 0; kk < jj; ++kk) dd -= H[jj][kk] * H[jj][kk] * H[kk][kk];
-    dd = fmx(dd, 1e-8f);
-    H[jj][jj] = dd;
-#pragma unroll
-    for (int ii = jj + 1; ii < 6; ++ii) {
-      float s = H[ii][jj];
-#pragma unroll
-      for (int kk = 0; kk < jj; ++kk) s -= H[ii][kk] * H[jj][kk] * H[kk][kk];
-      H[ii][jj] = s / dd;
-    }
-  }
-#pragma unroll
-  for (int ii = 0; ii < 6; ++ii) {
-    float s = b[ii];
-#pragma unroll
-    for (int kk = 0; kk < ii; ++kk) s -= H[ii][kk] * b[kk];
-    b[ii] = s;
-  }
-#pragma unroll
-  for (int ii = 0; ii < 6; ++ii) b[ii] /= H[ii][ii];
-#pragma unroll
-  for (int ii = 5; ii >= 0; --ii) {
-    float s = b[ii];
-#pragma unroll
-    for (int kk = ii + 1; kk < 6; ++kk) s -= H[kk][ii] * x[kk];
-    x[ii] = s;
-  }
+// avbd_solve6 (avbd.slang:324-387): LDL^T with a diagonal of at least 1e-8,
+// by the group's lanes: lane of row a holds H[a][0..5] (lower triangle) and
+// b[a]; every entry goes through the operations of the one-lane form in their
+// order, the rows of a column side by side (7 divisions deep instead of 21).
+// Returns the whole solution in every lane.
+BB_DI void av_solve(float (&H)[6], float b, uint32_t a, float (&x)[6]) {
+  float D[6], own = 1.0f;
+  static_for<6>([&](auto jc) __attribute__((always_inline)) {
+    constexpr int jj = decltype(jc)::value;
+    float s = H[jj];
+    static_for<jj>([&](auto kc) __attribute__((always_inline)) {
+      constexpr int kk = decltype(kc)::value;
+      s -= H[kk] * bc8<jj>(H[kk]) * D[kk];
+    });
+    D[jj] = fmx(bc8<jj>(s), 1e-8f);
+    own = a == (uint32_t)jj ? D[jj] : own;
+    if constexpr (jj < 5) H[jj] = s / D[jj];
+  });
+  static_for<5>([&](auto kc) __attribute__((always_inline)) {
+    constexpr int kk = decltype(kc)::value;
+    const float t = b - H[kk] * bc8<kk>(b);
+    b = a > (uint32_t)kk ? t : b;
+  });
+  b /= own;
+  float xa = b;  // this row's solution, once its step is done
+  static_for<6>([&](auto rc) __attribute__((always_inline)) {
+    constexpr int ii = 5 - decltype(rc)::value;
+    const float pr = H[ii] * xa;
+    float s = b;
+    static_for<5 - ii>([&](auto kc) __attribute__((always_inline)) {
+      constexpr int kk = ii + 1 + decltype(kc)::value;
+      s -= bc8<kk>(pr);
+    });
+    xa = a == (uint32_t)ii ? s : xa;
+    x[ii] = bc8<ii>(s);
+  });
 }
 
 // What the sweeps of an AVBD world read, prepared once per step (nothing of
@@ -3781,9 +3786,14 @@ struct AvData {
   int4* hdr;                // [slot]
   v3 *ar1, *ar2;            // [contact * np + slot]
   float2* c0t;              // [2 * (contact * np + slot)]
-  uint32_t *list0, *list1;  // first 8 * cap and the remaining list entries
+  // body lists: item x in list0 and the row on the other side of it in list1
+  // (bit 31: this body is the manifold's first), or, when they are longer than
+  // 8 * cap, items only, in list0 and then list1
+  uint32_t *list0, *list1;
   uint32_t* all;
   uint32_t np, cap8;
+  // bucket entry k: the row, its first item and its items
+  uint32_t *brow, *bfirst, *bcount;
   BB_DI AvData(const Dev& d, const WorldInfo& W) {
     dp = d.iw + 3u * (size_t)W.body_off;
     dth = dp + 1;
@@ -3800,10 +3810,14 @@ struct AvData {
     list1 = reinterpret_cast<uint32_t*>(d.sv_l + 24u * (size_t)np + 8u * (size_t)W.pair_off);
     all = d.sv_list + 8u * (size_t)W.pair_off;
     cap8 = 8u * W.pair_cap;
+    brow = d.bbucket + W.body_off;
+    bfirst = d.depth_snap + W.body_off;   // free after the grouping
+    bcount = d.bcolor_snap + W.body_off;  // free after the colouring
   }
   BB_DI size_t at(uint32_t slot, uint32_t j) const { return (size_t)j * np + slot; }
   BB_DI uint32_t& item(uint32_t x) const { return x < cap8 ? list0[x] : list1[x - cap8]; }
 };
+static constexpr uint32_t kAvFirst = 0x80000000u;
 
 // One contact of a manifold between rows h.x and h.y (rows of the world,
 // slots of the world): what both the primal and the dual update read of it.
@@ -3855,65 +3869,73 @@ BB_DI void group_sync() {
 // manifold order.  Lane l evaluates the body's contacts l, l + 8, ...: three
 // constraint rows each, left in the group's LDS words (rec) as Jacobian,
 // stiffness and force.  Then lane a < 6 sums row a of H and entry a of the
-// gradient over all rows in order: a wave issues an instruction every 8 or
+// gradient over all rows in order, and the rows' lanes solve the system
+// together (rows 0-2 in lanes 0-2, rows 3-5 in lanes 4-6): a wave issues an instruction every 8 or
 // more cycles whatever its lanes do, so a body's time is its instructions,
 // and here eight lanes share both the contacts and the sums (one lane per
 // manifold took four times as many on a manifold of four contacts, and the
 // sums went through 27 cross-lane moves per manifold).  avbd_solve6 reads the
 // lower triangle only.  Measured, per step, against one lane per manifold
-// that read both bodies' poses: 27 tower bodies 571 -> 330 us, a 1,501-body
-// world 4.1 -> 2.6 ms, the 20,000-body pile 8.2 -> 4.6 and the 100,000-body
-// pile 9.7 -> 6.2 ms.
+// that read both bodies' poses: 27 tower bodies 571 -> 313 us, a 1,501-body
+// world 4.1 -> 2.3 ms, the 20,000-body pile 8.2 -> 4.4 and the 100,000-body
+// pile 9.7 -> 6.0 ms.
 static constexpr uint32_t kAvGroup = 8;
 static constexpr uint32_t kAvRec = 8;                          // floats of a row's record
 static constexpr uint32_t kAvGroupLds = kAvGroup * 3 * kAvRec;  // LDS floats per group
-BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t i, float alpha, uint32_t l,
-                     float* rec) {
+// partners: the body lists name the other rows.
+BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t bk, bool partners, float alpha,
+                     uint32_t l, float* rec) {
+  const uint32_t i = D.brow[bk], c0 = D.bfirst[bk], cn = D.bcount[bk];
   const uint32_t off = W.body_off, g = off + i;
   const bool quirk = (W.quirks & BB_QUIRK_TRANSPOSED_WORLD_INERTIA) != 0;
   const float dt = W.dt;
   const float inv_dt2 = dt > 0.0f ? 1.0f / (dt * dt) : 0.0f;
-  const uint32_t c0 = d.poff[g], cn = d.pcount[g];
   v3 pos = ld3(d.cur.pos[g]);
   qt rot = ldq(d.cur.rot[g]);
   const v3 p0 = ld3(d.s_pos0[g]);
   const qt q0 = ldq(d.s_rot0[g]);
   const v3 dpo = ld3(D.dp[i * 3u]), dtho = ld3(D.dth[i * 3u]);
   const float4 m0 = D.iw0[i], m1 = D.iw1[i], m2 = D.iw2[i];
-  // inertial terms: row l of H, entry l of the gradient
+  // inertial terms: row a of H, entry a of the gradient
+  const uint32_t j = (l & 3u) < 3u ? l & 3u : 2u, a = (l >> 2) * 3u + j;
   float H[6], gr;
   {
     const float m_lin = m0.w * inv_dt2;
-    const mat3 I = mrows(ld3(m0), ld3(m1), ld3(m2));
+    // avbd_inverse3(world_inv_inertia): lane j of a quad computes column j of
+    // S I S^T (S = R, or R^T with the parity quirk), then row j of its inverse
     const mat3 R = qmat(rot);
-    const mat3 Rt = mT(R);
-    const mat3 Iw = avbd_inverse3(quirk ? mmul(Rt, mmul(I, mT(Rt))) : mmul(R, mmul(I, mT(R))));
+    const mat3 S = quirk ? mT(R) : R;
+    const v3 sj = j == 0u ? mrow(S, 0) : (j == 1u ? mrow(S, 1) : mrow(S, 2));
+    const v3 bj = mulmv(mrows(ld3(m0), ld3(m1), ld3(m2)), sj);
+    const v3 cj = mulmv(S, bj);
+    const v3 c1 = V(qr1(cj.x), qr1(cj.y), qr1(cj.z)), c2 = V(qr2(cj.x), qr2(cj.y), qr2(cj.z));
+    const v3 rj = cross(c1, c2);
+    const float det = qc0(dot(cj, rj));
+    const float inv = fab(det) > 1e-12f ? 1.0f / det : 0.0f;
+    const v3 iw = rj * inv;
     const v3 dpos = pos - ld3(d.s_post[g]);
     const v3 dth = small_angle_delta(rot, ldq(d.s_rott[g]));
-    const v3 ga = mulmv(Iw, dth) * inv_dt2;
-    const uint32_t r = l % 3u;  // lanes 0-2: position rows, 3-5: rotation rows
-    const bool ang = l >= 3u;
-    const float ix = r == 0u ? Iw.m[0][0] : (r == 1u ? Iw.m[1][0] : Iw.m[2][0]);
-    const float iy = r == 0u ? Iw.m[0][1] : (r == 1u ? Iw.m[1][1] : Iw.m[2][1]);
-    const float iz = r == 0u ? Iw.m[0][2] : (r == 1u ? Iw.m[1][2] : Iw.m[2][2]);
-    const float dl = r == 0u ? dpos.x : (r == 1u ? dpos.y : dpos.z);
-    const float gl = r == 0u ? ga.x : (r == 1u ? ga.y : ga.z);
-    H[0] = !ang && r == 0u ? m_lin : 0.0f;
-    H[1] = !ang && r == 1u ? m_lin : 0.0f;
-    H[2] = !ang && r == 2u ? m_lin : 0.0f;
-    H[3] = ang ? ix * inv_dt2 : 0.0f;
-    H[4] = ang ? iy * inv_dt2 : 0.0f;
-    H[5] = ang ? iz * inv_dt2 : 0.0f;
-    gr = ang ? gl : m_lin * dl;
+    const bool ang = l >= 4u;
+    const float dl = j == 0u ? dpos.x : (j == 1u ? dpos.y : dpos.z);
+    H[0] = !ang && j == 0u ? m_lin : 0.0f;
+    H[1] = !ang && j == 1u ? m_lin : 0.0f;
+    H[2] = !ang && j == 2u ? m_lin : 0.0f;
+    H[3] = ang ? iw.x * inv_dt2 : 0.0f;
+    H[4] = ang ? iw.y * inv_dt2 : 0.0f;
+    H[5] = ang ? iw.z * inv_dt2 : 0.0f;
+    gr = ang ? dot(iw, dth) * inv_dt2 : m_lin * dl;
   }
   float he[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, ge = 0.0f;  // the manifold's partial sum
   for (uint32_t r0 = 0; r0 < cn; r0 += kAvGroup) {
     if (r0 + l < cn) {
-      const uint32_t w = D.item(c0 + r0 + l), slot = w >> 3, j = w & 7u;
+      const uint32_t x = c0 + r0 + l;
+      const uint32_t w = D.item(x), slot = w >> 3, ct = w & 7u;
+      uint32_t o = partners ? D.list1[x] : 0u;
       const int4 h = D.hdr[slot];
-      const AvContact c = av_contact(d, W, D, slot, j);
-      const bool i1 = (uint32_t)h.x == i;
-      const uint32_t o = i1 ? (uint32_t)h.y : (uint32_t)h.x;
+      const AvContact c = av_contact(d, W, D, slot, ct);
+      if (!partners) o = (uint32_t)h.x == i ? (uint32_t)h.y | kAvFirst : (uint32_t)h.x;
+      const bool i1 = (o & kAvFirst) != 0u;
+      o &= ~kAvFirst;
       const float4 odp = D.dp[o * 3u];
       const v3 dpx = ld3(odp), dthx = ld3(D.dth[o * 3u]), px = ld3(d.s_pos0[off + o]);
       const bool omoves = odp.w != 0.0f;
@@ -3945,18 +3967,17 @@ BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t
       tangent(1, c.t0, c.c0t.x, c.lm.y, c.cm.y, 0u);
       // stiffnesses are positive: the sign bit of the last row's marks the
       // manifold's last contact
-      tangent(2, c.t1, c.c0t.y, c.lm.z, c.cm.z, j + 1u == ((uint32_t)h.z & 255u) ? 0x80000000u : 0u);
+      tangent(2, c.t1, c.c0t.y, c.lm.z, c.cm.z, ct + 1u == (uint32_t)h.z ? 0x80000000u : 0u);
     }
     group_sync();
     const uint32_t m = cn - r0 < kAvGroup ? cn - r0 : kAvGroup;
-    const uint32_t la = l < 6u ? l : 5u;
     for (uint32_t c = 0; c < m; ++c) {
       uint32_t kb = 0;
 #pragma unroll
       for (uint32_t t = 0; t < 3; ++t) {
         const float* q = rec + (c * 3u + t) * kAvRec;
         const float4 qa = reinterpret_cast<const float4*>(q)[0], qb = reinterpret_cast<const float4*>(q)[1];
-        const float ja = q[la];
+        const float ja = q[a];
         kb = __float_as_uint(qb.z);
         const float k = t == 2u ? __uint_as_float(kb & 0x7FFFFFFFu) : qb.z;
         const float kj = k * ja;
@@ -3970,9 +3991,9 @@ BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t
       }
       if (kb & 0x80000000u) {
 #pragma unroll
-        for (int a = 0; a < 6; ++a) {
-          H[a] += he[a];
-          he[a] = 0.0f;
+        for (int b = 0; b < 6; ++b) {
+          H[b] += he[b];
+          he[b] = 0.0f;
         }
         gr += ge;
         ge = 0.0f;
@@ -3980,23 +4001,8 @@ BB_DI void av_primal(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t
     }
     group_sync();
   }
-  // every lane solves the whole system
-  if (l < 6u) {
-    float4* q = reinterpret_cast<float4*>(rec + l * 8u);
-    q[0] = make_float4(H[0], H[1], H[2], H[3]);
-    q[1] = make_float4(H[4], H[5], gr, 0.0f);
-  }
-  group_sync();
-  float A[6][6], rhs[6], dx[6];
-#pragma unroll
-  for (int a = 0; a < 6; ++a) {
-    const float4* q = reinterpret_cast<const float4*>(rec + a * 8);
-    const float4 qa = q[0], qb = q[1];
-    A[a][0] = qa.x; A[a][1] = qa.y; A[a][2] = qa.z; A[a][3] = qa.w; A[a][4] = qb.x; A[a][5] = qb.y;
-    rhs[a] = -qb.z;
-  }
-  group_sync();  // the words are free for the group's next body
-  avbd_solve6(A, rhs, dx);
+  float dx[6];
+  av_solve(H, -gr, a, dx);
   pos = pos + V(dx[0], dx[1], dx[2]);
   const v3 half = V(dx[3], dx[4], dx[5]) * 0.5f;
   rot = qnorm(qmul(qt{half, 1.0f}, rot));
@@ -4190,8 +4196,9 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     d.pcount[g] = c;
   }
   t.sync();
-  (void)scan_range(t, N, [&](uint32_t i) { return d.pcount[off + i]; },
-                   [&](uint32_t i, uint32_t ex) { d.poff[off + i] = ex; });
+  const uint32_t items = scan_range(t, N, [&](uint32_t i) { return d.pcount[off + i]; },
+                                    [&](uint32_t i, uint32_t ex) { d.poff[off + i] = ex; });
+  const bool partners = items <= D.cap8;
   const uint32_t contacts = scan_range(
       t, P,
       [&](uint32_t p) {
@@ -4208,8 +4215,12 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     const uint32_t* l = adj + d.adj_off[g];
     uint32_t x = d.poff[g];
     for (uint32_t e = 0; e < d.deg[g]; ++e) {
-      const uint32_t c = (uint32_t)d.man_cur.hdr[l[e]].w;
-      for (uint32_t j = 0; j < c; ++j) D.item(x++) = (l[e] - W.pair_off) * 8u + j;
+      const int4 h = d.man_cur.hdr[l[e]];
+      const uint32_t o = (uint32_t)h.x == i ? (uint32_t)h.y | kAvFirst : (uint32_t)h.x;
+      for (uint32_t j = 0; j < (uint32_t)h.w; ++j, ++x) {
+        D.item(x) = (l[e] - W.pair_off) * 8u + j;
+        if (partners) D.list1[x] = o;
+      }
     }
   }
   t.sync();
@@ -4343,7 +4354,6 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     }
     __syncthreads();
   }
-  uint32_t* bb = d.bbucket + off;
   for (uint32_t i = tid; i < N; i += NT) {
     const uint32_t g = off + i;
     const uint32_t fl = d.cur.flags[g], c = d.bcolor[g];
@@ -4351,7 +4361,11 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     uint32_t layer = d.depth[g] < kAvbdLayers - 1 ? d.depth[g] : kAvbdLayers - 1;
     const uint32_t k = c * kAvbdLayers + layer;
     const uint32_t o = lc ? lc[AV_NB + k] + atomicAdd(&lc[k], 1u) : atomicAdd(&L.bcount[k], 1u);
-    if (o < N) bb[o] = i;  // the buckets hold at most the world's N rows
+    if (o < N) {  // the buckets hold at most the world's N rows
+      D.brow[o] = i;
+      D.bfirst[o] = d.poff[g];
+      D.bcount[o] = d.pcount[g];
+    }
   }
   t.sync();
   t.mark(kMarkAvGroup);
@@ -4366,7 +4380,8 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
   }
   float* const mine = rec + (threadIdx.x / G) * kAvGroupLds;
   auto primal = [&](uint32_t k0, uint32_t k1, float alpha) __attribute__((always_inline)) {
-    for (uint32_t k = k0 + tid / G; k < k1; k += NT / G) av_primal(d, W, D, bb[k], alpha, tid % G, mine);
+    for (uint32_t k = k0 + tid / G; k < k1; k += NT / G)
+      av_primal(d, W, D, k, partners, alpha, tid % G, mine);
   };
   // ---- main sweeps: 10 x (colours, dual) (rigid_body_manager.cpp:1366-1373)
   for (uint32_t it = 0; it < AV_ITERS; ++it) {
@@ -4799,6 +4814,7 @@ __global__ __launch_bounds__(256) void k_copy_calibrate(const float4* __restrict
 // holds the team kernel, the launch sequence and the small utility kernels.
 namespace bb {
 static constexpr int kStages = 7;
+static constexpr uint32_t kCus = 256;  // CUs of the chip
 template <int B>
 void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid);
 template <int B>
@@ -4814,7 +4830,7 @@ void launch_fused_b(const Lane& l, hipStream_t st);
 template <int B>
 Dev sweep_form(const Dev& d, uint32_t grid) {
   Dev r = d;
-  r.pgs_quad_rows = d.pgs_quads || grid <= 256u ? (uint32_t)B / 4u : 16u;
+  r.pgs_quad_rows = d.pgs_quads || grid <= kCus ? (uint32_t)B / 4u : 16u;
   return r;
 }
 // Stages of the per-world path, in launch order (k_team, when there is one,
@@ -4863,9 +4879,18 @@ template void launch_pgs_b<64>(const Dev&, hipStream_t, uint32_t);
 template __global__ void k_team<kTeamBlock, false>(Dev);
 template __global__ void k_team<kTeamBlock, true>(Dev);
 
+// Threads per workgroup of the AVBD stage.  While every world of the lane has
+// a CU to itself, 512-thread workgroups give way to 1,024-thread ones: a CU
+// issues 16 waves side by side at the rate of one, so a phase with more bodies
+// than 64 groups of lanes take at once saves its further rounds (1,501 bodies,
+// about 190 per colour: 2.96 -> 2.46 ms; 64 served worlds' lane 3.6 -> 2.9
+// ms).  The colour sweeps gain nothing by it (1,001 cubes: 437 against 456
+// us).
+static uint32_t avbd_block(const Lane& l) { return l.block == 512u && l.grid <= kCus ? 1024u : l.block; }
+
 static void launch_stage(int stage, const Lane& l, hipStream_t st) {
   if (l.grid == 0) return;
-  switch (l.block) {
+  switch (stage == 5 ? avbd_block(l) : l.block) {
     case 128: launch_stage_b<128>(stage, l.d, st, l.grid); break;
     case 512: launch_stage_b<512>(stage, l.d, st, l.grid); break;
     case 1024: launch_stage_b<1024>(stage, l.d, st, l.grid); break;

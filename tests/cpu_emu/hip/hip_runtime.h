@@ -112,6 +112,14 @@ static inline int emu_mov_dpp(int v, int ctrl) {
   return __shfl_down(v, (unsigned)(ctrl & 15), 16);
 }
 #define __builtin_amdgcn_mov_dpp(v, ctrl, row_mask, bank_mask, bound) emu_mov_dpp((v), (ctrl))
+// row_half_mirror (0x141) into the enabled banks of a row of 16
+static inline int emu_update_dpp(int old, int v, int ctrl, int bank_mask) {
+  const int lane = (int)(threadIdx.x & 63u);
+  const int m = ctrl == 0x141 ? __shfl(v, 7 - (lane & 7), 8) : emu_mov_dpp(v, ctrl);
+  return (bank_mask >> ((lane & 15) >> 2)) & 1 ? m : old;
+}
+#define __builtin_amdgcn_update_dpp(old, v, ctrl, row_mask, bank_mask, bound) \
+  emu_update_dpp((old), (v), (ctrl), (bank_mask))
 #define __builtin_amdgcn_readlane(v, l) __shfl((v), (l), 64)
 // lanes that share LDS words wait for each other in groups of eight
 #define __builtin_amdgcn_wave_barrier() ((void)__shfl(0, 0, 8))
