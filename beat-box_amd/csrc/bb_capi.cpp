@@ -214,6 +214,8 @@ bb_status alloc_arrays(bb_batch* b, Buffers& A, uint32_t W, uint32_t NB, uint32_
   d.sort_blocks = b->sort_blocks;
   d.pgs_quads = b->pgs_prefetch;
   d.pgs_quad_rows = 0;  // set per launch
+  d.spread = 1;         // likewise
+  d.lane_max = 0;       // set per lane
   d.walk_budget = b->walk_budget;
   d.teams = A.alloc<TeamTable>(1);
   d.team_ctl = A.alloc<TeamCtl>(kMaxTeams);
@@ -630,15 +632,24 @@ uint32_t pick_block(const bb_batch* b) {
 int lanes_of(const bb_batch* b, const Dev& d, Lane* out) {
   const uint32_t nw = std::min(b->n_wide, d.W);
   int nl = 0;
+  // largest world of all, and of each lane (teams aside)
+  uint32_t mx = 0, wide_max = 0, rest_max = 0;
+  for (auto& hw : b->worlds) {
+    const uint32_t n = (uint32_t)hw.bodies.size();
+    mx = std::max(mx, n);
+    if (b->team_bodies && n >= b->team_bodies && !hw.no_team) continue;
+    uint32_t& m = b->lane_bodies && n >= b->lane_bodies ? wide_max : rest_max;
+    m = std::max(m, n);
+  }
   if (nw) {
     Dev dw = d;
-    uint32_t mx = 0;
-    for (auto& hw : b->worlds) mx = std::max(mx, (uint32_t)hw.bodies.size());
     dw.pgs_lcap = std::min(mx, b->lane_lds);
+    dw.lane_max = wide_max;
     out[nl++] = Lane{dw, b->lane_block, nw, b->fused != 0};
   }
   Dev rest = d;
   rest.order = d.order + nw;
+  rest.lane_max = rest_max;
   out[nl++] = Lane{rest, pick_block(b), d.W - nw, b->fused != 0, b->pgs_block};
   return nl;
 }

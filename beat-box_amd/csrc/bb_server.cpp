@@ -348,6 +348,12 @@ bb_status ensure_graphs(bb_server* s, uint32_t p) {
     Dev d = dev_for(s->b, par);
     d.order = d.order + P.w0;
     d.pgs_lcap = P.lcap;
+    // the pools past the first hold worlds of hundreds of bodies in few of
+    // their slots: several workgroups for each world's broad and narrow phase
+    if (p) {
+      d.lane_max = kMAX;
+      d.spread = 4u;
+    }
     if (!P.teams) d.team_grid = 0;
     // with voxel shapes registered any team may hold voxel bodies
     d.team_vox = s->b->vox_shapes.empty() ? 0u : 1u;

@@ -19,6 +19,8 @@
 // world's results do not depend on the other worlds of the batch.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/bb_capi.h"
 #include "bb_dev.hpp"
 #include "bb_math.hpp"
@@ -26,6 +28,7 @@
 namespace bb {
 
 #define WAVE 64
+static constexpr uint32_t kCus = 256;  // CUs of the chip
 
 // ============================================================ block helpers
 template <int BLOCK>
@@ -264,12 +267,15 @@ struct BlockTeam {
   // empty AVBD cascade buckets skip their barrier
   static constexpr bool kSkipEmpty = true;
   static constexpr bool kGlobalScalars = false;  // stage scalars in LDS
+  static constexpr bool kSpread = false;
   static constexpr int kBlock = BLOCK;
   BB_DI uint32_t rank() const { return threadIdx.x; }
   BB_DI uint32_t size() const { return BLOCK; }
   // this workgroup's index in the team, and the team's workgroups
   BB_DI uint32_t group() const { return 0; }
   BB_DI uint32_t groups() const { return 1; }
+  // the thread that sets the stage scalars
+  BB_DI bool lead() const { return threadIdx.x == 0; }
   BB_DI void sync() const { __syncthreads(); }
   BB_DI void fence() const { __threadfence_block(); }
   // every leaf range is this workgroup's (see GroupTeam::leaves_local)
@@ -283,6 +289,25 @@ struct BlockTeam {
   BB_DI void mark(uint32_t) const {}
   BB_DI void mark_lead(uint32_t) const {}
   BB_DI bool sorted_in_a(bool in_a) const { return in_a; }
+};
+
+// Several workgroups on one world without a barrier between them: the
+// narrow phase's two parts handle every pair on its own, the broad phase's
+// walks every row.  Its barrier is the workgroup's, and so are the stage
+// scalars of the kernels that use it.
+template <int BLOCK>
+struct SpreadTeam {
+  uint32_t part, parts;
+  ScanLds<BLOCK>* scan_lds;
+  static constexpr bool kSpread = true;
+  static constexpr bool kGlobalScalars = false;
+  static constexpr int kBlock = BLOCK;
+  BB_DI uint32_t rank() const { return part * BLOCK + threadIdx.x; }
+  BB_DI uint32_t size() const { return parts * BLOCK; }
+  BB_DI uint32_t group() const { return 0; }
+  BB_DI uint32_t groups() const { return 1; }
+  BB_DI bool lead() const { return threadIdx.x == 0; }
+  BB_DI void sync() const { __syncthreads(); }
 };
 
 // Spins before a team barrier wait gives up (about a second).  A wait that
@@ -311,11 +336,13 @@ struct GroupTeam {
   // bucket offsets after the same barrier, so all of them skip the same ones)
   static constexpr bool kSkipEmpty = true;
   static constexpr bool kGlobalScalars = true;  // stage scalars in a global slot
+  static constexpr bool kSpread = false;
   static constexpr int kBlock = BLOCK;
   BB_DI uint32_t rank() const { return blk * BLOCK + threadIdx.x; }
   BB_DI uint32_t size() const { return nblocks * BLOCK; }
   BB_DI uint32_t group() const { return blk; }
   BB_DI uint32_t groups() const { return nblocks; }
+  BB_DI bool lead() const { return rank() == 0; }
   BB_DI void fence() const { __threadfence(); }
   // Clock mark m of this step, called right after a team barrier: every
   // workgroup has reached that point when rank 0 stamps it.
@@ -1098,29 +1125,92 @@ BB_DI void sort8(uint32_t (&k)[8]) {
 }
 
 struct BroadShared {
-  uint32_t carry;
-  uint32_t pairs;   // voxel worlds: pairs, as opposed to pair slots
   uint32_t ndefer;  // rows handed to a workgroup (coop_walk), listed in defer
   uint32_t defer[kMaxDefer];
 };
 
+// Small worlds skip the tree: a row's box against every later row's, 64 rows
+// at a time by a wave, which finds the same pairs (an inner node's box is the
+// exact union of its leaves', so a leaf that overlaps is always reached) and
+// finds them in ascending order.  A walk is a chain of node visits of about
+// 1,000 cycles each, up to the budget of 128; the flat form is N^2 / 128 wave
+// tests of about 14 instructions, spread over the team's waves.  The line
+// lies where those take about 17 us (a walk at its budget takes 55); with more
+// worlds than CUs at a fifth of that, since there the instructions count and
+// not the chain (4,096 worlds' wide lane: 533 us with the trees alone, 508 so,
+// 616 with the first line and a wave less per SIMD).  Measured: 49 bodies 51 -> 23 us; 1,001 bodies 144 -> 41 us and
+// 1,501 bodies 290 -> 76 us with 16 workgroups.
+// Not with a NaN box in the world: it reaches the root through the ordered
+// min / max, and the walks then end where it does.
+static constexpr uint32_t kFlatPerWave = 40960, kFlatCrowded = 8192;
 template <class T>
-BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds<T::kBlock>& F) {
+BB_DI bool broad_flat(const Dev& d, uint32_t nb, uint32_t N, const T& t) {
+  if constexpr (T::kGlobalScalars) return false;  // worlds this large keep the tree
+  const uint32_t per = gridDim.x > kCus ? kFlatCrowded : kFlatPerWave;
+  if (N < 2u || (uint64_t)N * N > (uint64_t)per * (t.size() / WAVE)) return false;
+  const float4 a = d.nmin[nb], b = d.nmax[nb];
+  return a.x == a.x && a.y == a.y && a.z == a.z && b.x == b.x && b.y == b.y && b.z == b.z;
+}
+// hits(i, j, m) for every 64 rows from a multiple of 64 on: m = the rows
+// among them (bit k: row j - lane + k) behind i whose boxes overlap row i's;
+// j is this lane's row.  Called by whole waves.
+template <class Hits>
+BB_DI void flat_row(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, Hits&& hits) {
+  constexpr uint32_t U = 4;
+  const uint32_t lane = threadIdx.x & (WAVE - 1), leaf = nb + N - 1u;
+  const v3 qmn = ld3(d.nmin[leaf + i]), qmx = ld3(d.nmax[leaf + i]);
+  for (uint32_t c0 = (i + 1u) & ~63u; c0 < N; c0 += U * WAVE) {
+    float4 mn[U], mx[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t j = c0 + u * WAVE + lane, k = j < N ? j : N - 1u;
+      mn[u] = d.nmin[leaf + k];
+      mx[u] = d.nmax[leaf + k];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t j = c0 + u * WAVE + lane;
+      const uint64_t m = __ballot(j > i && j < N && overlap(qmn, qmx, mn[u], mx[u]));
+      if (m) hits(j, m);
+    }
+  }
+}
+
+// The broad phase's parts.  s_broad_count: partner counts per row (slots of
+// voxel worlds), the first kPairStage partners staged; s_broad_scan: the rows'
+// offsets and the pair count; s_broad_write: the pair list.
+// voxel worlds: a pair with a voxel body takes six slots (one per contact-
+// face code), so the per-row offsets count slots, and the pair counter
+// counts pairs.
+template <class T>
+BB_DI void s_broad_count(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds<T::kBlock>& F) {
   const uint32_t tid = t.rank(), NT = t.size();
   const WorldInfo W = d.worlds[w];
   const uint32_t N = W.n, off = W.body_off, nb = 2 * off;
   uint32_t* stage = d.pick + W.pair_off;
-  // voxel worlds: a pair with a voxel body takes six slots (one per contact-
-  // face code), so the per-row offsets count slots, and the pair counter
-  // counts pairs
   const bool vox = (W.mode & kModeVoxel) != 0;
   auto is_vox = [&](uint32_t row) {
     return (shape_word(d.props.pmax[off + d.cur.id[off + row]].w) & 0xFFu) == BB_SHAPE_VOXEL;
   };
-  if (tid == 0) {
-    L.carry = 0;
-    L.pairs = 0;
-    L.ndefer = 0;
+  if (t.lead()) L.ndefer = 0;
+  if (broad_flat(d, nb, N, t)) {
+    for (uint32_t i = tid / WAVE; i < N; i += NT / WAVE) {
+      const bool vi = vox && is_vox(i);
+      uint32_t cnt = 0, slots = 0;
+      flat_row(d, nb, N, i, [&](uint32_t j, uint64_t m) {
+        const uint32_t n = (uint32_t)__popcll(m);
+        cnt += n;
+        if (!vox) return;
+        const bool mine = (m >> (threadIdx.x & (WAVE - 1))) & 1ull;
+        const uint64_t vm = vi ? m : __ballot(mine && is_vox(j));
+        slots += n + 5u * (uint32_t)__popcll(vm);
+      });
+      if ((threadIdx.x & (WAVE - 1)) == 0u) {
+        d.pcount[off + i] = cnt;
+        if (vox) d.poff[off + i] = slots;
+      }
+    }
+    return;
   }
   t.sync();
   // partner counts (slots of voxel worlds parked in poff); a row whose walk
@@ -1157,7 +1247,14 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
     const uint32_t cnt = coop_walk<T::kBlock>(d, nb, N, i, ld3(mn), ld3(mx), F, *t.scan_lds, nullptr, 0u);
     if (threadIdx.x == 0) d.pcount[off + i] = kDeferBit | cnt;
   }
-  if (nd) t.sync();
+}
+
+template <class T>
+BB_DI void s_broad_scan(const Dev& d, uint32_t w, const T& t) {
+  const uint32_t tid = t.rank();
+  const WorldInfo W = d.worlds[w];
+  const uint32_t N = W.n, off = W.body_off;
+  const bool vox = (W.mode & kModeVoxel) != 0;
   // per-row offsets of the pair slots (voxel worlds: slots parked in poff,
   // and the pairs counted apart)
   const uint32_t vox_pairs =
@@ -1169,14 +1266,106 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
         d.poff[off + i] = ex;
         d.pstart_cur[off + i] = ex;
       });
-  t.sync();
   const uint32_t cap = W.pair_cap;
   if (tid == 0) {
     d.npairs_cur[w] = P < cap ? P : cap;
     d.stats[w * ST_COUNT + ST_P] = vox ? vox_pairs : P;
     if (P > cap) d.stats[w * ST_COUNT + ST_OVERFLOW] = 1;
   }
-  uint2* pairs = d.pairs_cur + W.pair_off;
+}
+
+template <class T>
+BB_DI void s_broad_write(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds<T::kBlock>& F) {
+  const uint32_t tid = t.rank(), NT = t.size();
+  const WorldInfo W = d.worlds[w];
+  const uint32_t N = W.n, off = W.body_off, nb = 2 * off;
+  uint32_t* stage = d.pick + W.pair_off;
+  const bool vox = (W.mode & kModeVoxel) != 0;
+  const uint32_t cap = W.pair_cap;
+  auto is_vox = [&](uint32_t row) {
+    return (shape_word(d.props.pmax[off + d.cur.id[off + row]].w) & 0xFFu) == BB_SHAPE_VOXEL;
+  };
+  uint2* const pairs = d.pairs_cur + W.pair_off;
+  // Row i's partners by a walk of one thread into its slots from o on: the
+  // first that fit, in walk order, then sorted.  With voxel bodies the row's
+  // slots hold at least cnt entries; expanded from the back (an entry only
+  // moves to a higher or equal slot).
+  auto write_walked = [&](uint32_t i, uint32_t o, uint32_t cnt) {
+    const uint32_t room = cap - o;
+    const uint32_t keep = cnt < room ? cnt : room;
+    const float4 mn = d.nmin[nb + N - 1 + i], mx = d.nmax[nb + N - 1 + i];
+    traverse(d, nb, N, i, ld3(mn), ld3(mx), [&](uint32_t k, uint32_t j) {
+      if (k < keep) pairs[o + k] = make_uint2(i, j);
+    });
+    for (uint32_t a = 1; a < keep; ++a) {
+      uint2 x = pairs[o + a];
+      uint32_t b2 = a;
+      while (b2 > 0 && pairs[o + b2 - 1].y > x.y) {
+        pairs[o + b2] = pairs[o + b2 - 1];
+        --b2;
+      }
+      pairs[o + b2] = x;
+    }
+    if (!vox) return;
+    const bool vi = is_vox(i);
+    uint32_t end = o;
+    for (uint32_t a = 0; a < keep; ++a) end += (vi || is_vox(pairs[o + a].y)) ? 6u : 1u;
+    for (uint32_t a = keep; a-- > 0;) {
+      const uint32_t j = pairs[o + a].y;
+      const uint32_t rep = (vi || is_vox(j)) ? 6u : 1u;
+      end -= rep;
+      for (uint32_t r = 0; r < rep; ++r)
+        if (end + r < cap) pairs[end + r] = make_uint2(i, j);
+    }
+  };
+  if (broad_flat(d, nb, N, t)) {
+    const uint32_t lane = threadIdx.x & (WAVE - 1);
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (uint32_t i = tid / WAVE; i < N; i += NT / WAVE) {
+      const uint32_t o = d.poff[off + i], cnt = d.pcount[off + i];
+      if (cnt == 0u || o >= cap) continue;
+      if (cnt > cap - o && (!vox || cnt > kPairStage)) {
+        // cut by the capacity: the partners the walk finds first, or of a row
+        // that a workgroup would walk the first in order
+        uint32_t done = 0u;
+        if (lane == 0u) {
+          const uint32_t budget = vox ? kMAX : (d.walk_budget ? d.walk_budget : kWalkBudgetDefault);
+          const uint32_t leaf = nb + N - 1u + i;
+          done = walk(d, nb, N, i, ld3(d.nmin[leaf]), ld3(d.nmax[leaf]), __float_as_int(d.nmin[nb].w),
+                      __float_as_int(d.nmax[nb].w), budget, [] { return true; }, [](uint32_t, uint32_t) {}) != kMAX;
+          if (done) write_walked(i, o, cnt);
+        }
+        if (__shfl(done, 0, WAVE)) continue;
+      }
+      const bool vi = vox && is_vox(i);
+      uint32_t at = o;
+      flat_row(d, nb, N, i, [&](uint32_t j, uint64_t m) {
+        const bool mine = (m >> lane) & 1ull;
+        uint64_t vm = 0ull;
+        if (vox) vm = vi ? m : __ballot(mine && is_vox(j));
+        if (mine) {
+          const uint32_t p = at + (uint32_t)__popcll(m & below) + 5u * (uint32_t)__popcll(vm & below);
+          const uint32_t reps = (vm >> lane) & 1ull ? 6u : 1u;
+          for (uint32_t r = 0; r < reps; ++r)
+            if (p + r < cap) pairs[p + r] = make_uint2(i, j);
+        }
+        at += (uint32_t)__popcll(m) + 5u * (uint32_t)__popcll(vm);
+      });
+    }
+    return;
+  }
+  if constexpr (T::kSpread) {
+    // this workgroup's rows that were handed to a workgroup, listed again
+    if (t.lead()) L.ndefer = 0;
+    t.sync();
+    for (uint32_t i = tid; i < N; i += NT)
+      if (d.pcount[off + i] & kDeferBit) {
+        const uint32_t k = atomicAdd(&L.ndefer, 1u);
+        if (k < kMaxDefer) L.defer[k] = i;  // at most kMaxDefer of them were marked
+      }
+    t.sync();
+  }
+  const uint32_t nd = L.ndefer < kMaxDefer ? L.ndefer : kMaxDefer;
   if (vox) {
     // partners in ascending row order, each written 1 or 6 times; slots past
     // the capacity are dropped (the overflow flag is set)
@@ -1207,33 +1396,7 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
         });
         continue;
       }
-      // more partners than the staging area: traverse again into the slot
-      // range (it holds at least cnt entries), sort there, then expand from
-      // the back (an entry only moves to a higher or equal slot)
-      const uint32_t room = cap - o;
-      const uint32_t keep = cnt < room ? cnt : room;
-      float4 mn = d.nmin[nb + N - 1 + i], mx = d.nmax[nb + N - 1 + i];
-      traverse(d, nb, N, i, ld3(mn), ld3(mx), [&](uint32_t k, uint32_t j) {
-        if (k < keep) pairs[o + k] = make_uint2(i, j);
-      });
-      for (uint32_t a = 1; a < keep; ++a) {
-        uint2 x = pairs[o + a];
-        uint32_t b2 = a;
-        while (b2 > 0 && pairs[o + b2 - 1].y > x.y) {
-          pairs[o + b2] = pairs[o + b2 - 1];
-          --b2;
-        }
-        pairs[o + b2] = x;
-      }
-      uint32_t end = o;
-      for (uint32_t a = 0; a < keep; ++a) end += (vi || is_vox(pairs[o + a].y)) ? 6u : 1u;
-      for (uint32_t a = keep; a-- > 0;) {
-        const uint32_t j = pairs[o + a].y;
-        const uint32_t rep = (vi || is_vox(j)) ? 6u : 1u;
-        end -= rep;
-        for (uint32_t r = 0; r < rep; ++r)
-          if (end + r < cap) pairs[end + r] = make_uint2(i, j);
-      }
+      write_walked(i, o, cnt);
     }
     return;
   }
@@ -1258,21 +1421,7 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
       });
       continue;
     }
-    // more partners than the staging area holds: traverse again, writing the
-    // first `room` partners straight into the pair list, then sort them
-    float4 mn = d.nmin[nb + N - 1 + i], mx = d.nmax[nb + N - 1 + i];
-    traverse(d, nb, N, i, ld3(mn), ld3(mx), [&](uint32_t k, uint32_t j) {
-      if (k < keep) pairs[o + k] = make_uint2(i, j);
-    });
-    for (uint32_t a = 1; a < keep; ++a) {
-      uint2 x = pairs[o + a];
-      uint32_t b2 = a;
-      while (b2 > 0 && pairs[o + b2 - 1].y > x.y) {
-        pairs[o + b2] = pairs[o + b2 - 1];
-        --b2;
-      }
-      pairs[o + b2] = x;
-    }
+    write_walked(i, o, cnt);
   }
   // the rows handed to a workgroup: the first `room` partners, in order
   for (uint32_t k = t.group(); k < nd; k += t.groups()) {
@@ -1285,8 +1434,19 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
   }
 }
 
+template <class T>
+BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds<T::kBlock>& F) {
+  s_broad_count(d, w, t, L, F);
+  t.sync();
+  s_broad_scan(d, w, t);
+  t.sync();
+  s_broad_write(d, w, t, L, F);
+}
+
+// Eight waves per SIMD, which hide the walks' loads in a crowded launch (with
+// both forms the compiler would take 67 registers, which leaves seven).
 template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_broad(Dev d) {
+__global__ __launch_bounds__(BLOCK, 8) void k_broad(Dev d) {
   __shared__ BroadShared L;
   __shared__ ScanLds<BLOCK> S;
   __shared__ WalkLds<BLOCK> F;
@@ -1294,6 +1454,26 @@ __global__ __launch_bounds__(BLOCK) void k_broad(Dev d) {
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{&S, nullptr};
   s_broad(d, w, t, L, F);
+}
+// The same in three launches, the walks by several workgroups per world.
+template <int BLOCK, bool kWrite>
+__global__ __launch_bounds__(BLOCK) void k_broad_walk(Dev d) {
+  __shared__ BroadShared L;
+  __shared__ ScanLds<BLOCK> S;
+  __shared__ WalkLds<BLOCK> F;
+  const uint32_t w = d.order[blockIdx.x / d.spread];
+  if (d.worlds[w].mode & kModeTeam) return;
+  const SpreadTeam<BLOCK> t{blockIdx.x % d.spread, d.spread, &S};
+  if constexpr (kWrite) s_broad_write(d, w, t, L, F);
+  else s_broad_count(d, w, t, L, F);
+}
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_broad_scan(Dev d) {
+  __shared__ ScanLds<BLOCK> S;
+  const uint32_t w = d.order[blockIdx.x];
+  if (d.worlds[w].mode & kModeTeam) return;
+  const BlockTeam<BLOCK> t{&S, nullptr};
+  s_broad_scan(d, w, t);
 }
 
 // ==================================================== narrow phase (SAT)
@@ -2222,17 +2402,17 @@ BB_DI void s_narrow(const Dev& d, uint32_t w, const T& t) {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_narrow_vox(Dev d) {
-  const uint32_t w = d.order[blockIdx.x];
+  const uint32_t w = d.order[blockIdx.x / d.spread];
   if (d.worlds[w].mode & kModeTeam) return;
-  const BlockTeam<BLOCK> t{nullptr, nullptr};
+  const SpreadTeam<BLOCK> t{blockIdx.x % d.spread, d.spread, nullptr};
   s_narrow<true>(d, w, t);
 }
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_narrow(Dev d) {
-  const uint32_t w = d.order[blockIdx.x];
+  const uint32_t w = d.order[blockIdx.x / d.spread];
   if (d.worlds[w].mode & kModeTeam) return;
-  const BlockTeam<BLOCK> t{nullptr, nullptr};
+  const SpreadTeam<BLOCK> t{blockIdx.x % d.spread, d.spread, nullptr};
   s_narrow<false>(d, w, t);
 }
 
@@ -2330,9 +2510,9 @@ BB_DI void s_contacts(const Dev& d, uint32_t w, const T& t) {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK) void k_contacts(Dev d) {
-  const uint32_t w = d.order[blockIdx.x];
+  const uint32_t w = d.order[blockIdx.x / d.spread];
   if (d.worlds[w].mode & kModeTeam) return;
-  const BlockTeam<BLOCK> t{nullptr, nullptr};
+  const SpreadTeam<BLOCK> t{blockIdx.x % d.spread, d.spread, nullptr};
   s_contacts(d, w, t);
 }
 
@@ -4814,7 +4994,7 @@ __global__ __launch_bounds__(256) void k_copy_calibrate(const float4* __restrict
 // holds the team kernel, the launch sequence and the small utility kernels.
 namespace bb {
 static constexpr int kStages = 7;
-static constexpr uint32_t kCus = 256;  // CUs of the chip
+static constexpr uint32_t kMaxSpread = 16, kMinBroadSpread = 4, kMinBroadRows = 256;
 template <int B>
 void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid);
 template <int B>
@@ -4833,6 +5013,20 @@ Dev sweep_form(const Dev& d, uint32_t grid) {
   r.pgs_quad_rows = d.pgs_quads || grid <= kCus ? (uint32_t)B / 4u : 16u;
   return r;
 }
+// A launch of few worlds leaves CUs idle, and the narrow phase's pairs and the
+// broad phase's rows need no workgroup of their own: up to kMaxSpread
+// workgroups per world, as far as the chip has CUs for them (one 1,501-body
+// world: narrow 147 -> 28, contacts 200 -> 45 us), or as many as the caller
+// asks for (d.spread: most slots of a serving pool are empty, and a workgroup
+// that finds none of its own ends at once).  The broad phase pays two more
+// launches for it, about 6 us, so it takes kMinBroadSpread workgroups and
+// worlds of more than kMinBroadRows bodies (1,001 bodies: 144 -> 41 us; a
+// world of 49 is through in 23 us with one).
+static Dev spread_form(const Dev& d, uint32_t grid) {
+  Dev r = d;
+  r.spread = std::max(std::max(1u, d.spread), std::min(kMaxSpread, kCus / grid));
+  return r;
+}
 // Stages of the per-world path, in launch order (k_team, when there is one,
 // goes before the first).  Stage k of the timed launch is bracketed by events
 // ev[k] and ev[k + 1]; the narrow phase's two kernels share stage 2; the
@@ -4843,12 +5037,25 @@ void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid) {
   const dim3 g(grid), b(B);
   switch (stage) {
     case 0: hipLaunchKernelGGL(k_build<B>, g, b, 0, st, d); break;
-    case 1: hipLaunchKernelGGL(k_broad<B>, g, b, 0, st, d); break;
-    case 2:
-      hipLaunchKernelGGL(k_narrow<B>, g, b, 0, st, d);
-      if (d.any_voxel) hipLaunchKernelGGL(k_narrow_vox<B>, g, b, 0, st, d);
-      hipLaunchKernelGGL(k_contacts<B>, g, b, 0, st, d);
+    case 1: {
+      const Dev s = spread_form(d, grid);
+      if (s.spread < kMinBroadSpread || d.lane_max <= kMinBroadRows) {
+        hipLaunchKernelGGL(k_broad<B>, g, b, 0, st, d);
+        break;
+      }
+      hipLaunchKernelGGL((k_broad_walk<B, false>), dim3(grid * s.spread), b, 0, st, s);
+      hipLaunchKernelGGL(k_broad_scan<B>, g, b, 0, st, s);
+      hipLaunchKernelGGL((k_broad_walk<B, true>), dim3(grid * s.spread), b, 0, st, s);
       break;
+    }
+    case 2: {
+      const Dev s = spread_form(d, grid);
+      const dim3 gs(grid * s.spread);
+      hipLaunchKernelGGL(k_narrow<B>, gs, b, 0, st, s);
+      if (s.any_voxel) hipLaunchKernelGGL(k_narrow_vox<B>, gs, b, 0, st, s);
+      hipLaunchKernelGGL(k_contacts<B>, gs, b, 0, st, s);
+      break;
+    }
     case 3: hipLaunchKernelGGL(k_post<B>, g, b, 0, st, d); break;
     case 4:
       if (d.any_island) hipLaunchKernelGGL(k_levels<B>, g, b, 0, st, d);
