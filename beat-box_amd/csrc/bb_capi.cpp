@@ -1687,33 +1687,19 @@ bb_status read_world(bb_batch* b, uint32_t w, bb_body_state* out, uint32_t n, bb
   if (n < hw.bodies.size()) return BB_ERR_INVALID;
   bb_status st = build(b);
   if (st != BB_OK) return st;
-  HIPCHK(hipStreamSynchronize(b->stream));
-  const uint32_t N = hw.n, g0 = hw.body_off;
-  const Rows& R = b->rows[b->latest];
-  std::vector<uint32_t> id(N), fl(N), isl(N, kMAX), ent(N);
-  std::vector<float4> pos(N), rot(N), vel(N), omg(N);
+  // packed by a kernel into the contact points' array, which a step writes
+  // before it reads (128 bytes for each of at least 8 n pair slots, and a
+  // state is 68), and copied once
+  static_assert(sizeof(bb_body_state) <= 8 * 8 * sizeof(float4), "");
+  const uint32_t N = hw.n;
   if (N) {
-    HIPCHK(hipMemcpy(id.data(), R.id + g0, N * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(fl.data(), R.flags + g0, N * 4, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(pos.data(), R.pos + g0, N * 16, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(rot.data(), R.rot + g0, N * 16, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(vel.data(), R.vel + g0, N * 16, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(omg.data(), R.omg + g0, N * 16, hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(ent.data(), b->entries[b->latest] + g0, N * 4, hipMemcpyDeviceToHost));
-    if (b->stepped) HIPCHK(hipMemcpy(isl.data(), b->base.islot + g0, N * 4, hipMemcpyDeviceToHost));
+    std::lock_guard<std::mutex> lock(b->read_mutex);
+    const Dev d = dev_for(b, b->latest);
+    launch_pack(d, hw.body_off, N, order == BB_ORDER_BY_ID, b->stepped, d.sv_cp, b->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(out, d.sv_cp, (size_t)N * sizeof(bb_body_state), hipMemcpyDeviceToHost, b->stream));
   }
-  for (uint32_t k = 0; k < N; ++k) {
-    uint32_t row = order == BB_ORDER_BY_ID ? ent[k] : k;
-    bb_body_state& o = out[k];
-    o.id = id[row];
-    o.flags = fl[row];
-    o.island_index = isl[row];
-    o.row = row;
-    o.position[0] = pos[row].x; o.position[1] = pos[row].y; o.position[2] = pos[row].z;
-    o.rotation[0] = rot[row].x; o.rotation[1] = rot[row].y; o.rotation[2] = rot[row].z; o.rotation[3] = rot[row].w;
-    o.velocity[0] = vel[row].x; o.velocity[1] = vel[row].y; o.velocity[2] = vel[row].z;
-    o.omega[0] = omg[row].x; o.omega[1] = omg[row].y; o.omega[2] = omg[row].z;
-  }
+  HIPCHK(hipStreamSynchronize(b->stream));
   return BB_OK;
 }
 

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <functional>
+#include <mutex>
 #include <vector>
 
 #include "../../include/bb_capi.h"
@@ -22,6 +23,7 @@ void launch_step_timed(const Lane* lanes, int nl, hipStream_t st, hipEvent_t* ev
 void launch_copy(const float4* src, float4* dst, size_t n, hipStream_t st);
 void launch_sum_counts(const Dev& d, unsigned long long* out, hipStream_t st);
 void launch_energy(const Dev& d, double* out, hipStream_t st);
+void launch_pack(const Dev& d, uint32_t body_off, uint32_t n, bool by_id, bool stepped, void* dst, hipStream_t st);
 void launch_instances(const Dev& d, uint32_t w, uint32_t n, float* dst, hipStream_t st);
 // World w's `nodes` (= 2n-1) BVH nodes as 40-byte LBVHNode records into dst.
 void launch_lbvh_export(const Dev& d, uint32_t w, uint32_t nodes, void* dst, hipStream_t st);
@@ -147,6 +149,7 @@ struct bb_batch {
   int latest = 0;  // buffer set holding the newest state
   uint32_t NB = 0, NA = 0, NP = 0;
   hipStream_t stream = nullptr;
+  std::mutex read_mutex;  // readbacks share the scratch they are packed in
   uint32_t block = 0;
   uint32_t pgs_lds = 512;  // BB_PARAM_PGS_LDS_ROWS
   uint32_t team_bodies = 8192;  // BB_PARAM_TEAM_BODIES: worlds this large run in k_team

@@ -4846,6 +4846,35 @@ __global__ __launch_bounds__(256) void k_instances(Dev d, uint32_t w, float* __r
   o[2] = make_float4(R.m[2][0], R.m[2][1], R.m[2][2], p.z);
 }
 
+// Readback of one world: n bb_body_state records (17 words) in dst, by id or
+// by row, with the row's island slot (kMAX before the first step).  Eight
+// copies gathered on the host cost a frame of 27 bodies 75 of its 542 us and
+// one of 1,001 bodies 80 of 1,010 more than this and one copy.  The records are put
+// together in LDS (17 words apart: no bank conflict) and leave in one stream
+// of words, since a lane's own record would touch two lines per store.
+static constexpr uint32_t kStateWords = sizeof(bb_body_state) / 4u;
+__global__ __launch_bounds__(256) void k_pack(Dev d, uint32_t body_off, uint32_t n, uint32_t by_id, uint32_t stepped,
+                                              uint32_t* __restrict__ dst) {
+  static_assert(kStateWords == 17, "the record as it is written below");
+  __shared__ uint32_t rec[256 * kStateWords];
+  const uint32_t i0 = blockIdx.x * 256u, i = i0 + threadIdx.x;
+  if (i < n) {
+    const uint32_t row = by_id ? d.entries_cur[body_off + i] : i, g = body_off + row;
+    uint32_t* r = rec + threadIdx.x * kStateWords;
+    const float4 p = d.cur.pos[g], q = d.cur.rot[g], v = d.cur.vel[g], o = d.cur.omg[g];
+    const float f[13] = {p.x, p.y, p.z, q.x, q.y, q.z, q.w, v.x, v.y, v.z, o.x, o.y, o.z};
+    r[0] = d.cur.id[g];
+    r[1] = d.cur.flags[g];
+    r[2] = stepped ? d.islot[g] : kMAX;
+    r[3] = row;
+#pragma unroll
+    for (uint32_t k = 0; k < 13u; ++k) r[4u + k] = __float_as_uint(f[k]);
+  }
+  __syncthreads();
+  const uint32_t words = (n - i0 < 256u ? n - i0 : 256u) * kStateWords;
+  for (uint32_t k = threadIdx.x; k < words; k += 256u) dst[(size_t)i0 * kStateWords + k] = rec[k];
+}
+
 // LBVH hand-off (RigidBodyManager::get_lbvh_node_buffer, src/
 // rigid_body_manager.cpp:1601-1604, consumed as procedural AABB geometry
 // with a 40-byte stride by src/acceleration_structure_manager.cpp:490-535):
@@ -5153,6 +5182,12 @@ void launch_sum_counts(const Dev& d, unsigned long long* out, hipStream_t st) {
 
 void launch_instances(const Dev& d, uint32_t w, uint32_t n, float* dst, hipStream_t st) {
   if (n) hipLaunchKernelGGL(k_instances, dim3((n + 255u) / 256u), dim3(256), 0, st, d, w, dst);
+}
+
+void launch_pack(const Dev& d, uint32_t body_off, uint32_t n, bool by_id, bool stepped, void* dst, hipStream_t st) {
+  if (n)
+    hipLaunchKernelGGL(k_pack, dim3((n + 255u) / 256u), dim3(256), 0, st, d, body_off, n, by_id ? 1u : 0u,
+                       stepped ? 1u : 0u, static_cast<uint32_t*>(dst));
 }
 
 void launch_lbvh_export(const Dev& d, uint32_t w, uint32_t nodes, void* dst, hipStream_t st) {
