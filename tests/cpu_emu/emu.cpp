@@ -279,7 +279,10 @@ void launch(dim3 grid, dim3 block, size_t shmem, std::function<void()> fn) {
     for (auto& t : th) t.join();
     return;
   }
-  if (G <= 256) {
+  // every workgroup at once (teams meet at barriers), as far as the stacks'
+  // mappings go (two per thread, 65,530 by default); launches beyond have no
+  // barrier between workgroups
+  if (G <= 256 && (uint64_t)G * block.x <= 30000u) {
     std::vector<std::thread> th;
     th.reserve(G);
     for (uint32_t b = 0; b < G; ++b) th.emplace_back([&, b] { run_block(b, grid, block, shmem, fn); });
