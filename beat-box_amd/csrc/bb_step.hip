@@ -3301,7 +3301,9 @@ BB_DI float qmulmv(v3 m, float x) { return (m.x * qc0(x) + m.y * qc1(x)) + m.z *
 // What the PGS sweeps of a world keep in LDS, in floats: for its first `rows`
 // body rows velocity, inverse mass, angular velocity, position at detection
 // and world inverse inertia (19 of kBodyLds floats each; the rest stay in
-// HBM).  kMem: every body row in LDS, none, or by row.
+// HBM).  kMem: every body row in LDS, none, or by row.  lds: 16-byte aligned
+// (the kernels declare their dynamic LDS as float4, which follows any static
+// LDS at that alignment).
 static constexpr uint32_t kBodyLds = 20;
 static constexpr int kPgsPre = 4;
 enum : int { kMemLds = 0, kMemHbm = 1, kMemBoth = 2 };
@@ -3856,7 +3858,8 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t 
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_pgs(Dev d) {
-  HIP_DYNAMIC_SHARED(float, pgs_lds)
+  HIP_DYNAMIC_SHARED(float4, dyn_lds)
+  float* const pgs_lds = reinterpret_cast<float*>(dyn_lds);
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{nullptr, nullptr};
@@ -3865,7 +3868,8 @@ __global__ __launch_bounds__(BLOCK, 4) void k_pgs(Dev d) {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_pgs_island(Dev d) {
-  HIP_DYNAMIC_SHARED(float, pgs_lds)
+  HIP_DYNAMIC_SHARED(float4, dyn_lds)
+  float* const pgs_lds = reinterpret_cast<float*>(dyn_lds);
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{nullptr, nullptr};
@@ -4793,7 +4797,8 @@ size_t fused_lds(uint32_t pgs_rows) {
 
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
-  HIP_DYNAMIC_SHARED(float, pgs_lds)
+  HIP_DYNAMIC_SHARED(float4, dyn_lds)
+  float* const pgs_lds = reinterpret_cast<float*>(dyn_lds);
   __shared__ FusedShared<BLOCK> G;
   __shared__ ScanLds<BLOCK> S;
   const uint32_t w = d.order[blockIdx.x];

@@ -2,7 +2,8 @@
 
 The kernels of beat-box_amd/csrc/bb_step.hip and the host code of the C-ABI
 (bb_capi.cpp, bb_server.cpp) are compiled unchanged by g++, against the HIP
-emulation header in tests/cpu_emu/hip/, with AddressSanitizer.  emu_main
+emulation header in tests/cpu_emu/hip/, with AddressSanitizer and checks of
+every access's alignment.  emu_main
 (main.cpp) steps the worlds of a scene file through the C-ABI.
 """
 from __future__ import annotations
@@ -17,6 +18,7 @@ REPO = os.path.dirname(os.path.dirname(HERE))
 CSRC = os.path.join(REPO, "beat-box_amd", "csrc")
 OUT_DIR = os.path.join(HERE, "_build")
 FLAGS = ["-std=c++17", "-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address",
+         "-fsanitize=alignment", "-fno-sanitize-recover=alignment",
          "-ffp-contract=off", "-w", "-I", HERE]
 # (source, compile as C++, extra flags, object name): bb_step_block.hip once
 # per workgroup size, as the library's build does

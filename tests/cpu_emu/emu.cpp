@@ -59,7 +59,7 @@ std::atomic<long> g_inactive_src{0};
 
 Fiber* cur() { return t_cur; }
 const dim3& tid_of(Fiber* f) { return f->tid; }
-void* dyn_lds() { return t_blk->dyn.data(); }
+void* dyn_lds(size_t align) { return t_blk->dyn.data() + (align < 16 ? align : 16); }
 
 static void to_sched(Fiber* f) {
 #if EMU_ASAN
@@ -195,7 +195,7 @@ static void run_block(uint32_t bx, dim3 grid, dim3 block, size_t shmem, const st
   t_grid = grid;
   t_bdim = block;
   B.fn = &fn;
-  B.dyn.assign(shmem ? shmem : 16, (char)0xA5);
+  B.dyn.assign((shmem ? shmem : 16) + 16, (char)0xA5);
   const uint32_t n = block.x;
   B.f.resize(n);
   for (uint32_t i = 0; i < n; ++i) {

@@ -27,17 +27,19 @@
 #define __launch_bounds__(...)
 #define __shared__ static thread_local
 #define __align__(x) alignas(x)
-#define HIP_DYNAMIC_SHARED(type, var) type* var = (type*)emu::dyn_lds();
+// dynamic LDS follows the static LDS at no more than its declared alignment
+#define HIP_DYNAMIC_SHARED(type, var) type* var = (type*)emu::dyn_lds(alignof(type));
 
 struct dim3 {
   uint32_t x, y, z;
   constexpr dim3(uint32_t a = 1, uint32_t b = 1, uint32_t c = 1) : x(a), y(b), z(c) {}
 };
 
+// (the vectors of two and four with the alignment they have on the device)
 #define EMU_VEC4(T, N)                                                  \
-  struct N##4 { T x, y, z, w; };                                        \
+  struct alignas(sizeof(T) < 8 ? 16 : 8) N##4 { T x, y, z, w; };        \
   struct N##3 { T x, y, z; };                                           \
-  struct N##2 { T x, y; };                                              \
+  struct alignas(8) N##2 { T x, y; };                                   \
   static inline N##4 make_##N##4(T a, T b, T c, T d) { return N##4{a, b, c, d}; } \
   static inline N##3 make_##N##3(T a, T b, T c) { return N##3{a, b, c}; } \
   static inline N##2 make_##N##2(T a, T b) { return N##2{a, b}; }
@@ -55,7 +57,7 @@ void barrier();
 void yield();
 [[noreturn]] void end_program();
 uint64_t wave_op(int kind, uint64_t v, int arg, int width);
-void* dyn_lds();
+void* dyn_lds(size_t align);
 void launch(dim3 grid, dim3 block, size_t shmem, std::function<void()> fn);
 }  // namespace emu
 

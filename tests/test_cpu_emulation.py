@@ -52,11 +52,11 @@ def _scene(path, worlds, shapes=()):
 
 
 def _run(exe, scene, out, steps, team_bodies, block, graph=1, lane_bodies=0, single=0, team_spin=0,
-         max_blocks=0, sort_blocks=0, walk_budget=0, pgs_block=0, pgs_lds=512):
+         max_blocks=0, sort_blocks=0, walk_budget=0, pgs_block=0, pgs_lds=512, fused=0):
     env = dict(ENV, EMU_MAX_BLOCKS=str(max_blocks)) if max_blocks else ENV
     r = subprocess.run([exe, scene, str(steps), str(team_bodies), str(block), str(graph), out, str(lane_bodies),
                         str(single), str(team_spin), str(sort_blocks), str(walk_budget), str(pgs_block),
-                        str(pgs_lds)],
+                        str(pgs_lds), str(fused)],
                        capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stderr[-3000:]
     assert "AddressSanitizer" not in r.stderr, r.stderr[-3000:]
@@ -358,3 +358,19 @@ def test_broad_phase_rows_handed_to_the_workgroup_equal_one_thread_walks(emu_mai
     for team, block, budget in ((0, 256, 1), (0, 1024, 4), (600, 256, 1), (600, 0, 4)):
         log, x = _run(emu_main, scene, str(tmp_path / "x.bin"), 4, team, block, walk_budget=budget)
         assert log == ref_log and x == ref, (team, block, budget)
+
+
+@pytest.mark.parametrize("block", [128, 512])
+def test_one_launch_steps_are_aligned_and_identical(emu_main, tmp_path, block):
+    """The one-launch step (BB_PARAM_FUSED) of a PGS and an AVBD world: its
+    vector accesses to dynamic LDS keep their alignment (the emulation places
+    that LDS at its declared alignment and no better), and its steps are the
+    staged ones."""
+    avbd = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10,
+                                                      morton_bits=63, quirks=0))
+    pgs = beatbox.WorldDesc.make(**scenes.world_desc(iterations=8, morton_bits=63, quirks=0))
+    scene = str(tmp_path / "scene.bin")
+    _scene(scene, [(avbd, scenes.serving_pile(41, 80)), (pgs, scenes.serving_pile(42, 90))])
+    a, x = _run(emu_main, scene, str(tmp_path / "a.bin"), 3, 0, block, graph=0, fused=1)
+    b, y = _run(emu_main, scene, str(tmp_path / "b.bin"), 3, 0, block, graph=0)
+    assert a == b and x == y
