@@ -3441,13 +3441,18 @@ BB_DI void pgs_fetch(const PgsRows& S, uint32_t k, uint32_t ln, PgsRow& R) {
 }
 // Row k of the world's rows, fetched into R.  kWarm: the warm-start impulses
 // of pre_step; otherwise one solve (with bias, or a relaxation).  kPlain: PGS
-// (the per-island path) instead of PGS_SOFT.  kUsual: impulses accumulate
-// and there is friction (the default flags), so neither is tested per
-// contact.  ln: this lane's place in its quad.
-template <bool kPlain, bool kWarm, bool kUsual, int kMem>
+// (the per-island path) instead of PGS_SOFT.  kFlags: whether impulses
+// accumulate and whether there is friction, or kPgsAny (tested per contact).
+// ln: this lane's place in its quad.
+static constexpr uint32_t kPgsUsual = BB_SIM_ACCUM_IMPULSE | BB_SIM_FRICTION;  // the default
+static constexpr uint32_t kPgsAny = 1u << 31;
+template <uint32_t kFlags>
+using PgsForm = std::integral_constant<uint32_t, kFlags>;
+template <bool kPlain, bool kWarm, uint32_t kFlags, int kMem>
 BB_DI void pgs_solve(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc, uint32_t k, uint32_t ln, const Pgs& s,
                      bool use_bias, const PgsRow& R) {
-  const bool accum = kUsual || s.accum, friction = kUsual || s.friction;
+  const bool accum = kFlags & kPgsAny ? s.accum : (kFlags & BB_SIM_ACCUM_IMPULSE) != 0;
+  const bool friction = kFlags & kPgsAny ? s.friction : (kFlags & BB_SIM_FRICTION) != 0;
   const uint32_t q = k * 4u + ln;
   const int4 h = R.h;
   const int count = h.z & 255;
@@ -3572,10 +3577,11 @@ BB_DI void pgs_fetch_lane(const PgsRows& S, uint32_t k, PgsLaneRow& R) {
   R.t0z = S.t0z[k];
   R.c0 = pgs_contact(S, k, 0);
 }
-// Row k by one lane, with the default flags (impulses accumulate, friction).
-template <bool kPlain, bool kWarm, int kMem>
+// Row k by one lane.
+template <bool kPlain, bool kWarm, uint32_t kFlags, int kMem>
 BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc, uint32_t k, const Pgs& s,
                           bool use_bias, const PgsLaneRow& R) {
+  constexpr bool accum = (kFlags & BB_SIM_ACCUM_IMPULSE) != 0, friction = (kFlags & BB_SIM_FRICTION) != 0;
   const int4 h = R.h;
   const int count = h.z & 255;
   const bool da = (h.z & 256) != 0, db = (h.z & 512) != 0;
@@ -3611,25 +3617,33 @@ BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc
     v3 l = x.l;
     if constexpr (kWarm) {
       v3 P = n * l.x;
-      P = P + t0 * l.y;
-      P = P + t1 * l.z;
+      if (friction) {
+        P = P + t0 * l.y;
+        P = P + t1 * l.z;
+      }
       apply(P, r1, r2);
     } else {
       const float pen = x.cp.w, nm = x.m.x;
       auto rel_vel = [&]() __attribute__((always_inline)) {
         return ((vb + cross(wb, r2)) - va) - cross(wa, r1);
       };
-      const v3 rv = rel_vel();
-      const float maxf = fr * l.x;
-      auto tangent = [&](v3 t, float tmass, float& lt) __attribute__((always_inline)) {
-        const float ti = tmass * -dot(rv, t);
-        const float nw = fcl(lt + ti, -maxf, maxf);
-        const float di = nw - lt;
-        lt = nw;
-        apply(t * di, r1, r2);
-      };
-      tangent(t0, x.m.y, l.y);
-      tangent(t1, x.m.z, l.z);
+      if (friction) {
+        const v3 rv = rel_vel();
+        const float maxf = fr * l.x;
+        auto tangent = [&](v3 t, float tmass, float& lt) __attribute__((always_inline)) {
+          float ti = tmass * -dot(rv, t);
+          if (accum) {
+            const float nw = fcl(lt + ti, -maxf, maxf);
+            ti = nw - lt;
+            lt = nw;
+          } else {
+            ti = fcl(ti, -maxf, maxf);
+          }
+          apply(t * ti, r1, r2);
+        };
+        tangent(t0, x.m.y, l.y);
+        tangent(t1, x.m.z, l.z);
+      }
       const float nv = dot(rel_vel(), n);
       float imp;
       if (kPlain) {
@@ -3641,9 +3655,14 @@ BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc
         const float impulse_scale = soft ? impulse_coef : 0.0f;
         imp = -nm * mass_scale * (nv + bias) - impulse_scale * l.x;
       }
-      const float old = l.x;
-      l.x = fmx(old + imp, 0.0f);
-      apply(n * (l.x - old), r1, r2);
+      if (accum) {
+        const float old = l.x;
+        l.x = fmx(old + imp, 0.0f);
+        imp = l.x - old;
+      } else {
+        imp = fmx(imp, 0.0f);
+      }
+      apply(n * imp, r1, r2);
       reinterpret_cast<v3*>(S.l_at(c))[k] = l;
     }
     x = next;
@@ -3656,15 +3675,14 @@ BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc
 // dependency levels), c < nr, a barrier after each non-empty one, then the
 // rows [ovf_lo, ovf_hi) one after another by the first quad.  Row k is always
 // solved by the same lanes.  Ranges of at most quad_rows rows go to quads,
-// longer ones to single lanes (kUsual; otherwise all go to quads).
-template <bool kPlain, bool kWarm, bool kUsual, int kMem, class T>
+// longer ones to single lanes (kPgsAny: all to quads).
+template <bool kPlain, bool kWarm, uint32_t kFlags, int kMem, class T>
 BB_DI void pgs_sweep(const Dev& d, const T& t, const PgsLds<kMem>& vc, const Pgs& s, const PgsRows& S,
                      const uint32_t* ro, uint32_t nr, uint32_t ovf_lo, uint32_t ovf_hi, bool use_bias,
                      uint32_t quad_rows) {
   const uint32_t tid = t.rank(), NT = t.size();
   const uint32_t ln = tid & 3u, q = tid >> 2, NQ = NT >> 2;
   const uint32_t wl = tid & (WAVE - 1);
-  if (kWarm && !s.accum) return;
   // offsets of up to WAVE - 1 ranges, one per lane
   uint32_t chunk = 0, offs = wl <= nr ? ro[wl] : 0u;
   auto bound = [&](uint32_t c) __attribute__((always_inline)) {  // ro[c], c uniform and ascending
@@ -3684,23 +3702,23 @@ BB_DI void pgs_sweep(const Dev& d, const T& t, const PgsLds<kMem>& vc, const Pgs
   bool have = false;  // R holds this quad's first row of the range
   for (uint32_t c = 0; c < nr && lo < end; ++c) {
     const uint32_t hi2 = c + 2 <= nr ? bound(c + 2) : hi;
-    if (!kUsual || hi - lo <= quad_rows) {
+    if (kFlags == kPgsAny || hi - lo <= quad_rows) {
       if (!have) pgs_fetch(S, in(lo + q), ln, R);
       for (uint32_t k0 = lo; k0 < hi; k0 += NQ) {
         const uint32_t k = k0 + q;
         PgsRow X;
         pgs_fetch(S, in((k0 + NQ < hi ? k0 + NQ : hi) + q), ln, X);
-        if (k < hi) pgs_solve<kPlain, kWarm, kUsual, kMem>(d, S, vc, k, ln, s, use_bias, R);
+        if (k < hi) pgs_solve<kPlain, kWarm, kFlags, kMem>(d, S, vc, k, ln, s, use_bias, R);
         R = X;
       }
       have = true;
-    } else {
+    } else if constexpr (kFlags != kPgsAny) {
       have = false;
       PgsLaneRow L;
       pgs_fetch_lane(S, in(lo + tid), L);
       for (uint32_t k0 = lo; k0 < hi; k0 += NT) {
         const uint32_t k = k0 + tid;
-        if (k < hi) pgs_solve_lane<kPlain, kWarm, kMem>(d, S, vc, k, s, use_bias, L);
+        if (k < hi) pgs_solve_lane<kPlain, kWarm, kFlags, kMem>(d, S, vc, k, s, use_bias, L);
         if (k0 + NT < hi) pgs_fetch_lane(S, in(k + NT), L);
       }
     }
@@ -3712,7 +3730,7 @@ BB_DI void pgs_sweep(const Dev& d, const T& t, const PgsLds<kMem>& vc, const Pgs
     if (q == 0)
       for (uint32_t r = ovf_lo; r < ovf_hi; ++r) {
         pgs_fetch(S, r, ln, R);
-        pgs_solve<kPlain, kWarm, kUsual, kMem>(d, S, vc, r, ln, s, use_bias, R);
+        pgs_solve<kPlain, kWarm, kFlags, kMem>(d, S, vc, r, ln, s, use_bias, R);
       }
     t.sync();
   }
@@ -3774,20 +3792,45 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t 
   const uint32_t nr = nlev ? nlev : used;
   const uint32_t olo = nlev ? 0u : ovf_lo, ohi = nlev ? 0u : ovf_hi;
   const PgsRows S(d, base);
-  const bool usual = s.accum && s.friction;
+  const uint32_t flags = W.flags & kPgsUsual;
   const uint32_t quad_rows = T::kGlobalScalars ? NT / 4u : d.pgs_quad_rows;
-  auto sweep_in = [&](auto warm, auto vc, bool use_bias) __attribute__((always_inline)) {
+  auto sweep_in = [&](auto form, auto warm, auto vc, bool use_bias) __attribute__((always_inline)) {
+    constexpr uint32_t kFlags = decltype(form)::value;
+    pgs_sweep<kPlain, decltype(warm)::value, kFlags>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
+  };
+  // Flags other than the usual ones: one instance for each, whatever the body
+  // rows' place, so that no contact tests them (tested per contact, 1,024
+  // worlds without friction swept 3.45 ms a step instead of 2.23, without
+  // accumulation 4.77 instead of 2.82).  The dependency levels of the
+  // per-island path are mostly shorter than a wave of quads and take quads
+  // only, with the flags tested: there single lanes for the long ones cost
+  // every form registers (usual flags 13.8 -> 14.4 ms, no friction 9.8 ->
+  // 11.1).
+  auto sweep_other = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
     constexpr bool kWarm = decltype(warm)::value;
-    if (usual) pgs_sweep<kPlain, kWarm, true>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
-    else pgs_sweep<kPlain, kWarm, false>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
+    if constexpr (kIsland) {
+      if (kWarm && !s.accum) return;
+      if constexpr (T::kGlobalScalars) sweep_in(PgsForm<kPgsAny>{}, warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
+      else if (ncache == N) sweep_in(PgsForm<kPgsAny>{}, warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
+      else sweep_in(PgsForm<kPgsAny>{}, warm, cache, use_bias);
+    } else {
+      const PgsLds<T::kGlobalScalars ? kMemHbm : kMemBoth> vc{pgs_lds, off, ncache};
+      if (flags == BB_SIM_ACCUM_IMPULSE) sweep_in(PgsForm<BB_SIM_ACCUM_IMPULSE>{}, warm, vc, use_bias);
+      if constexpr (!kWarm) {
+        if (flags == BB_SIM_FRICTION) sweep_in(PgsForm<BB_SIM_FRICTION>{}, warm, vc, use_bias);
+        if (flags == 0u) sweep_in(PgsForm<0u>{}, warm, vc, use_bias);
+      }
+    }
   };
   auto sweep = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
-    if constexpr (T::kGlobalScalars) {  // teams keep no rows in LDS
-      sweep_in(warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
+    if (flags != kPgsUsual) {
+      sweep_other(warm, use_bias);
+    } else if constexpr (T::kGlobalScalars) {  // teams keep no rows in LDS
+      sweep_in(PgsForm<kPgsUsual>{}, warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
     } else if (ncache == N) {
-      sweep_in(warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
+      sweep_in(PgsForm<kPgsUsual>{}, warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
     } else {
-      sweep_in(warm, cache, use_bias);
+      sweep_in(PgsForm<kPgsUsual>{}, warm, cache, use_bias);
     }
   };
   sweep(std::true_type{}, false);

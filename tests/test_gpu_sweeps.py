@@ -2,7 +2,7 @@
 places their body rows can lie (all in LDS, some, none) give the oracle's
 bits: sizes around a wave of quads, a workgroup of quads and a second round,
 the flags that change the contact's arithmetic, manifolds of more than four
-contacts and the serial bucket's rows included."""
+contacts and the rows past the last colour, which are solved in turn."""
 from __future__ import annotations
 
 import numpy as np
@@ -58,6 +58,38 @@ def test_sweep_forms_equal_oracle(pgs_block, lds, quads):
             g, r = b.read_world(w, n), o.read_bodies()
             for f in FIELDS:
                 assert np.array_equal(g[f], r[f]), (w, n, f)
+
+
+@pytest.mark.parametrize("worlds,lds", [(4, 512), (300, 0), (300, 100)])
+def test_rows_past_the_colours_equal_oracle(worlds, lds):
+    """Spheres closer than their radius need more colours than there are, with
+    each of the flags, in a lone launch and in a crowded one."""
+    b = beatbox.Batch()
+    b.set_param(beatbox.PARAM_BLOCK, 256)
+    b.set_param(beatbox.PARAM_PAIR_SCALE, 8)
+    b.set_param(beatbox.PARAM_LANE_BODIES, 0)
+    b.set_param(beatbox.PARAM_PGS_LDS_ROWS, lds)
+    bodies = scenes.dense_spheres(0xBB92, side=6)
+    oracles = []
+    for flags in _flags():
+        d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=3, flags=flags, morton_bits=63, quirks=0,
+                                                       gravity=0.0))
+        b.add_world(d, bodies)
+        o = OracleWorld(d)
+        o.add_bodies(bodies)
+        oracles.append(o)
+    tiny = beatbox.WorldDesc.make(**scenes.world_desc(iterations=2, morton_bits=63, quirks=0))
+    for k in range(worlds - len(oracles)):
+        b.add_world(tiny, scenes.random_boxes(5000 + k, 2, extent=0.6, y0=0.55, y1=1.5))
+    for step in range(2):
+        b.step(1)
+        b.sync()
+        for w, o in enumerate(oracles):
+            o.step(1)
+            assert step or o.stats()["graph_color_overflow"] > 0
+            g, r = b.read_world(w, len(bodies)), o.read_bodies()
+            for f in FIELDS:
+                assert np.array_equal(g[f], r[f]), (step, w, f)
 
 
 def _plate(n: int):
