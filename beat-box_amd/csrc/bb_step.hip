@@ -1140,21 +1140,32 @@ struct BroadShared {
 // at a time by a wave, which finds the same pairs (an inner node's box is the
 // exact union of its leaves', so a leaf that overlaps is always reached) and
 // finds them in ascending order.  A walk is a chain of node visits of about
-// 1,000 cycles each, up to the budget of 128; the flat form is N^2 / 128 wave
-// tests of about 14 instructions, spread over the team's waves.  The line
-// lies where those take about 17 us (a walk at its budget takes 55); with more
-// worlds than CUs at a fifth of that, since there the instructions count and
-// not the chain (4,096 worlds' wide lane: 533 us with the trees alone, 508 so,
-// 616 with the first line and a wave less per SIMD).  Measured: 49 bodies 51 -> 23 us; 1,001 bodies 144 -> 41 us and
-// 1,501 bodies 290 -> 76 us with 16 workgroups.
+// 1,000 cycles each, up to the budget of 128 (less in a world of stacks, whose
+// rows have few partners, than in a pile); the flat form is N^2 / 128 wave
+// tests of about 14 instructions, spread over the team's waves.  The lines,
+// with the broad phase's times for stacks | piles, flat against tree:
+//  - several workgroups per world (three launches): N^2 = 40,960 per wave.
+//    32 worlds of 1,000 rows (31,250): 139 | 139 us against 184 | 191; eight
+//    of 1,500 (35,156): 140 | 139 against 182 | 208; 32 of 1,200 (45,000):
+//    195 | 224 against 123 | 193;
+//  - one workgroup per world, whose waves share a CU's issue slots: 16,384
+//    per wave.  200 worlds of 127 rows (4,032): 60 | 61 against 78 | 160; of
+//    255 (16,256): 120 | 122 against 110 | 167; of 400 (40,000): 241 | 247
+//    against 142 | 207;
+//  - and N^2 = 10 million over the launch, since with several worlds on a
+//    CU the instructions count and not the chain.  1,024 worlds of 63 rows
+//    (4.1 million): 51 | 51 against 55 | 106; of 127 (16.5 million): 94 | 95
+//    against 90 | 197; 4,096 worlds of 31 (3.9 million): 89 against 105; of
+//    63 (16.3 million): 168 against 102 (stacks).
 // Not with a NaN box in the world: it reaches the root through the ordered
 // min / max, and the walks then end where it does.
-static constexpr uint32_t kFlatPerWave = 40960, kFlatCrowded = 8192;
+static constexpr uint32_t kFlatPerWave = 40960, kFlatPerWaveOne = 16384, kFlatLaunch = 10000000;
 template <class T>
 BB_DI bool broad_flat(const Dev& d, uint32_t nb, uint32_t N, const T& t) {
   if constexpr (T::kGlobalScalars) return false;  // worlds this large keep the tree
-  const uint32_t per = gridDim.x > kCus ? kFlatCrowded : kFlatPerWave;
-  if (N < 2u || (uint64_t)N * N > (uint64_t)per * (t.size() / WAVE)) return false;
+  const uint64_t n2 = (uint64_t)N * N;
+  if (N < 2u || n2 > (uint64_t)(T::kSpread ? kFlatPerWave : kFlatPerWaveOne) * (t.size() / WAVE)) return false;
+  if (!T::kSpread && gridDim.x > kCus && n2 * gridDim.x > kFlatLaunch) return false;
   const float4 a = d.nmin[nb], b = d.nmax[nb];
   return a.x == a.x && a.y == a.y && a.z == a.z && b.x == b.x && b.y == b.y && b.z == b.z;
 }
@@ -1451,7 +1462,8 @@ BB_DI void s_broad(const Dev& d, uint32_t w, const T& t, BroadShared& L, WalkLds
 }
 
 // Eight waves per SIMD, which hide the walks' loads in a crowded launch (with
-// both forms the compiler would take 67 registers, which leaves seven).
+// both forms the compiler would take 67 registers, which leaves seven: 616
+// against 508 us in the wide lane of 4,096 worlds).
 template <int BLOCK>
 __global__ __launch_bounds__(BLOCK, 8) void k_broad(Dev d) {
   __shared__ BroadShared L;

@@ -1,9 +1,10 @@
 """The broad phase over every pair of rows (small worlds) and by several
 workgroups in three launches, and the narrow phase by several workgroups per
 world, give the oracle's bits: sizes around a wave, around the lines where
-the tree takes over (N^2 = 40,960 or, with more worlds than CUs, 8,192 per
-wave) and around the smallest world of the three launches, voxel worlds with
-their expanded slots, and a row of more partners than the tree form stages."""
+the tree takes over (N^2 = 40,960 per wave in three launches, 16,384 in one,
+10 million over a launch of more worlds than CUs) and around the smallest world of
+the three launches, voxel worlds with their expanded slots, and a row of more
+partners than the tree form stages."""
 from __future__ import annotations
 
 import numpy as np
@@ -49,7 +50,8 @@ def _worlds(b, sizes, seed):
 @pytest.mark.parametrize("block,worlds,sizes", [
     (256, 1, (2,)), (256, 1, (65,)), (256, 1, (256,)), (256, 1, (257,)), (256, 1, (1619,)), (256, 1, (1620,)),
     (512, 1, (1025,)), (1024, 1, (700,)), (128, 20, (63, 64, 300)),
-    (256, 100, (128, 404, 405)), (512, 100, (572, 573)), (256, 300, (180, 181, 182, 404, 600))])
+    (256, 100, (128, 404, 405)), (512, 100, (572, 573)), (256, 300, (180, 181, 182, 404, 600)),
+    (256, 200, (256, 257)), (256, 300, (182, 183)), (128, 1024, (98, 99))])
 def test_broad_and_narrow_spread_equal_oracle(block, worlds, sizes):
     b = beatbox.Batch()
     b.set_param(beatbox.PARAM_BLOCK, block)
