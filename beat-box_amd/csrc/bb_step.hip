@@ -4270,7 +4270,6 @@ BB_DI void av_dual(const Dev& d, const WorldInfo& W, const AvData& D, uint32_t s
   const v3 th1 = ld3(D.dth[(uint32_t)h.x * 3u]), th2 = ld3(D.dth[(uint32_t)h.y * 3u]);
   const v3 x1 = ld3(d.s_pos0[off + h.x]), x2 = ld3(d.s_pos0[off + h.y]);
   const bool d1 = p1.w != 0.0f, d2 = p2.w != 0.0f;
-  if (!d1 && !d2) return;
   const v3 v1 = ld3(p1) + cross(th1, c.p - x1), v2 = ld3(p2) + cross(th2, c.p - x2);
   const v3 u1 = ld3(p1) + cross(th1, c.ar1), u2 = ld3(p2) + cross(th2, c.ar2);
   float4 lm = c.lm, cm = c.cm;
@@ -4430,34 +4429,40 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     D.dp[i * 3u] = st3(pn - p, 1.0f);
     D.dth[i * 3u] = st3(small_angle_delta(qtl, q), 0.0f);
   }
-  // contacts per row, and the lists of contacts (per row in ascending
-  // manifold order, and of the whole world)
+  // contacts per moving row and per manifold between rows of which one moves
+  // (hdr.z), and the lists of them (per row in ascending manifold order, and
+  // of the whole world): the sweeps of a world that sleeps have none (4,096
+  // settled worlds of 16 to 128 bodies: 409 -> 333 us)
+  auto moves = [&](uint32_t row) {
+    const uint32_t fl = d.cur.flags[off + row];
+    return (fl & BB_BODY_DYNAMIC) && !(fl & BB_BODY_SLEEPING);
+  };
   for (uint32_t i = tid; i < N; i += NT) {
     const uint32_t g = off + i;
     uint32_t c = 0;
-    if (d.cur.flags[g] & BB_BODY_DYNAMIC) {
+    if (moves(i)) {
       const uint32_t* l = adj + d.adj_off[g];
       for (uint32_t e = 0; e < d.deg[g]; ++e) c += (uint32_t)d.man_cur.hdr[l[e]].w;
     }
     d.pcount[g] = c;
+  }
+  for (uint32_t p = tid; p < P; p += NT) {
+    const int4 h = d.man_cur.hdr[W.pair_off + p];
+    D.hdr[p].z = h.w > 0 && (moves((uint32_t)h.x) || moves((uint32_t)h.y)) ? h.w : 0;
   }
   t.sync();
   const uint32_t items = scan_range(t, N, [&](uint32_t i) { return d.pcount[off + i]; },
                                     [&](uint32_t i, uint32_t ex) { d.poff[off + i] = ex; });
   const bool partners = items <= D.cap8;
   const uint32_t contacts = scan_range(
-      t, P,
-      [&](uint32_t p) {
-        const int c = d.man_cur.hdr[W.pair_off + p].w;
-        return c > 0 ? (uint32_t)c : 0u;
-      },
+      t, P, [&](uint32_t p) { return (uint32_t)D.hdr[p].z; },
       [&](uint32_t p, uint32_t ex) {
-        const int c = d.man_cur.hdr[W.pair_off + p].w;
+        const int c = D.hdr[p].z;
         for (int j = 0; j < c; ++j) D.all[ex + (uint32_t)j] = p * 8u + (uint32_t)j;
       });
   for (uint32_t i = tid; i < N; i += NT) {
     const uint32_t g = off + i;
-    if (!(d.cur.flags[g] & BB_BODY_DYNAMIC)) continue;
+    if (!moves(i)) continue;
     const uint32_t* l = adj + d.adj_off[g];
     uint32_t x = d.poff[g];
     for (uint32_t e = 0; e < d.deg[g]; ++e) {
@@ -4485,7 +4490,8 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
       const qt q1c = qconj(q1), q2c = qconj(q2);
       const float f1 = d.props.mass[off + d.cur.id[ga]].z, f2 = d.props.mass[off + d.cur.id[gb]].z;
       const float mu = __builtin_sqrtf(fmx(f1, 0.0f) * fmx(f2, 0.0f));
-      D.hdr[p] = make_int4(h.x, h.y, h.w, __float_as_int(mu));
+      const bool swept = D.hdr[p].z != 0;
+      D.hdr[p] = make_int4(h.x, h.y, D.hdr[p].z, __float_as_int(mu));
       const v3 t0 = ld3(d.man_cur.t0[slot]), t1 = ld3(d.man_cur.t1[slot]);
       for (int j = 0; j < h.w; ++j) {
         const uint32_t cs = slot * 8 + j;
@@ -4520,6 +4526,7 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
         d.man_cur.cmas[cs] = cmv;
         d.man_cur.cana[cs] = ca;
         d.man_cur.canb[cs] = cb;
+        if (!swept) continue;
         const v3 ar1 = avbd_q_rotate(q1, ld3(ca)), ar2 = avbd_q_rotate(q2, ld3(cb));
         const v3 gap = (x2 + ar2) - (x1 + ar1);
         const size_t at = D.at(p, (uint32_t)j);

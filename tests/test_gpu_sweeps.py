@@ -141,3 +141,34 @@ def test_avbd_groups_equal_oracle(block, team, fused):
             g, r = b.read_world(w, n), o.read_bodies()
             for f in FIELDS:
                 assert np.array_equal(g[f], r[f]), (w, n, f)
+
+
+@pytest.mark.parametrize("team", [0, 9])
+def test_avbd_sleeping_worlds_equal_oracle(team):
+    """Worlds that fall asleep, wholly or but for a box that drops among the
+    sleepers: manifolds between rows that do not move take no part in the
+    sweeps."""
+    b = beatbox.Batch()
+    b.set_param(beatbox.PARAM_BLOCK, 256)
+    b.set_param(beatbox.PARAM_TEAM_BODIES, team)
+    b.set_param(beatbox.PARAM_LANE_BODIES, 0)
+    d = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10, morton_bits=63, quirks=0))
+    oracles, asleep = [], [0, 0]
+    for late in (False, True):
+        bodies = scenes.random_boxes(61, 12, extent=1.5, y0=0.55, y1=2.0)
+        if late:
+            bodies[-1]["position"] = (0.1, 16.0, 0.2)
+        b.add_world(d, bodies)
+        o = OracleWorld(d)
+        o.add_bodies(bodies)
+        oracles.append((o, len(bodies)))
+    for _ in range(24):
+        b.step(10)
+        b.sync()
+        for w, (o, n) in enumerate(oracles):
+            o.step(10)
+            g, r = b.read_world(w, n), o.read_bodies()
+            for f in FIELDS:
+                assert np.array_equal(g[f], r[f]), (w, f)
+            asleep[w] = max(asleep[w], o.stats()["sleeping_count"])
+    assert min(asleep) > 0, asleep
