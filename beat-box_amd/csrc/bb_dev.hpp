@@ -231,7 +231,7 @@ struct Dev {
   uint32_t pgs_quads;     // 1: sweep by quads of lanes whenever the workgroup has enough
   uint32_t pgs_quad_rows; // ranges of at most this many rows are swept by quads of lanes, longer ones by lanes
   uint32_t lane_max;      // bodies of the launch's largest world (0: not told)
-  uint32_t spread;        // workgroups per world of the broad and narrow phase: the least (1), set per launch
+  uint32_t spread;        // workgroups per world of the broad and narrow phase, set per launch
   uint32_t walk_budget;   // nodes a broad-phase thread walks before its workgroup takes the row
                           // (0: kWalkBudgetDefault)
   // set (bit 0) by any world whose step flags an overflow; the host reads

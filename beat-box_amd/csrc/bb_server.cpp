@@ -4,9 +4,11 @@
 // active and pair capacities that the HBM budget holds.  A world occupies one
 // slot and one contiguous range in each arena (first fit); the kernels find
 // it through its slot's WorldInfo, so admitting or retiring a world only
-// rewrites its table entry and its ranges.  Empty slots have n = 0 and their
-// workgroups return at once, so a step launch (one hipGraph per parity over a
-// slot range) never changes shape.
+// rewrites its table entry and its ranges.  A pool's order of slots puts the
+// resident worlds first; a step launches workgroups for them, their number
+// rounded up to a power of two (one hipGraph per parity and launch size, made
+// when first needed).  Empty slots among them have n = 0 and their workgroups
+// return at once.
 //
 // Pools: the slots are split into up to three pools by world size (small
 // worlds, one workgroup each; mid-sized worlds, one larger workgroup each;
@@ -184,7 +186,7 @@ struct Pool {
   std::vector<uint32_t> free_slots;
   std::deque<StepRecord> inflight;
   Chunk chunks[kChunks];
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  std::map<uint32_t, hipGraphExec_t> graph[2];  // by launch size
   int latest = 1;  // parity holding the newest rows of this pool's worlds
   uint64_t step_counter = 0;
   bool table_dirty = false;
@@ -337,31 +339,44 @@ bb_status finish_oldest(bb_server* s, uint32_t p) {
   return BB_OK;
 }
 
-// The step graphs of pool p (one per parity): k_team first when the pool has
-// teams, then the per-world stage kernels over its slots in its order.
-bb_status ensure_graphs(bb_server* s, uint32_t p) {
+// Workgroups of pool p's next step: its worlds that no team steps, rounded up
+// to a power of two.  The launch chooses its form from it (several workgroups
+// per world, wider ones, sweeps by quads), so it has to be what is resident
+// and not what there is room for: 64 requests of 64 to 20,000 bodies through
+// pools of 4,096 slots took 872 ms when the launches had a workgroup for every
+// slot, and take 688 so.
+uint32_t launch_size(const bb_server* s, const Pool& P) {
+  uint32_t n = 0, g = 1;
+  for (uint32_t w = P.w0; w < P.w1; ++w) {
+    const WorldInfo& wi = s->b->infos[w];
+    if (wi.n && !(wi.mode & kModeTeam)) ++n;
+  }
+  while (g < n) g *= 2;
+  return std::min(g, P.w1 - P.w0);
+}
+
+// The step graph of pool p for a parity and a launch size: k_team first when
+// the pool has teams, then the per-world stage kernels over the first slots
+// of its order.
+bb_status step_graph(bb_server* s, uint32_t p, int par, uint32_t grid, hipGraphExec_t* out) {
   Pool& P = s->pools[p];
-  for (int par = 0; par < 2; ++par) {
-    if (P.graph[par]) continue;
+  hipGraphExec_t& exec = P.graph[par][grid];
+  if (!exec) {
     hipGraph_t g;
     HIPCHK(hipStreamBeginCapture(P.stream, hipStreamCaptureModeThreadLocal));
     Dev d = dev_for(s->b, par);
     d.order = d.order + P.w0;
     d.pgs_lcap = P.lcap;
-    // the pools past the first hold worlds of hundreds of bodies in few of
-    // their slots: several workgroups for each world's broad and narrow phase
-    if (p) {
-      d.lane_max = kMAX;
-      d.spread = 4u;
-    }
+    if (p) d.lane_max = kMAX;  // the pools past the first hold worlds of hundreds of bodies
     if (!P.teams) d.team_grid = 0;
     // with voxel shapes registered any team may hold voxel bodies
     d.team_vox = s->b->vox_shapes.empty() ? 0u : 1u;
-    launch_step(Lane{d, P.block, P.w1 - P.w0}, P.stream, true);
+    launch_step(Lane{d, P.block, grid}, P.stream, true);
     HIPCHK(hipStreamEndCapture(P.stream, &g));
-    HIPCHK(hipGraphInstantiate(&P.graph[par], g, nullptr, nullptr, 0));
+    HIPCHK(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0));
     HIPCHK(hipGraphDestroy(g));
   }
+  *out = exec;
   return BB_OK;
 }
 
@@ -535,11 +550,12 @@ bb_status pool_step(bb_server* s, uint32_t p) {
     HIPCHK(hipEventRecord(s->first, stream));
     s->started = true;
   }
-  // ---- the step: every slot of the pool, one launch sequence
-  st = ensure_graphs(s, p);
-  if (st != BB_OK) return st;
+  // ---- the step: the pool's resident worlds, one launch sequence
   const int cur = P.latest ^ 1;
-  HIPCHK(hipGraphLaunch(P.graph[cur], stream));
+  hipGraphExec_t graph = nullptr;
+  st = step_graph(s, p, cur, launch_size(s, P), &graph);
+  if (st != BB_OK) return st;
+  HIPCHK(hipGraphLaunch(graph, stream));
   P.latest = cur;
   // ---- per-world bookkeeping; read-back and release of finished worlds
   for (uint32_t w = P.w0; w < P.w1; ++w) {
@@ -808,11 +824,11 @@ static bb_status shapes_changed(bb_server* s) {
     }
   for (Pool& P : s->pools) {
     HIPCHK(hipStreamSynchronize(P.stream));
-    for (hipGraphExec_t& g : P.graph)
-      if (g) {
-        HIPCHK(hipGraphExecDestroy(g));
-        g = nullptr;
-      }
+    for (auto& m : P.graph) {
+      for (auto& g : m)
+        if (g.second) HIPCHK(hipGraphExecDestroy(g.second));
+      m.clear();
+    }
   }
   bb_batch* b = s->b;
   bb_status st = upload_voxels(b);
@@ -1226,8 +1242,9 @@ void bb_server_destroy(bb_server* s) {
   for (Pool& P : s->pools)
     if (P.stream) (void)hipStreamSynchronize(P.stream);
   for (Pool& P : s->pools) {
-    for (auto& g : P.graph)
-      if (g) (void)hipGraphExecDestroy(g);
+    for (auto& m : P.graph)
+      for (auto& g : m)
+        if (g.second) (void)hipGraphExecDestroy(g.second);
     for (auto& rec : P.inflight) {
       if (rec.done) (void)hipEventDestroy(rec.done);
       if (rec.admit) (void)hipEventDestroy(rec.admit);

@@ -5119,15 +5119,13 @@ Dev sweep_form(const Dev& d, uint32_t grid) {
 // A launch of few worlds leaves CUs idle, and the narrow phase's pairs and the
 // broad phase's rows need no workgroup of their own: up to kMaxSpread
 // workgroups per world, as far as the chip has CUs for them (one 1,501-body
-// world: narrow 147 -> 28, contacts 200 -> 45 us), or as many as the caller
-// asks for (d.spread: most slots of a serving pool are empty, and a workgroup
-// that finds none of its own ends at once).  The broad phase pays two more
-// launches for it, about 6 us, so it takes kMinBroadSpread workgroups and
+// world: narrow 147 -> 28, contacts 200 -> 45 us).  The broad phase pays two
+// more launches for it, about 6 us, so it takes kMinBroadSpread workgroups and
 // worlds of more than kMinBroadRows bodies (1,001 bodies: 144 -> 41 us; a
 // world of 49 is through in 23 us with one).
 static Dev spread_form(const Dev& d, uint32_t grid) {
   Dev r = d;
-  r.spread = std::max(std::max(1u, d.spread), std::min(kMaxSpread, kCus / grid));
+  r.spread = std::max(1u, std::min(kMaxSpread, kCus / grid));
   return r;
 }
 // Stages of the per-world path, in launch order (k_team, when there is one,

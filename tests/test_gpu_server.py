@@ -218,3 +218,33 @@ def test_server_voxel_requests_equal_alone_and_checkpoint():
         assert server.report()["reruns"] == 0
     srv.destroy()
     restored.destroy()
+
+
+def test_launches_follow_the_resident_worlds():
+    """Pools with more slots than worlds: as worlds retire the launches shrink
+    from more workgroups than CUs (512-thread AVBD groups, one workgroup per
+    world) to a few (1,024-thread groups, several workgroups per world), and
+    every checked world ends as it does alone."""
+    avbd = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10,
+                                                      morton_bits=63, quirks=0))
+    pgs = beatbox.WorldDesc.make(**scenes.world_desc(iterations=4, morton_bits=63, quirks=0))
+    srv = beatbox.Server(budget_bytes=4 << 30, max_worlds=700, split_bodies=64, team_bodies=2000)
+    checked = []
+    for k in range(300):  # all in the second pool
+        n = 64 + k % 23 if k % 50 else 257 + k
+        steps = 2 + k // 25
+        bodies = scenes.serving_pile(3000 + k, n)
+        t = srv.submit(avbd if k % 2 == 0 else pgs, bodies, steps)
+        if k % 25 == 0 or k == 299:
+            checked.append((t, avbd if k % 2 == 0 else pgs, bodies, steps))
+    srv.step(1)
+    assert srv.report()["resident_worlds"] == 300
+    srv.drain()
+    assert srv.report()["retired"] == 300
+    for t, d, bodies, steps in checked:
+        state, got, _ = srv.poll(t, len(bodies))
+        assert state == beatbox.REQ_DONE
+        ref, _ = _alone(d, bodies, steps)
+        for f in FIELDS:
+            assert got[f].tobytes() == ref[f].tobytes(), (t, f)
+    srv.destroy()
