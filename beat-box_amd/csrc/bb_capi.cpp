@@ -523,7 +523,7 @@ bb_status build(bb_batch* b) {
   b->base.any_voxel = 0;
   for (auto& hw : b->worlds)
     if (hw.has_voxel) b->base.any_voxel = 1;
-  b->base.any_island = any_island(b);
+  b->base.paths = solver_paths(b);
   b->built = true;
   b->dirty = false;
   b->stepped = false;
@@ -582,7 +582,7 @@ bb_status grow_pairs(bb_batch* b) {
   b->buf = std::move(nb);
   b->base.pgs_lcap = base0.pgs_lcap;
   b->base.any_voxel = base0.any_voxel;
-  b->base.any_island = base0.any_island;
+  b->base.paths = base0.paths;
   b->base.team_grid = base0.team_grid;
   b->base.team_vox = base0.team_vox;
   b->vox_dirty = false;  // the pools came over with the rest
@@ -717,12 +717,15 @@ bb_status upload_infos(bb_batch* b, bool one_shot) {
   return BB_OK;
 }
 
-// Whether any world runs the per-island solver path (k_levels and
-// k_pgs_island are then part of the launch sequence).
-uint32_t any_island(const bb_batch* b) {
-  for (const WorldInfo& wi : b->infos)
-    if (wi.solver != BB_SOLVER_AVBD && !(wi.flags & BB_SIM_USE_GRAPH_COLORING)) return 1u;
-  return 0u;
+uint32_t solver_paths(const bb_batch* b) {
+  constexpr uint32_t kUsual = BB_SIM_ACCUM_IMPULSE | BB_SIM_FRICTION;
+  uint32_t paths = 0u;
+  for (const WorldInfo& wi : b->infos) {
+    if (wi.solver == BB_SOLVER_AVBD) continue;
+    if (!(wi.flags & BB_SIM_USE_GRAPH_COLORING)) paths |= kPathIsland;
+    else paths |= (wi.flags & kUsual) == kUsual ? kPathUsual : kPathFlags;
+  }
+  return paths;
 }
 
 bb_status refresh_infos(bb_batch* b) {
@@ -731,11 +734,11 @@ bb_status refresh_infos(bb_batch* b) {
     wi.mode = b->infos[w].mode;
     b->infos[w] = wi;
   }
-  // a solver or flag change can add or drop the per-island kernels: a
-  // captured step graph holds the old launch sequence
-  const uint32_t p = any_island(b);
-  if (p != b->base.any_island) {
-    b->base.any_island = p;
+  // a solver or flag change can add or drop a path's kernels: a captured step
+  // graph holds the old launch sequence
+  const uint32_t p = solver_paths(b);
+  if (p != b->base.paths) {
+    b->base.paths = p;
     if (b->graph) {
       (void)hipGraphExecDestroy(b->graph);
       b->graph = nullptr;

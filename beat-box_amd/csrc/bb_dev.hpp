@@ -144,13 +144,18 @@ struct Manifolds {  // pair-indexed slots; contact arrays are [slot*8 + c]
   uint32_t* cws; // warm start counter
 };
 
+// Dev::paths: the per-island path (k_levels and k_pgs_island are launched);
+// colour sweeps without friction or accumulation (k_pgs_flags); colour sweeps
+// with both (k_pgs)
+enum : uint32_t { kPathIsland = 1u, kPathFlags = 2u, kPathUsual = 4u };
+
 struct Dev {
   WorldInfo* worlds;
   uint32_t W;
   // voxel shape pools, shared by the batch's worlds; any_voxel: a world has
-  // voxel bodies (k_narrow_vox is launched); any_island: a world runs the
-  // per-island solver path (k_levels and k_pgs_island are launched)
-  uint32_t any_voxel, any_island;
+  // voxel bodies (k_narrow_vox is launched); paths: the PGS paths that a world
+  // runs (kPath*)
+  uint32_t any_voxel, paths;
   const VoxShape* vshape;
   const uint32_t* vocc;
   const uint32_t* vsurf;

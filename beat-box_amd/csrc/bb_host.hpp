@@ -252,8 +252,8 @@ uint32_t assign_teams(bb_batch* b, uint32_t grid_cap);
 // (ties by index), team worlds last (their workgroups exit at once).
 void world_order(const std::vector<WorldInfo>& infos, uint32_t* out);
 Dev dev_for(const bb_batch* b, int cur);
-// 1 when a world of the batch runs the per-island solver path.
-uint32_t any_island(const bb_batch* b);
+// The PGS paths that a world of the batch runs (kPath*).
+uint32_t solver_paths(const bb_batch* b);
 // One step of every world of a built batch on b->stream (flips the parity).
 bb_status launch_one(bb_batch* b);
 // Bodies of world w (n >= its body count) in `order`, after b->stream drains.

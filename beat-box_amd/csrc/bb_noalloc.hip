@@ -127,7 +127,7 @@ bb_status step_noalloc(const bb_world_desc* desc, const bb_body_desc* bodies, ui
   b.latest = 1;  // the first step reads set 1 and writes set 0
   b.base.pgs_lcap = pgs_lds_rows(&b);
   b.base.any_voxel = 0;
-  b.base.any_island = any_island(&b);
+  b.base.paths = solver_paths(&b);
   b.base.team_grid = 0;
   b.built = true;
   b.dirty = false;

@@ -3628,10 +3628,7 @@ BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc
       wb = wb + mulmv(Ib, cross(r2, P));
     }
   };
-  PgsContact x = R.c0;
-  for (int c = 0; c < count; ++c) {
-    // (the last contact fetches itself again)
-    const PgsContact next = pgs_contact(S, k, c + 1 < count ? c + 1 : c);
+  auto contact = [&](int c, const PgsContact& x) __attribute__((always_inline)) {
     const v3 r1 = ld3(x.cp) - pa, r2 = ld3(x.cp) - pb;
     v3 l = x.l;
     if constexpr (kWarm) {
@@ -3684,7 +3681,26 @@ BB_DI void pgs_solve_lane(const Dev& d, const PgsRows& S, const PgsLds<kMem>& vc
       apply(n * imp, r1, r2);
       reinterpret_cast<v3*>(S.l_at(c))[k] = l;
     }
-    x = next;
+  };
+  if constexpr (friction) {
+    PgsContact x = R.c0;
+    for (int c = 0; c < count; ++c) {
+      // (the last contact fetches itself again)
+      const PgsContact next = pgs_contact(S, k, c + 1 < count ? c + 1 : c);
+      contact(c, x);
+      x = next;
+    }
+  } else {
+    // a contact is a third of the instructions and does not cover the next
+    // one's loads: the first ones together (in bounds whatever the count)
+    PgsContact x[kPgsPre];
+    x[0] = R.c0;
+#pragma unroll
+    for (int c = 1; c < kPgsPre; ++c) x[c] = pgs_contact(S, k, c);
+#pragma unroll
+    for (int c = 0; c < kPgsPre; ++c)
+      if (c < count) contact(c, x[c]);
+    for (int c = kPgsPre; c < count; ++c) contact(c, pgs_contact(S, k, c));
   }
   if (da) vc.store_lane(d, (uint32_t)h.x, va, wa);
   if (db) vc.store_lane(d, (uint32_t)h.y, vb, wb);
@@ -3771,14 +3787,18 @@ BB_DI qt apply_angular_velocity(qt q, v3 om, float dt) {
 
 // kIsland: the instances for the per-island path (k_pgs_island), which
 // sweep dependency levels; kPlain: PGS (per-island path only) rather than
-// PGS_SOFT.  k_pgs, the colour sweeps, carries neither.
-template <bool kIsland, bool kPlain, class T>
+// PGS_SOFT.  k_pgs, the colour sweeps, carries neither.  kOnly: the flags of
+// the worlds that the instance steps (kPgsAll: any).
+static constexpr uint32_t kPgsAll = 0xFFFFFFFFu;
+template <bool kIsland, bool kPlain, uint32_t kOnly = kPgsAll, class T>
 BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t lcap) {
   const uint32_t tid = t.rank(), NT = t.size();
   const WorldInfo W = d.worlds[w];
   if (W.solver == BB_SOLVER_AVBD || W.n == 0) return;
   if (((W.flags & BB_SIM_USE_GRAPH_COLORING) == 0) != kIsland) return;
   if ((W.solver == BB_SOLVER_PGS) != kPlain) return;
+  const uint32_t flags = W.flags & kPgsUsual;
+  if (kOnly != kPgsAll && flags != kOnly) return;
   const uint32_t off = W.body_off, N = W.n, A = W.a, NP = d.np;
   Pgs s;
   s.accum = (W.flags & BB_SIM_ACCUM_IMPULSE) != 0;
@@ -3811,27 +3831,34 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t 
   const uint32_t nr = nlev ? nlev : used;
   const uint32_t olo = nlev ? 0u : ovf_lo, ohi = nlev ? 0u : ovf_hi;
   const PgsRows S(d, base);
-  const uint32_t flags = W.flags & kPgsUsual;
   const uint32_t quad_rows = T::kGlobalScalars ? NT / 4u : d.pgs_quad_rows;
   auto sweep_in = [&](auto form, auto warm, auto vc, bool use_bias) __attribute__((always_inline)) {
     constexpr uint32_t kFlags = decltype(form)::value;
     pgs_sweep<kPlain, decltype(warm)::value, kFlags>(d, t, vc, s, S, ro, nr, olo, ohi, use_bias, quad_rows);
   };
-  // Flags other than the usual ones: one instance for each, whatever the body
-  // rows' place, so that no contact tests them (tested per contact, 1,024
-  // worlds without friction swept 3.45 ms a step instead of 2.23, without
-  // accumulation 4.77 instead of 2.82).  The dependency levels of the
-  // per-island path are mostly shorter than a wave of quads and take quads
-  // only, with the flags tested: there single lanes for the long ones cost
-  // every form registers (usual flags 13.8 -> 14.4 ms, no friction 9.8 ->
-  // 11.1).
+  auto sweep_form = [&](auto form, auto warm, bool use_bias) __attribute__((always_inline)) {
+    if constexpr (T::kGlobalScalars) {  // teams keep no rows in LDS
+      sweep_in(form, warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
+    } else if (ncache == N) {
+      sweep_in(form, warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
+    } else {
+      sweep_in(form, warm, cache, use_bias);
+    }
+  };
+  // No contact tests the flags: tested per contact, 1,024 worlds without
+  // friction swept 3.45 ms a step instead of 2.22, without accumulation 4.77
+  // instead of 2.92.  The stage kernels have an instance per set of flags;
+  // teams and the one-launch step, which hold all stages, one sweep for each
+  // set but the usual one, whatever the body rows' place.  The dependency
+  // levels of the per-island path are mostly shorter than a wave of quads and
+  // take quads only, with the flags tested: there single lanes for the long
+  // ones cost every form registers (usual flags 13.8 -> 14.4 ms, no friction
+  // 9.8 -> 11.1).
   auto sweep_other = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
     constexpr bool kWarm = decltype(warm)::value;
     if constexpr (kIsland) {
       if (kWarm && !s.accum) return;
-      if constexpr (T::kGlobalScalars) sweep_in(PgsForm<kPgsAny>{}, warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
-      else if (ncache == N) sweep_in(PgsForm<kPgsAny>{}, warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
-      else sweep_in(PgsForm<kPgsAny>{}, warm, cache, use_bias);
+      sweep_form(PgsForm<kPgsAny>{}, warm, use_bias);
     } else {
       const PgsLds<T::kGlobalScalars ? kMemHbm : kMemBoth> vc{pgs_lds, off, ncache};
       if (flags == BB_SIM_ACCUM_IMPULSE) sweep_in(PgsForm<BB_SIM_ACCUM_IMPULSE>{}, warm, vc, use_bias);
@@ -3842,14 +3869,12 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t 
     }
   };
   auto sweep = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
-    if (flags != kPgsUsual) {
-      sweep_other(warm, use_bias);
-    } else if constexpr (T::kGlobalScalars) {  // teams keep no rows in LDS
-      sweep_in(PgsForm<kPgsUsual>{}, warm, PgsLds<kMemHbm>{pgs_lds, off, 0u}, use_bias);
-    } else if (ncache == N) {
-      sweep_in(PgsForm<kPgsUsual>{}, warm, PgsLds<kMemLds>{pgs_lds, off, ncache}, use_bias);
-    } else {
-      sweep_in(PgsForm<kPgsUsual>{}, warm, cache, use_bias);
+    constexpr bool kWarm = decltype(warm)::value;
+    if constexpr (kOnly == kPgsAll) {
+      if (flags == kPgsUsual) sweep_form(PgsForm<kPgsUsual>{}, warm, use_bias);
+      else sweep_other(warm, use_bias);
+    } else if constexpr (!kWarm || (kOnly & BB_SIM_ACCUM_IMPULSE)) {
+      sweep_form(PgsForm<kOnly>{}, warm, use_bias);
     }
   };
   sweep(std::true_type{}, false);
@@ -3925,7 +3950,19 @@ __global__ __launch_bounds__(BLOCK, 4) void k_pgs(Dev d) {
   const uint32_t w = d.order[blockIdx.x];
   if (d.worlds[w].mode & kModeTeam) return;
   const BlockTeam<BLOCK> t{nullptr, nullptr};
-  s_pgs<false, false>(d, w, t, pgs_lds, d.pgs_lcap);
+  s_pgs<false, false, kPgsUsual>(d, w, t, pgs_lds, d.pgs_lcap);
+}
+// the colour sweeps of worlds without friction or accumulation
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK, 4) void k_pgs_flags(Dev d) {
+  HIP_DYNAMIC_SHARED(float4, dyn_lds)
+  float* const pgs_lds = reinterpret_cast<float*>(dyn_lds);
+  const uint32_t w = d.order[blockIdx.x];
+  if (d.worlds[w].mode & kModeTeam) return;
+  const BlockTeam<BLOCK> t{nullptr, nullptr};
+  s_pgs<false, false, BB_SIM_ACCUM_IMPULSE>(d, w, t, pgs_lds, d.pgs_lcap);
+  s_pgs<false, false, BB_SIM_FRICTION>(d, w, t, pgs_lds, d.pgs_lcap);
+  s_pgs<false, false, 0u>(d, w, t, pgs_lds, d.pgs_lcap);
 }
 
 template <int BLOCK>
@@ -4884,12 +4921,12 @@ __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
   __syncthreads();
   s_post(d, w, t, G.post.p);
   __syncthreads();
-  if (d.any_island) {
+  if (d.paths & kPathIsland) {
     s_levels(d, w, t, G.post.p, &G.post.lv);
     __syncthreads();
   }
   s_pgs<false, false>(d, w, t, pgs_lds, d.pgs_lcap);
-  if (d.any_island) {
+  if (d.paths & kPathIsland) {
     __syncthreads();
     if (d.worlds[w].solver == BB_SOLVER_PGS) s_pgs<true, true>(d, w, t, pgs_lds, d.pgs_lcap);
     else s_pgs<true, false>(d, w, t, pgs_lds, d.pgs_lcap);
@@ -5159,8 +5196,8 @@ void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid) {
     }
     case 3: hipLaunchKernelGGL(k_post<B>, g, b, 0, st, d); break;
     case 4:
-      if (d.any_island) hipLaunchKernelGGL(k_levels<B>, g, b, 0, st, d);
-      if (d.any_island)
+      if (d.paths & kPathIsland) hipLaunchKernelGGL(k_levels<B>, g, b, 0, st, d);
+      if (d.paths & kPathIsland)
         hipLaunchKernelGGL(k_pgs_island<B>, g, b, (size_t)d.pgs_lcap * kBodyLds * 4, st, sweep_form<B>(d, grid));
       break;
     case 5: hipLaunchKernelGGL(k_avbd<B>, g, b, 0, st, d); break;
@@ -5169,7 +5206,9 @@ void launch_stage_b(int stage, const Dev& d, hipStream_t st, uint32_t grid) {
 }
 template <int B>
 void launch_pgs_b(const Dev& d, hipStream_t st, uint32_t grid) {
-  hipLaunchKernelGGL(k_pgs<B>, dim3(grid), dim3(B), (size_t)d.pgs_lcap * kBodyLds * 4, st, sweep_form<B>(d, grid));
+  const size_t lds = (size_t)d.pgs_lcap * kBodyLds * 4;
+  if (d.paths & kPathUsual) hipLaunchKernelGGL(k_pgs<B>, dim3(grid), dim3(B), lds, st, sweep_form<B>(d, grid));
+  if (d.paths & kPathFlags) hipLaunchKernelGGL(k_pgs_flags<B>, dim3(grid), dim3(B), lds, st, sweep_form<B>(d, grid));
 }
 template <int B>
 void launch_fused_b(const Lane& l, hipStream_t st) {

@@ -92,6 +92,27 @@ def test_rows_past_the_colours_equal_oracle(worlds, lds):
                 assert np.array_equal(g[f], r[f]), (step, w, f)
 
 
+def test_changed_flags_equal_oracle():
+    """A world whose flags change between steps: the launch sequence follows
+    (usual colour sweeps, those without friction or accumulation, the
+    per-island path)."""
+    d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=4, morton_bits=63, quirks=0))
+    bodies = scenes.random_boxes(77, 40, extent=2.0, y0=0.55, y1=2.5)
+    w, o = beatbox.RigidBodyManager(d), OracleWorld(d)
+    w.add_bodies(bodies)
+    o.add_bodies(bodies)
+    for flags in (scenes.SIM_DEFAULT_FLAGS, *_flags(), scenes.SIM_DEFAULT_FLAGS & ~scenes.SIM_USE_GRAPH_COLORING,
+                  scenes.SIM_DEFAULT_FLAGS):
+        w.clear_sim_flags(0xFFFFFFFF)
+        w.set_sim_flags(flags)
+        o.set_flags(flags)
+        w.simulate(4)
+        o.step(4)
+        g, r = w.read_bodies(), o.read_bodies()
+        for f in FIELDS:
+            assert np.array_equal(g[f], r[f]), (flags, f)
+
+
 def _plate(n: int):
     """A dynamic plate on the ground under n spheres: the plate's contacts
     take several rounds of its group."""
