@@ -1684,6 +1684,22 @@ bb_status overflow_worlds(bb_batch* b, uint32_t* worlds, uint32_t cap, uint32_t*
   return clear_overflow(b);
 }
 
+// Makes the stream's device current while in scope (kernels go to the current
+// device; a thread that only reads states need not have chosen the world's).
+struct StreamDevice {
+  int was = -1;
+  explicit StreamDevice(hipStream_t stream) {
+    hipDevice_t dev = 0;
+    int cur = 0;
+    if (hipStreamGetDevice(stream, &dev) == hipSuccess && hipGetDevice(&cur) == hipSuccess && dev != cur &&
+        hipSetDevice(dev) == hipSuccess)
+      was = cur;
+  }
+  ~StreamDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 bb_status read_world(bb_batch* b, uint32_t w, bb_body_state* out, uint32_t n, bb_order order) {
   if (w >= b->worlds.size() || !out) return BB_ERR_INVALID;
   HostWorld& hw = b->worlds[w];
@@ -1697,6 +1713,7 @@ bb_status read_world(bb_batch* b, uint32_t w, bb_body_state* out, uint32_t n, bb
   const uint32_t N = hw.n;
   if (N) {
     std::lock_guard<std::mutex> lock(b->read_mutex);
+    const StreamDevice on(b->stream);
     const Dev d = dev_for(b, b->latest);
     launch_pack(d, hw.body_off, N, order == BB_ORDER_BY_ID, b->stepped, d.sv_cp, b->stream);
     HIPCHK(hipGetLastError());

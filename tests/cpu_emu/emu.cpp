@@ -305,7 +305,10 @@ void launch(dim3 grid, dim3 block, size_t shmem, std::function<void()> fn) {
 }  // namespace emu
 
 // ------------------------------------------------------------- host API
+static thread_local int t_device = 0;  // the calling thread's current device
+static thread_local hipError_t t_error = hipSuccess;
 struct emu_stream {
+  int device = t_device;
   bool capturing = false;
   std::vector<std::function<void()>> cap;
   emu_stream* redirect = nullptr;  // joined the capture of another stream
@@ -329,6 +332,11 @@ void submit(hipStream_t st, std::function<void()> fn) {
   if (st && st->redirect) st = st->redirect;
   if (st && st->capturing) st->cap.push_back(std::move(fn));
   else fn();
+}
+// a kernel goes to a stream of the current device only
+void submit_kernel(hipStream_t st, std::function<void()> fn) {
+  if (st && st->device != t_device) t_error = hipErrorInvalidHandle;
+  else submit(st, std::move(fn));
 }
 }  // namespace emu
 
@@ -436,17 +444,24 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
   *ms = (float)(b->t - a->t);
   return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() { return std::exchange(t_error, hipSuccess); }
 const char* hipGetErrorString(hipError_t) { return "emu error"; }
 hipError_t hipGetDeviceCount(int* n) {
-  *n = 1;
+  *n = 2;
   return hipSuccess;
 }
 hipError_t hipGetDevice(int* d) {
-  *d = 0;
+  *d = t_device;
   return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipSetDevice(int d) {
+  t_device = d;
+  return hipSuccess;
+}
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) {
+  *d = s ? s->device : t_device;
+  return hipSuccess;
+}
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
   if (a == hipDeviceAttributeWallClockRate) {
     *v = 100000;  // kHz, the rate of wall_clock64 above

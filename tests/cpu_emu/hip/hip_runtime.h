@@ -176,7 +176,7 @@ static inline T atomicCAS(T* p, T cmp, T v) {
 #define __hip_atomic_fetch_add(p, v, o, s) __atomic_fetch_add((p), (v), __ATOMIC_SEQ_CST)
 
 // ------------------------------------------------------------- host API
-typedef enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 } hipError_t;
+typedef enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400 } hipError_t;
 typedef struct emu_stream* hipStream_t;
 typedef struct emu_event* hipEvent_t;
 typedef struct emu_graph* hipGraph_t;
@@ -227,6 +227,8 @@ const char* hipGetErrorString(hipError_t e);
 hipError_t hipGetDeviceCount(int* n);
 hipError_t hipGetDevice(int* d);
 hipError_t hipSetDevice(int d);
+typedef int hipDevice_t;
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d);
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int dev);
 template <class K>
 static inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, K, int, size_t) {
@@ -237,6 +239,7 @@ static inline hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, K,
 namespace emu {
 // Records fn into the stream's capture, or runs it now.
 void submit(hipStream_t st, std::function<void()> fn);
+void submit_kernel(hipStream_t st, std::function<void()> fn);
 }
 #define hipLaunchKernelGGL(K, G, B, SH, ST, ...)                                       \
-  emu::submit((ST), [=]() { emu::launch(dim3(G), dim3(B), (SH), [=]() { K(__VA_ARGS__); }); })
+  emu::submit_kernel((ST), [=]() { emu::launch(dim3(G), dim3(B), (SH), [=]() { K(__VA_ARGS__); }); })

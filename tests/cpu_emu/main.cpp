@@ -9,6 +9,7 @@
 #include <cstdlib>
 #include <vector>
 #include "../../include/bb_capi.h"
+#include "hip/hip_runtime.h"
 
 struct Shape {
   bb_voxel_shape_desc vd{};
@@ -118,12 +119,15 @@ int main(int argc, char** argv) {
     }
     std::fflush(stdout);
   }
+  // the states are read with another device current
+  if (argc > 15 && hipSetDevice(std::atoi(argv[15]))) return 5;
   FILE* o = std::fopen(argv[6], "wb");
   for (uint32_t w = 0; w < nw; ++w) {
     const uint32_t n = (uint32_t)worlds[w].bodies.size();
     std::vector<bb_body_state> out(n);
-    if (single) bb_world_read_bodies(sw, out.data(), n, BB_ORDER_BY_ID);
-    else bb_batch_read_world(b, w, out.data(), n, BB_ORDER_BY_ID);
+    const int st = single ? bb_world_read_bodies(sw, out.data(), n, BB_ORDER_BY_ID)
+                          : bb_batch_read_world(b, w, out.data(), n, BB_ORDER_BY_ID);
+    if (st) { std::fprintf(stderr, "read %d\n", st); return 5; }
     std::fwrite(out.data(), sizeof(bb_body_state), n, o);
   }
   std::fclose(o);

@@ -52,11 +52,11 @@ def _scene(path, worlds, shapes=()):
 
 
 def _run(exe, scene, out, steps, team_bodies, block, graph=1, lane_bodies=0, single=0, team_spin=0,
-         max_blocks=0, sort_blocks=0, walk_budget=0, pgs_block=0, pgs_lds=512, fused=0):
+         max_blocks=0, sort_blocks=0, walk_budget=0, pgs_block=0, pgs_lds=512, fused=0, read_device=0):
     env = dict(ENV, EMU_MAX_BLOCKS=str(max_blocks)) if max_blocks else ENV
     r = subprocess.run([exe, scene, str(steps), str(team_bodies), str(block), str(graph), out, str(lane_bodies),
                         str(single), str(team_spin), str(sort_blocks), str(walk_budget), str(pgs_block),
-                        str(pgs_lds), str(fused)],
+                        str(pgs_lds), str(fused), str(read_device)],
                        capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stderr[-3000:]
     assert "AddressSanitizer" not in r.stderr, r.stderr[-3000:]
@@ -415,3 +415,15 @@ def test_row_of_more_partners_than_threads_equals_oracle(emu_main, tmp_path):
     ref = o.read_bodies()
     for f in ("position", "rotation", "velocity", "omega", "flags"):
         assert got[f].tobytes() == ref[f].tobytes(), f
+
+
+@pytest.mark.parametrize("single", [0, 1])
+def test_states_are_read_with_another_device_current(emu_main, tmp_path, single):
+    """A thread whose current device is not the world's reads its states: the
+    kernel that packs them goes to the world's device."""
+    d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=2, morton_bits=63, quirks=0))
+    scene = str(tmp_path / "scene.bin")
+    _scene(scene, [(d, scenes.random_boxes(51, 9, extent=1.0, y0=0.55, y1=2.0))])
+    _, x = _run(emu_main, scene, str(tmp_path / "a.bin"), 2, 0, 0, graph=0, single=single)
+    _, y = _run(emu_main, scene, str(tmp_path / "b.bin"), 2, 0, 0, graph=0, single=single, read_device=1)
+    assert x == y
