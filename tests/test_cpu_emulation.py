@@ -427,3 +427,69 @@ def test_states_are_read_with_another_device_current(emu_main, tmp_path, single)
     _, x = _run(emu_main, scene, str(tmp_path / "a.bin"), 2, 0, 0, graph=0, single=single)
     _, y = _run(emu_main, scene, str(tmp_path / "b.bin"), 2, 0, 0, graph=0, single=single, read_device=1)
     assert x == y
+
+
+def _cut_in_the_ground(cluster=78, marbles=300):
+    """A cluster of spheres that all overlap, sorted before the ground and its
+    marbles: their pairs leave the ground's row less room than it has
+    partners, and the walk of that row is past its budget."""
+    rng = np.random.default_rng(4)
+    bodies = np.zeros(1 + cluster + marbles, scenes.BODY_DESC)
+    scenes._ground(bodies[0])
+    b = bodies[1:]
+    b["shape"] = scenes.SHAPE_SPHERE
+    b["flags"] = scenes.BODY_DYNAMIC
+    b["rotation"] = (0.0, 0.0, 0.0, 1.0)
+    b["mass"], b["friction"] = 0.1, 0.5
+    side = int(np.ceil(marbles ** 0.5))
+    cx, cz = np.divmod(np.arange(marbles), side)
+    b["position"][:cluster] = rng.uniform(-0.3, 0.3, (cluster, 3)) + (-80.0, -40.0, -80.0)
+    b["position"][cluster:] = np.stack([1.0 + 0.6 * cx, 0.19 + 0.0 * cx, 1.0 + 0.6 * cz], 1)
+    r = np.where(np.arange(cluster + marbles) < cluster, 1.0, 0.2)
+    b["radius"] = r
+    b["minimum"], b["maximum"] = -r[:, None], r[:, None]
+    n = len(bodies)
+    assert cluster * (cluster - 1) // 2 < 8 * n + 64 < cluster * (cluster - 1) // 2 + marbles
+    return bodies
+
+
+def _nan_box():
+    bodies = scenes.random_boxes(71, 80, extent=2.5, y0=0.55, y1=3.0)
+    bodies["omega"][7] = 1e38  # its length overflows: the next pose is NaN
+    return bodies
+
+
+@pytest.mark.parametrize("name", ["ground", "spheres", "order", "voxels", "nan"])
+def test_broad_phase_forms_keep_the_same_pairs(emu_main, tmp_path, name):
+    """Row against row (alone, in three launches), the tree by one workgroup
+    (among 70 worlds) and the tree by a team: the same steps where pairs are
+    cut by the capacity, in a row that its workgroup walks or in one that a
+    thread walks (its first partners in the walk's order: in "order" they are
+    not the first in ascending order), with voxel slots, and with a NaN box in
+    the world."""
+    d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=2, morton_bits=63, quirks=0, gravity=0.0))
+    shapes = []
+    if name == "voxels":
+        shapes, bodies = scenes.voxel_mixed_pile(0xBB93, 90)
+        shapes = [(cells, scenes.VOXEL_SIZE, scenes.VOXEL_DENSITY) for _, cells in shapes]
+        bodies["position"][1:] *= 0.2  # pressed together
+    else:
+        bodies = {"ground": _cut_in_the_ground, "spheres": lambda: scenes.dense_spheres(0xBB94, side=6),
+                  "order": lambda: scenes.dense_spheres(5, side=5), "nan": _nan_box}[name]()
+    tiny = [(d, scenes.random_boxes(7000 + k, 1, extent=0.6, y0=0.55, y1=1.5)) for k in range(69)]
+    alone, among = str(tmp_path / "alone.bin"), str(tmp_path / "among.bin")
+    _scene(alone, [(d, bodies)], shapes)
+    _scene(among, [(d, bodies)] + tiny, shapes)
+    steps = 3
+    log, flat = _run(emu_main, alone, str(tmp_path / "a.bin"), steps, 0, 128, graph=0)
+    log_t, team = _run(emu_main, alone, str(tmp_path / "b.bin"), steps, 50, 128, graph=0)
+    log_w, tree = _run(emu_main, among, str(tmp_path / "c.bin"), steps, 0, 128, graph=0)
+    assert (" overflow world 0" in log) == (name != "nan")
+    assert log_t == log
+    assert [l for l in _world_lines(log_w) if " world 0 " in l] == _world_lines(log)
+    a = np.frombuffer(flat, dtype=beatbox.BODY_STATE)
+    for raw in (team, tree[:len(flat)]):
+        b = np.frombuffer(raw, dtype=beatbox.BODY_STATE)
+        for f in a.dtype.names:  # (a NaN's sign is the compiler's)
+            assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype.kind == "f"), f
+    assert np.isnan(a["rotation"]).any() == (name == "nan")

@@ -133,11 +133,15 @@ def _plate(n: int):
     return np.concatenate([bodies, top])
 
 
-@pytest.mark.parametrize("block,team,fused", [(128, 0, 0), (256, 0, 1), (512, 0, 0), (1024, 0, 0), (256, 9, 0)])
-def test_avbd_groups_equal_oracle(block, team, fused):
+@pytest.mark.parametrize("block,team,fused,more", [
+    (128, 0, 0, 0), (256, 0, 1, 0), (512, 0, 0, 0), (1024, 0, 0, 0), (256, 9, 0, 0),
+    (512, 0, 0, 300), (128, 0, 1, 0), (512, 0, 1, 0), (1024, 0, 1, 0)])
+def test_avbd_groups_equal_oracle(block, team, fused, more):
     """Bodies solved by groups of eight lanes: one contact and several
     rounds of them per body, sizes around a workgroup's groups, both inertia
-    conventions, every workgroup size and workgroup teams."""
+    conventions, every workgroup size (512 threads run the stage with 1,024
+    up to 256 worlds, so once with 300 more), the one-launch step and workgroup
+    teams."""
     b = beatbox.Batch()
     b.set_param(beatbox.PARAM_BLOCK, block)
     b.set_param(beatbox.PARAM_TEAM_BODIES, team)
@@ -154,6 +158,10 @@ def test_avbd_groups_equal_oracle(block, team, fused):
             o = OracleWorld(d)
             o.add_bodies(bodies)
             oracles.append((o, len(bodies)))
+    tiny = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=2, morton_bits=63,
+                                                      quirks=0))
+    for k in range(more):
+        b.add_world(tiny, scenes.random_boxes(5000 + k, 2, extent=0.6, y0=0.55, y1=1.5))
     for steps in (1, 5):
         b.step(steps)
         b.sync(allow_overflow=True)
@@ -193,3 +201,33 @@ def test_avbd_sleeping_worlds_equal_oracle(team):
                 assert np.array_equal(g[f], r[f]), (w, f)
             asleep[w] = max(asleep[w], o.stats()["sleeping_count"])
     assert min(asleep) > 0, asleep
+
+
+@pytest.mark.parametrize("team", [0, 9])
+def test_avbd_lists_without_partners_equal_oracle(team):
+    """Plates pressed into each other, eight contacts a pair: the body lists
+    have more entries than there is room for the other rows beside them."""
+    m = 20
+    rng = np.random.default_rng(3)
+    bodies = np.zeros(m, scenes.BODY_DESC)
+    bodies["shape"] = scenes.SHAPE_BOX
+    bodies["flags"] = scenes.BODY_DYNAMIC
+    bodies["position"][:, 1] = 0.004 * np.arange(m)
+    bodies["rotation"] = scenes.yaw_quat(rng.uniform(0.0, np.pi / 2, m))
+    bodies["minimum"], bodies["maximum"] = (-1.0, -0.1, -1.0), (1.0, 0.1, 1.0)
+    bodies["mass"], bodies["friction"] = 1.0, 0.5
+    d = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10, morton_bits=63, quirks=0,
+                                                   gravity=0.0))
+    b, o = beatbox.Batch(), OracleWorld(d)
+    b.set_param(beatbox.PARAM_TEAM_BODIES, team)
+    b.add_world(d, bodies)
+    o.add_bodies(bodies)
+    for step in range(3):
+        b.step(1)
+        b.sync()
+        o.step(1)
+        # two entries a contact, eight a pair slot (8 m + 64) beside the partners
+        assert step or 2 * o.stats()["contact_count"] > 8 * (8 * m + 64)
+        g, r = b.read_world(0, m), o.read_bodies()
+        for f in FIELDS:
+            assert np.array_equal(g[f], r[f]), (step, f)
