@@ -193,13 +193,15 @@ struct Dev {
   uint32_t* islot;    // [body] island slot (ascending root order)
   uint32_t* ascratch; // [active slot] per-island scratch
   uint32_t* color;    // [pair slot]
-  uint32_t* pick;     // [pair slot]
+  uint32_t* pick;     // [pair slot] broad phase: staged partners; colouring; sweeps: the first tangent's z
   uint32_t* mask;     // [body]
   uint32_t* owner;    // [body*32], zero between rounds
   uint32_t* bucket;   // [pair slot] manifold slots grouped by colour
   uint32_t* bucket_off;  // [W * (kBuckets+1)]
   uint32_t* nlev;        // [W] exact dependency levels of the per-island path (0: none)
-  float4* iw;         // [body*3] cached world inverse inertia rows, row0.w = inv_mass
+  // [body*3] cached world inverse inertia rows, row0.w = inv_mass; AVBD
+  // worlds: the pose's change since the step start (AvData::dp, dth)
+  float4* iw;
   // PGS solver rows (colour-sorted, [pair slot]; contact c of row k at c*np+k)
   uint32_t np;        // pair slots in the batch
   uint32_t pgs_lcap;  // rows per world whose body state k_pgs keeps in LDS (80 B each)
@@ -209,8 +211,8 @@ struct Dev {
   float* sv_m;        // [8*np*3] normal mass, tangent masses 0 and 1 (the arrays
   float* sv_l;        // [8*np*3] normal/tangent impulses        hold 8*np float4)
   uint32_t* sv_list;  // [8*np] AVBD: the world's contacts, slot * 8 + contact
-  // AVBD
-  float4* s_pos0;     // [body] pos_start, w = support depth bits
+  // AVBD (s_pos0 also: position at detection of the PGS rows outside LDS)
+  float4* s_pos0;     // [body] step-start pose
   float4* s_rot0;
   float4* s_post;
   float4* s_rott;

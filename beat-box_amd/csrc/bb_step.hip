@@ -3222,10 +3222,11 @@ BB_DI bool pgs_solvable(const Dev& d, uint32_t off, int4 h) {
 }
 
 // Solver row k from manifold slot: the velocity-independent quantities of
-// PGS_SOFT::pre_step (arms, effective masses).  The row keeps the normal
-// only: the tangents are recomputed from it exactly as Manifold::compute_basis
-// made them, and the soft coefficients depend only on whether either body
-// is immovable (contact hertz doubled, bit 1024 of the count word).
+// PGS_SOFT::pre_step (effective masses; the arms follow from the contact
+// points).  Of the tangents (Manifold::compute_basis) the row keeps the two
+// components of the first that are not zero, and the soft coefficients depend
+// only on whether either body is immovable (contact hertz doubled, bit 1024 of
+// the count word).
 BB_DI void pgs_compact(const Dev& d, const WorldInfo& W, uint32_t k, uint32_t slot) {
   const uint32_t off = W.body_off, NP = d.np;
   const int4 h = d.man_cur.hdr[slot];
@@ -3277,20 +3278,23 @@ BB_DI void pgs_compact(const Dev& d, const WorldInfo& W, uint32_t k, uint32_t sl
 // four waves per SIMD issue side by side at that rate.  So a phase takes the
 // instructions of a row, and the lanes are free until a CU has 16 busy waves.
 // Rows are therefore solved in two forms, chosen per range of rows:
-//  - by quads of lanes (QuadRow): lane i < 3 holds component i of every
+//  - by quads of lanes (pgs_solve): lane i < 3 holds component i of every
 //    vector of the row and row i of its matrices; lane 3 computes along and
 //    is never read (it carries the w component of what was loaded).  Scalars
 //    are computed by all four lanes alike.  A contact takes about 165
 //    instructions instead of 350, and dot and matrix-vector products take
 //    their operands from the neighbours through DPP quad permutations;
-//  - by single lanes (LaneRow): half the instructions per row in total, for
-//    ranges with more rows than the workgroup has quads and for launches
-//    whose worlds fill every CU, which are bound by the chip's issue rate.
+//  - by single lanes (pgs_solve_lane): half the instructions per row in
+//    total, for ranges with more rows than the workgroup has quads and, in
+//    launches whose worlds fill every CU, for ranges of more than one wave of
+//    quads.  Quads for all of them are as fast there: 4,096 worlds with
+//    one-wave workgroups 5.9 | 5.7 ms a step (lanes | quads), which the
+//    autotuner finds out per batch.
 // Each component is the same expression of the same operands in both, so the
 // results are the same bits.  Measured before (one lane per row, 311 spilled
 // registers and both row forms' code in one loop) and after: a fresh 49-body
-// world's sweeps 753 -> about 480 us a step, 513 worlds on the per-island
-// path 17.3 -> 13.0 ms, 4,096 batched worlds 6.6 -> 6.0 ms.
+// world's sweeps 753 -> 356 us a step, 513 worlds on the per-island path 17.3
+// -> 13.0 ms, 4,096 batched worlds 6.0 -> 5.7-5.9 ms.
 template <int CTRL>
 BB_DI float quad_perm(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
@@ -3438,7 +3442,8 @@ struct PgsRows {
 // last component and the first kPgsPre contacts (kPgsPre float4 pairs are
 // loaded whatever the row's count: the contact arrays hold 8 entries per row
 // slot, so the loads stay in bounds, and entries past the count are never
-// used), one dword per lane and float4.  No row's sweep writes any of it, so
+// used), one dword per lane and float4.  No other row's sweep writes any of it
+// (its own writes the impulses), so
 // a quad fetches its next row (of this colour or the next one, across the
 // barrier) before it solves this one and the loads are in flight meanwhile.
 struct PgsRow {

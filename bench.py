@@ -238,7 +238,7 @@ def single_world(name: str, desc, bodies, steps: int, warmup: int, profile: int,
         # and the team launch's size for a team world) and leaves the state
         b.autotune(2)
     params = {n: b.get_param(getattr(beatbox, "PARAM_" + n.upper()))
-              for n in ("sort_blocks", "team_blocks", "block", "avbd_lanes")}
+              for n in ("sort_blocks", "team_blocks", "block")}
     t0 = time.perf_counter()
     b.step(steps, use_graph=True)
     b.sync(allow_overflow=True)

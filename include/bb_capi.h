@@ -534,7 +534,9 @@ bb_status bb_batch_set_block_size(bb_batch* b, uint32_t threads);
  * result: every world's trajectory is bit-identical for every setting. */
 typedef enum bb_param {
   BB_PARAM_BLOCK = 0,        /* threads per world workgroup: 0 = automatic,
-                                128, 256, 512 or 1024                       */
+                                128, 256, 512 or 1024.  The AVBD stage of a
+                                512-thread launch of at most 256 worlds runs
+                                with 1024                                   */
   BB_PARAM_PGS_LDS_ROWS = 1, /* rows per world whose velocities and world
                                 inverse inertia the PGS sweeps keep in LDS
                                 (80 B each): 0..2048                        */
@@ -582,8 +584,11 @@ typedef enum bb_param {
                                 solved by four lanes whenever the workgroup
                                 has enough of them; 0 (default) = that form
                                 while the launch has a CU for every world,
-                                one lane per row otherwise.  The next row is
-                                fetched while one is solved either way      */
+                                otherwise for ranges of up to 16 rows, and
+                                one lane per row for longer ones.  The next
+                                row is fetched while one is solved either
+                                way.  The per-island path without friction
+                                or accumulation always has four lanes       */
   BB_PARAM_WALK_BUDGET = 12, /* broad phase: tree nodes one thread walks for
                                 its body before the body is handed to its
                                 whole workgroup (up to 64 bodies per world;
@@ -613,8 +618,9 @@ bb_status bb_world_set_param(bb_world* w, bb_param p, uint32_t value);
  * each replay restarting from the same state, and keeps the fastest: first
  * the grid of workgroup size x PGS LDS rows, then, one at a time from the
  * best so far, one launch per step or per stage (BB_PARAM_FUSED), the PGS
- * sweep tile (BB_PARAM_PGS_PREFETCH, when a world runs PGS), the radix sort's sub-team (BB_PARAM_SORT_BLOCKS, when a world
- * runs as a workgroup team), the colour sweeps' workgroup and LDS rows
+ * sweep tile (BB_PARAM_PGS_PREFETCH, when a world runs PGS), the radix
+ * sort's sub-team (BB_PARAM_SORT_BLOCKS, when a world runs as a workgroup
+ * team), the colour sweeps' workgroup and LDS rows
  * (BB_PARAM_PGS_BLOCK) and the team launch's size (BB_PARAM_TEAM_BLOCKS:
  * half or all of the resident workgroups).  The broad phase's walk budget
  * keeps its value: an early step cannot show how long the walks grow once

@@ -203,8 +203,8 @@ def test_launch_params_do_not_change_results():
         solver=scenes.SOLVER_AVBD if w == 1 else scenes.SOLVER_PGS_SOFT,
         iterations=8, morton_bits=63, quirks=0)) for w in range(len(sizes))]
     runs = []
-    # (block, LDS rows, one launch per step, AVBD lanes per body, PGS prefetch,
-    # colour-sweep workgroup of the first lane)
+    # (block, LDS rows, one launch per step, AVBD lanes per body (kept without
+    # effect), PGS sweep form, colour-sweep workgroup of the first lane)
     for blk, lds, fused, lanes, pre, pb in ((256, 0, 0, 4, 0, 0), (512, 256, 0, 4, 0, 0), (1024, 768, 0, 4, 1, 0),
                                             (256, 512, 0, 4, 1, 0), (512, 2048, 0, 4, 0, 0),
                                             (256, 512, 1, 4, 1, 0), (512, 256, 1, 2, 0, 0), (256, 0, 0, 1, 1, 0),
@@ -244,8 +244,8 @@ def test_autotune_leaves_state_unchanged():
     avbd = beatbox.WorldDesc.make(**scenes.world_desc(solver=scenes.SOLVER_AVBD, iterations=10,
                                                       morton_bits=63, quirks=0))
     tuned, plain = beatbox.Batch(), beatbox.Batch()
-    # world 1 runs AVBD (the lanes-per-body tile is tuned), world 4 runs as a
-    # workgroup team (the sort's sub-team is tuned)
+    # world 1 runs AVBD, world 4 runs as a workgroup team (the sort's sub-team
+    # is tuned)
     for b in (tuned, plain):
         b.set_param(beatbox.PARAM_TEAM_BODIES, 1000)
     for w, bodies in enumerate(worlds):
