@@ -931,8 +931,7 @@ BB_DI bool overlap(v3 amn, v3 amx, float4 bmn, float4 bmx) {  // Aabb::overlap, 
 // node whose children are (l, r); emit(k, j) receives the k-th partner j.
 // Leaf k holds row k, and a Karras node's left subtree covers the rows before
 // its right subtree's, so partners come out in ascending row order but for a
-// right child that is a leaf, which comes before the left subtree's; kOrdered:
-// it waits on the stack for its turn.
+// right child that is a leaf, which comes before the left subtree's.
 //
 // A left subtree whose rows all lie at or below i is skipped without loading
 // it: the left child of a node with split s covers rows [first, s], and s
@@ -941,7 +940,7 @@ BB_DI bool overlap(v3 amn, v3 amx, float4 bmn, float4 bmx) {  // Aabb::overlap, 
 //
 // `budget` bounds the nodes a thread expands; when it runs out, over_budget()
 // decides: true hands the row over (walk returns kMAX), false walks on.
-template <bool kOrdered = false, class Emit, class Over>
+template <class Emit, class Over>
 BB_DI uint32_t walk(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 qmn, v3 qmx, int l, int r,
                     uint32_t budget, Over&& over_budget, Emit&& emit) {
   // depth of a Karras tree is at most key bits + index bits (63 + 32 < 128)
@@ -972,11 +971,8 @@ BB_DI uint32_t walk(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 qmn, v
     const bool rl = __float_as_int(rm.w) < 0;
     const uint32_t rp = (uint32_t)__float_as_int(rx.w);
     if (ol && ll && i < lp) emit(cnt++, lp);
+    if (orr && rl && i < rp) emit(cnt++, rp);
     const bool tl = ol && !ll, tr = orr && !rl;
-    if (orr && rl && i < rp) {
-      if (kOrdered && tl && sp < 128) stack[sp++] = make_int2(-1, (int)rp);
-      else emit(cnt++, rp);
-    }
     if (tl) {
       if (tr && sp < 128) stack[sp++] = make_int2(__float_as_int(rm.w), __float_as_int(rx.w));
       l = __float_as_int(lm.w);
@@ -985,8 +981,6 @@ BB_DI uint32_t walk(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 qmn, v
       l = __float_as_int(rm.w);
       r = __float_as_int(rx.w);
     } else {
-      if (kOrdered)
-        while (sp && stack[sp - 1].x < 0) emit(cnt++, (uint32_t)stack[--sp].y);
       if (sp == 0) break;
       const int2 c = stack[--sp];
       l = c.x;
@@ -1010,8 +1004,11 @@ BB_DI uint32_t traverse(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 qm
 // below the root is widened level by level, in leaf order, until it holds a
 // node per thread, then each thread walks below its frontier nodes.  The
 // frontier's nodes cover disjoint runs of rows in ascending order, so an
-// exclusive scan of the per-thread counts places the partners in ascending
-// order (which the warm start's binary search in a row's partners needs).
+// exclusive scan of the per-thread counts puts the runs in order.  A row of no
+// more partners than the workgroup has threads has leaves only in its frontier
+// and comes out in ascending order.  Of a longer one a run below an inner node
+// comes out in the walk's order, and the next step's warm start, which looks
+// partners up by binary search, takes those out of order for new contacts.
 template <int BLOCK>
 struct WalkLds {
   uint32_t fr[2][2 * BLOCK];  // frontier nodes (leaf index N - 1 + row for a partner)
@@ -1021,7 +1018,7 @@ static constexpr uint32_t kDeferBit = 0x80000000u;  // pcount mark of such a row
 
 // Count (out == nullptr) or write the first `keep` partners of row i to
 // out[0..keep): called by every thread of the workgroup; returns the count.
-template <int BLOCK, bool kOrdered>
+template <int BLOCK>
 BB_DI uint32_t coop_walk(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 qmn, v3 qmx, WalkLds<BLOCK>& F,
                          ScanLds<BLOCK>& S, uint2* out, uint32_t keep) {
   const uint32_t tid = threadIdx.x;
@@ -1086,8 +1083,8 @@ BB_DI uint32_t coop_walk(const Dev& d, uint32_t nb, uint32_t N, uint32_t i, v3 q
       emit(0u, (uint32_t)(x - leaf_off));
       return 1u;
     }
-    return walk<kOrdered>(d, nb, N, i, qmn, qmx, __float_as_int(d.nmin[nb + x].w), __float_as_int(d.nmax[nb + x].w),
-                      kMAX, [] { return false; }, emit);
+    return walk(d, nb, N, i, qmn, qmx, __float_as_int(d.nmin[nb + x].w), __float_as_int(d.nmax[nb + x].w), kMAX,
+                [] { return false; }, emit);
   };
   uint32_t mine = 0;
   for (uint32_t q = 0; q < per; ++q) {
@@ -1262,7 +1259,7 @@ BB_DI void s_broad_count(const Dev& d, uint32_t w, const T& t, BroadShared& L, W
   for (uint32_t k = t.group(); k < nd; k += t.groups()) {
     const uint32_t i = L.defer[k];
     const float4 mn = d.nmin[nb + N - 1 + i], mx = d.nmax[nb + N - 1 + i];
-    const uint32_t cnt = coop_walk<T::kBlock, !T::kGlobalScalars>(d, nb, N, i, ld3(mn), ld3(mx), F, *t.scan_lds, nullptr, 0u);
+    const uint32_t cnt = coop_walk<T::kBlock>(d, nb, N, i, ld3(mn), ld3(mx), F, *t.scan_lds, nullptr, 0u);
     if (threadIdx.x == 0) d.pcount[off + i] = kDeferBit | cnt;
   }
 }
@@ -1448,7 +1445,7 @@ BB_DI void s_broad_write(const Dev& d, uint32_t w, const T& t, BroadShared& L, W
     if (o >= cap) continue;  // workgroup-uniform
     const uint32_t cnt = d.pcount[off + i] & ~kDeferBit, room = cap - o;
     const float4 mn = d.nmin[nb + N - 1 + i], mx = d.nmax[nb + N - 1 + i];
-    (void)coop_walk<T::kBlock, !T::kGlobalScalars>(d, nb, N, i, ld3(mn), ld3(mx), F, *t.scan_lds, pairs + o, cnt < room ? cnt : room);
+    (void)coop_walk<T::kBlock>(d, nb, N, i, ld3(mn), ld3(mx), F, *t.scan_lds, pairs + o, cnt < room ? cnt : room);
   }
 }
 

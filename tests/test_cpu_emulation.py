@@ -376,47 +376,6 @@ def test_one_launch_steps_are_aligned_and_identical(emu_main, tmp_path, block):
     assert a == b and x == y
 
 
-def _marbles(n):
-    """n spheres rolling on the ground: the ground's row has a partner each."""
-    bodies = np.zeros(n + 1, scenes.BODY_DESC)
-    scenes._ground(bodies[0])
-    rng = np.random.default_rng(1)
-    side = int(np.ceil(n ** 0.5))
-    cx, cz = np.divmod(np.arange(n), side)
-    b = bodies[1:]
-    b["shape"] = scenes.SHAPE_SPHERE
-    b["flags"] = scenes.BODY_DYNAMIC | scenes.BODY_GRAVITY
-    b["position"] = np.stack([0.6 * (cx - side / 2) + rng.uniform(-0.1, 0.1, n), 0.19 + rng.uniform(0.0, 0.02, n),
-                              0.6 * (cz - side / 2) + rng.uniform(-0.1, 0.1, n)], 1)
-    b["velocity"] = rng.uniform(-0.3, 0.3, (n, 3))
-    b["rotation"] = (0.0, 0.0, 0.0, 1.0)
-    b["radius"] = 0.2
-    b["minimum"], b["maximum"] = -0.2, 0.2
-    b["mass"], b["friction"] = 0.1, 0.5
-    return bodies
-
-
-def test_row_of_more_partners_than_threads_equals_oracle(emu_main, tmp_path):
-    """A row with more partners than its workgroup has threads is walked by
-    the workgroup, several partners per thread: they come out in ascending
-    order, in which the next step's warm start looks them up."""
-    from oracle_bind import OracleWorld
-
-    d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=4, morton_bits=63, quirks=0))
-    bodies = _marbles(1200)  # past the line of the row against row form
-    scene = str(tmp_path / "scene.bin")
-    _scene(scene, [(d, bodies)])
-    steps = 4
-    _, raw = _run(emu_main, scene, str(tmp_path / "o.bin"), steps, 0, 128, graph=0)
-    got = np.frombuffer(raw, dtype=beatbox.BODY_STATE)
-    o = OracleWorld(d)
-    o.add_bodies(bodies)
-    o.step(steps)
-    ref = o.read_bodies()
-    for f in ("position", "rotation", "velocity", "omega", "flags"):
-        assert got[f].tobytes() == ref[f].tobytes(), f
-
-
 @pytest.mark.parametrize("single", [0, 1])
 def test_states_are_read_with_another_device_current(emu_main, tmp_path, single):
     """A thread whose current device is not the world's reads its states: the
@@ -481,9 +440,11 @@ def test_broad_phase_forms_keep_the_same_pairs(emu_main, tmp_path, name):
     _scene(alone, [(d, bodies)], shapes)
     _scene(among, [(d, bodies)] + tiny, shapes)
     steps = 3
-    log, flat = _run(emu_main, alone, str(tmp_path / "a.bin"), steps, 0, 128, graph=0)
-    log_t, team = _run(emu_main, alone, str(tmp_path / "b.bin"), steps, 50, 128, graph=0)
-    log_w, tree = _run(emu_main, among, str(tmp_path / "c.bin"), steps, 0, 128, graph=0)
+    # (the ground's row: a workgroup of more threads than the row has partners)
+    block = 512 if name == "ground" else 128
+    log, flat = _run(emu_main, alone, str(tmp_path / "a.bin"), steps, 0, block, graph=0)
+    log_t, team = _run(emu_main, alone, str(tmp_path / "b.bin"), steps, 50, block, graph=0)
+    log_w, tree = _run(emu_main, among, str(tmp_path / "c.bin"), steps, 0, block, graph=0)
     assert (" overflow world 0" in log) == (name != "nan")
     assert log_t == log
     assert [l for l in _world_lines(log_w) if " world 0 " in l] == _world_lines(log)
