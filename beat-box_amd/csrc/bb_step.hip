@@ -4675,8 +4675,10 @@ BB_DI void s_avbd(const Dev& d, uint32_t w, const T& t, AvbdShared& L, float* re
     for (uint32_t k = k0 + tid / G; k < k1; k += NT / G)
       av_primal(d, W, D, k, partners, alpha, tid % G, mine);
   };
-  // ---- main sweeps: 10 x (colours, dual) (rigid_body_manager.cpp:1366-1373)
-  for (uint32_t it = 0; it < AV_ITERS; ++it) {
+  // ---- main sweeps: 10 x (colours, dual) (rigid_body_manager.cpp:1366-1373);
+  // none for a world that sleeps
+  const uint32_t iters = used || contacts ? AV_ITERS : 0u;
+  for (uint32_t it = 0; it < iters; ++it) {
     for (uint32_t c = 0; c < used; ++c) {
       primal(boff[c * kAvbdLayers], boff[(c + 1) * kAvbdLayers], 1.0f);
       t.sync();
