@@ -3270,10 +3270,11 @@ BB_DI void pgs_compact(const Dev& d, const WorldInfo& W, uint32_t k, uint32_t sl
 
 // ---- the sweeps.  A colour phase of a world is one row's chain of
 // operations, contact after contact.  A wave issues one vector operation
-// about every 8 cycles (10-12 with DPP or 64-bit encodings) however few of
-// its lanes are on and whether or not the operations depend on each other;
-// four waves per SIMD issue side by side at that rate.  So a phase takes the
-// instructions of a row, and the lanes are free until a CU has 16 busy waves.
+// about every 5 cycles (6 with DPP or 64-bit encodings) however few of its
+// lanes are on and whether or not the operations depend on each other; two
+// waves per SIMD run side by side at that rate (DPP operands at two thirds of
+// it), four at half.  So a phase takes the instructions of a row, and the
+// lanes are free until a CU has 8 busy waves.
 // Rows are therefore solved in two forms, chosen per range of rows:
 //  - by quads of lanes (pgs_solve): lane i < 3 holds component i of every
 //    vector of the row and row i of its matrices; lane 3 computes along and
@@ -4155,7 +4156,7 @@ BB_DI void group_sync() {
 // constraint rows each, left in the group's LDS words (rec) as Jacobian,
 // stiffness and force.  Then lane a < 6 sums row a of H and entry a of the
 // gradient over all rows in order, and the rows' lanes solve the system
-// together (rows 0-2 in lanes 0-2, rows 3-5 in lanes 4-6): a wave issues an instruction every 8 or
+// together (rows 0-2 in lanes 0-2, rows 3-5 in lanes 4-6): a wave issues an instruction every 5 or
 // more cycles whatever its lanes do, so a body's time is its instructions,
 // and here eight lanes share both the contacts and the sums (one lane per
 // manifold took four times as many on a manifold of four contacts, and the
@@ -5231,9 +5232,10 @@ template __global__ void k_team<kTeamBlock, false>(Dev);
 template __global__ void k_team<kTeamBlock, true>(Dev);
 
 // Threads per workgroup of the AVBD stage.  While every world of the lane has
-// a CU to itself, 512-thread workgroups give way to 1,024-thread ones: a CU
-// issues 16 waves side by side at the rate of one, so a phase with more bodies
-// than 64 groups of lanes take at once saves its further rounds (1,501 bodies,
+// a CU to itself, 512-thread workgroups give way to 1,024-thread ones: 16
+// waves issue at half the rate of 8 but hide each other's loads and LDS
+// accesses, and a phase with more bodies than 64 groups of lanes take at once
+// saves its further rounds (1,501 bodies,
 // about 190 per colour: 2.96 -> 2.46 ms; 64 served worlds' lane 3.6 -> 2.9
 // ms).  The colour sweeps gain nothing by it (1,001 cubes: 437 against 456
 // us).

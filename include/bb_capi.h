@@ -531,7 +531,10 @@ uint64_t bb_batch_device_bytes(const bb_batch* b);
 bb_status bb_batch_set_block_size(bb_batch* b, uint32_t threads);
 
 /* Launch parameters (no reference counterpart).  None of them changes any
- * result: every world's trajectory is bit-identical for every setting. */
+ * result: every world's trajectory is bit-identical for every setting, except
+ * while a body overlaps more bodies than its workgroup has threads (a ground
+ * under a wide pile): which of those contacts are warm started then depends on
+ * the workgroup's size and on whether a team steps the world. */
 typedef enum bb_param {
   BB_PARAM_BLOCK = 0,        /* threads per world workgroup: 0 = automatic,
                                 128, 256, 512 or 1024.  The AVBD stage of a
