@@ -3851,19 +3851,18 @@ BB_DI void s_pgs(const Dev& d, uint32_t w, const T& t, float* pgs_lds, uint32_t 
   // No contact tests the flags: tested per contact, 1,024 worlds without
   // friction swept 3.45 ms a step instead of 2.22, without accumulation 4.77
   // instead of 2.92.  The stage kernels have an instance per set of flags;
-  // teams and the one-launch step, which hold all stages, one sweep for each
-  // set but the usual one, whatever the body rows' place.  The dependency
-  // levels of the per-island path are mostly shorter than a wave of quads and
-  // take quads only, with the flags tested: there single lanes for the long
-  // ones cost every form registers (usual flags 13.8 -> 14.4 ms, no friction
-  // 9.8 -> 11.1).
+  // teams, which hold all stages, one sweep for each set but the usual one.
+  // The dependency levels of the per-island path are mostly shorter than a
+  // wave of quads and take quads only, with the flags tested: there single
+  // lanes for the long ones cost every form registers (usual flags 13.8 ->
+  // 14.4 ms, no friction 9.8 -> 11.1).
   auto sweep_other = [&](auto warm, bool use_bias) __attribute__((always_inline)) {
     constexpr bool kWarm = decltype(warm)::value;
     if constexpr (kIsland) {
       if (kWarm && !s.accum) return;
       sweep_form(PgsForm<kPgsAny>{}, warm, use_bias);
     } else {
-      const PgsLds<T::kGlobalScalars ? kMemHbm : kMemBoth> vc{pgs_lds, off, ncache};
+      const PgsLds<kMemHbm> vc{pgs_lds, off, 0u};
       if (flags == BB_SIM_ACCUM_IMPULSE) sweep_in(PgsForm<BB_SIM_ACCUM_IMPULSE>{}, warm, vc, use_bias);
       if constexpr (!kWarm) {
         if (flags == BB_SIM_FRICTION) sweep_in(PgsForm<BB_SIM_FRICTION>{}, warm, vc, use_bias);
@@ -4930,7 +4929,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_fused(Dev d) {
     s_levels(d, w, t, G.post.p, &G.post.lv);
     __syncthreads();
   }
-  s_pgs<false, false>(d, w, t, pgs_lds, d.pgs_lcap);
+  s_pgs<false, false, kPgsUsual>(d, w, t, pgs_lds, d.pgs_lcap);  // see launch_step
   if (d.paths & kPathIsland) {
     __syncthreads();
     if (d.worlds[w].solver == BB_SOLVER_PGS) s_pgs<true, true>(d, w, t, pgs_lds, d.pgs_lcap);
@@ -5266,9 +5265,13 @@ static void launch_team(const Dev& d, hipStream_t st) {
   else hipLaunchKernelGGL((k_team<kTeamBlock, false>), dim3(d.team_grid), dim3(kTeamBlock), 0, st, d);
 }
 
+// The one-launch step sweeps the usual flags only: with the others' instances
+// it ran 7% slower (1,024 worlds 1.90 -> 2.05 ms a step), and a batch that has
+// such worlds is faster by stages (1.40 ms against 2.02 of the one-launch step
+// that tested the flags).
 void launch_step(const Lane& l, hipStream_t st, bool team) {
   if (team) launch_team(l.d, st);
-  if (l.fused && l.grid) {
+  if (l.fused && l.grid && !(l.d.paths & kPathFlags)) {
     switch (l.block) {
       case 128: launch_fused_b<128>(l, st); break;
       case 512: launch_fused_b<512>(l, st); break;

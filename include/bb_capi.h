@@ -577,7 +577,9 @@ typedef enum bb_param {
   BB_PARAM_FUSED = 9,        /* 1: the per-world stages of a step run as one
                                 launch per lane (k_fused: a world's
                                 workgroup goes from stage to stage without
-                                waiting for the lane's slowest world); 0
+                                waiting for the lane's slowest world), except
+                                in a batch with worlds whose colour sweeps
+                                run without friction or accumulation; 0
                                 (default): one launch per stage.  Profiling
                                 (bb_batch_profile) always times the stages  */
   BB_PARAM_AVBD_LANES = 10,  /* accepted (1, 2, 4 or 8; 0 = the default 4)

@@ -92,6 +92,30 @@ def test_rows_past_the_colours_equal_oracle(worlds, lds):
                 assert np.array_equal(g[f], r[f]), (step, w, f)
 
 
+@pytest.mark.parametrize("others", [False, True])
+def test_one_launch_step_with_flags_equals_oracle(others):
+    """BB_PARAM_FUSED with worlds of the usual flags, and of every set of
+    them (which the batch then runs by stages)."""
+    b = beatbox.Batch()
+    b.set_param(beatbox.PARAM_FUSED, 1)
+    oracles = []
+    for k, flags in enumerate(_flags() if others else _flags()[:1] * 2):
+        d = beatbox.WorldDesc.make(**scenes.world_desc(iterations=4, flags=flags, morton_bits=63, quirks=0))
+        bodies = scenes.random_boxes(300 + k, 60 + k, extent=2.5, y0=0.55, y1=3.0)
+        b.add_world(d, bodies)
+        o = OracleWorld(d)
+        o.add_bodies(bodies)
+        oracles.append((o, len(bodies)))
+    for steps in (1, 6):
+        b.step(steps, use_graph=steps > 1)
+        b.sync()
+        for w, (o, n) in enumerate(oracles):
+            o.step(steps)
+            g, r = b.read_world(w, n), o.read_bodies()
+            for f in FIELDS:
+                assert np.array_equal(g[f], r[f]), (w, n, f)
+
+
 def test_changed_flags_equal_oracle():
     """A world whose flags change between steps: the launch sequence follows
     (usual colour sweeps, those without friction or accumulation, the
